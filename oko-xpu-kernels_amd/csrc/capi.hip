@@ -243,12 +243,11 @@ size_t linear_work_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 // quantize + GEMM + dequant of xpuint8_linear_stream on checked arguments.
-// wp (optional): pack_weight's copy of w8, read instead of w8 by the kernels
-// that take the block layout (the split-K, persistent and skinny ones).
+// wp (optional): pack_weight's copy of w8, read instead of w8 wherever the
+// product is not split in K across blocks.
 int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_scale,
                const void* bias, int32_t bias_bf16, void* out, int64_t M, int64_t N, int64_t K,
                void* work, const int8_t* wp = nullptr) {
-    const int8_t* wb = wp ? wp : w8;
     int8_t* q = static_cast<int8_t*>(work);
     float* xs = reinterpret_cast<float*>(static_cast<char*>(work) + linear_work_q_bytes(M, K));
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
@@ -265,26 +264,16 @@ int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_s
         return launched(dequant_slices(st, part, N, nsl, M * N, out, xs, w_scale, b32, b16, M, N),
                         "linear (dequant)");
     }
-    // narrow outputs with a long K take the split-K kernel, which reads q in
-    // the MFMA block layout; the other shapes a row-major q
-    if (splitk_applies(int(M), int(N), int(K)) && rowquant_can_tile(int(K))) {
+    // q in the MFMA block layout: for every kernel that reads the packed weight,
+    // and for the split-K and persistent kernels on the row-major one
+    if (rowquant_can_tile(int(K)) && (wp || xt_applies(int(M), int(N), int(K)))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
-        return launched(gemm_dequant_xt(st, q, wb, K, out, N, xs, w_scale, b32, b16, int(M),
-                                        int(N), int(K), wp != nullptr),
-                        "linear (gemm)");
-    }
-    // the persistent kernel reads q in the MFMA block layout too
-    if (pp_applies(int(M), int(N), int(K), false) && rowquant_can_tile(int(K))) {
-        XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
-        return launched(gemm_dequant_pp_xt(st, q, wb, K, out, N, xs, w_scale, b32, b16, int(M),
-                                           int(N), int(K), wp != nullptr),
-                        "linear (gemm)");
-    }
-    // and the skinny one, given the packed weight
-    if (wp && skinny_applies(int(M), false) && rowquant_can_tile(int(K))) {
-        XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
-        return launched(gemm_dequant_skinny_xt(st, q, wp, out, N, xs, w_scale, b32, b16, int(M),
-                                               int(N), int(K)),
+        if (wp)
+            return launched(gemm_dequant_packed(st, q, wp, out, N, xs, w_scale, b32, b16, int(M),
+                                                int(N), int(K)),
+                            "linear (gemm)");
+        return launched(gemm_dequant_xt(st, q, w8, K, out, N, xs, w_scale, b32, b16, int(M),
+                                        int(N), int(K)),
                         "linear (gemm)");
     }
     XPU_TRY(launched(convrot_quantize(st, x, q, xs, M, int(K), 0), "linear (quantize)"));
@@ -610,11 +599,7 @@ int xpuint8_linear_gemm_tiled_stream(const void* stream, const int8_t* xq, const
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
     hipStream_t st = as_stream(stream);
-    if (pp_applies(int(M), int(N), int(K), false))
-        return launched(gemm_dequant_pp_xt(st, xq, w8, K, out, N, x_scale, w_scale, b32, b16,
-                                           int(M), int(N), int(K)),
-                        "linear_gemm_tiled");
-    if (splitk_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0)
+    if (xt_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0)
         return launched(gemm_dequant_xt(st, xq, w8, K, out, N, x_scale, w_scale, b32, b16,
                                         int(M), int(N), int(K)),
                         "linear_gemm_tiled");
@@ -675,15 +660,18 @@ int xpuint8_linear_residual_packed_stream(const void* stream, const void* x, con
     float* xs = reinterpret_cast<float*>(static_cast<char*>(work) + linear_work_q_bytes(M, K));
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
-    // the kernels that read x in the MFMA block layout (and the packed weight)
-    if (rowquant_can_tile(int(K)) &&
-        (pp_applies(int(M), int(N), int(K), false) ||
-         (splitk_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0))) {
+    // the kernels that read x in the MFMA block layout
+    if (rowquant_can_tile(int(K)) && (w8_packed || xt_applies(int(M), int(N), int(K)))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)),
                          "linear_residual (quantize)"));
-        return launched(gemm_dequant_residual_xt(st, q, w8_packed ? w8_packed : w8, K, out, N, xs,
-                                                 w_scale, b32, b16, residual, N, residual_scale,
-                                                 int(M), int(N), int(K), w8_packed != nullptr),
+        if (w8_packed)
+            return launched(gemm_dequant_residual_packed(st, q, w8_packed, out, N, xs, w_scale,
+                                                         b32, b16, residual, N, residual_scale,
+                                                         int(M), int(N), int(K)),
+                            "linear_residual (gemm)");
+        return launched(gemm_dequant_residual_xt(st, q, w8, K, out, N, xs, w_scale, b32, b16,
+                                                 residual, N, residual_scale, int(M), int(N),
+                                                 int(K)),
                         "linear_residual (gemm)");
     }
     XPU_TRY(launched(convrot_quantize(st, x, q, xs, M, int(K), 0), "linear_residual (quantize)"));
@@ -705,11 +693,13 @@ int xpuint8_linear_acc_packed_stream(const void* stream, const void* x, const in
     XPU_TRY(ensure_device());
     hipStream_t st = as_stream(stream);
     int8_t* q = static_cast<int8_t*>(work);
-    if (rowquant_can_tile(int(K)) && pp_applies(int(M), int(N), int(K), false)) {
+    if (rowquant_can_tile(int(K)) && (w8_packed || pp_applies(int(M), int(N), int(K), false))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, x_scale, M, int(K)),
                          "linear_acc (quantize)"));
-        return launched(gemm_i32_pp_xt(st, q, w8_packed ? w8_packed : w8, K, acc, N, int(M),
-                                       int(N), int(K), w8_packed != nullptr),
+        if (w8_packed)
+            return launched(gemm_i32_packed(st, q, w8_packed, acc, N, int(M), int(N), int(K)),
+                            "linear_acc (gemm)");
+        return launched(gemm_i32_pp_xt(st, q, w8, K, acc, N, int(M), int(N), int(K)),
                         "linear_acc (gemm)");
     }
     XPU_TRY(launched(convrot_quantize(st, x, q, x_scale, M, int(K), 0), "linear_acc (quantize)"));
@@ -731,17 +721,10 @@ int xpuint8_linear_gemm_packed_stream(const void* stream, const int8_t* xq, cons
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
     hipStream_t st = as_stream(stream);
-    if (pp_applies(int(M), int(N), int(K), false))
-        return launched(gemm_dequant_pp_xt(st, xq, w8_packed, 0, out, N, x_scale, w_scale, b32,
-                                           b16, int(M), int(N), int(K), true),
-                        "linear_gemm_packed");
-    if (splitk_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0)
-        return launched(gemm_dequant_xt(st, xq, w8_packed, 0, out, N, x_scale, w_scale, b32, b16,
-                                        int(M), int(N), int(K), true),
-                        "linear_gemm_packed");
-    if (skinny_applies(int(M), false) && gemm_slices(int(M), int(N), int(K)) == 0)
-        return launched(gemm_dequant_skinny_xt(st, xq, w8_packed, out, N, x_scale, w_scale, b32,
-                                               b16, int(M), int(N), int(K)),
+    if (gemm_slices(int(M), int(N), int(K)) == 0 &&
+        (M <= 64 || xt_applies(int(M), int(N), int(K))))
+        return launched(gemm_dequant_packed(st, xq, w8_packed, out, N, x_scale, w_scale, b32, b16,
+                                            int(M), int(N), int(K)),
                         "linear_gemm_packed");
     return fail(2, "linear_gemm_packed: this shape does not read the block layouts");
 }

@@ -857,7 +857,8 @@ hipError_t launch_cfg(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t
 }
 
 // ------------------------------------------------------------ ping-pong
-// BM x BN tiles (256 x 320) for one persistent block of 8 waves per CU, in two
+// BM x BN tiles (256 x 320; with both operands in the block layout also the
+// smaller ones of pp_tile) for one persistent block of 8 waves per CU, in two
 // groups of 4 (group = the tile's row half, 2 x 4 waves of 128 x 80, or 4 x 2
 // of 64 x 160 for paired epilogues), a ring of S = 4 LDS slots of 64-byte K
 // steps filled by direct global->LDS loads.  Block b takes tiles b, b + G,
@@ -876,7 +877,8 @@ hipError_t launch_cfg(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t
 // Between tiles: once a tile's last MFMAs are issued (every fragment read is
 // complete), each wave issues the next tile's steps 0-2 into slots 1-3 and
 // the global loads of its row/column operands, and only then runs this tile's
-// epilogue, staged through slot 0.  Those loads are older than the epilogue's
+// epilogue, staged through slot 0 (or, where a slot is smaller than the 32 KB
+// the eight waves stage, an area of its own).  Those loads are older than the epilogue's
 // stores, so they land while it runs; one vmcnt(0) afterwards (the stores
 // included) and a barrier start the next tile.  The epilogue's per-row and
 // per-column operands come from LDS (two buffers after the ring, filled one
@@ -900,14 +902,15 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     constexpr int XB = BM / 16, WB = BN / 16, NB = XB + WB;
     constexpr int PER = (NB + NW - 1) / NW;                     // loads per wave per step (max)
     constexpr int REM = NB % NW;                                // waves < REM issue PER
-    static_assert(REM == 0 || REM == 4, "group 0 issues PER, group 1 PER or PER - 1");
-    constexpr int PER0 = PER, PER1 = REM == 0 ? PER : PER - 1;
     constexpr int STAGE_BYTES = NB * 1024;
     constexpr int RING = S * STAGE_BYTES;
     static_assert(S == 4, "a tile's last slot stages the epilogue while the next tile's steps 0-2 "
                           "fill the other three");
     constexpr bool STAGED = Epi::kStaged;
-    static_assert(!STAGED || NW * 16 * 256 <= STAGE_BYTES, "epilogue staging fits in one slot");
+    // the epilogue is staged through the slot of the tile's last step, or, where
+    // a slot is too small, through an area of its own after the operands
+    constexpr int STG_BYTES = NW * 16 * 256;
+    constexpr int STG_OWN = STAGED && STG_BYTES > STAGE_BYTES ? STG_BYTES : 0;
     constexpr bool PAIRED = Epi::kPaired;
     static_assert(!PAIRED || (STAGED && TN % 2 == 0), "pairs are whole per wave");
     constexpr int OUT_TN = PAIRED ? TN / 2 : TN;
@@ -921,8 +924,10 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     constexpr int SPT = (NSCALE + 511) / 512;                   // operand values per thread
     // the activation table's LDS window, for an epilogue that has one
     constexpr int WIN_BYTES = has_window<Epi>() ? 2 * kWinSize : 0;
-    __shared__ __attribute__((aligned(1024))) int8_t smem[RING + 2 * SCALE_BYTES + WIN_BYTES + 16];
-    static_assert(RING + 2 * SCALE_BYTES + WIN_BYTES + 16 <= 160 * 1024, "LDS");
+    constexpr int LDS_BYTES = RING + STG_OWN + 2 * SCALE_BYTES + WIN_BYTES + 16;
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) int8_t smem[LDS_BYTES];
+    constexpr int SCALES = RING + STG_OWN;                      // LDS offset of the operands
     Epi epi_w = epi;                    // the epilogue, with the window's address once filled
 
     const int tiles = tiles_m * tiles_n;
@@ -930,13 +935,18 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     const int g = wm / (WGM / 2);                               // group: the row half
+    // issues PER loads per step, else PER - 1 (REM = 4: group 0 and group 1)
+    const bool full_share = REM == 0 || (REM == 4 ? g == 0 : wave < REM);
 
     // tile origin of sequence number i: each XCD (i % 8, as blockIdx % 8)
-    // takes a contiguous eighth of the tiles, walked in column bands of 8 row
-    // tiles
+    // takes a contiguous eighth of the tiles (rounded up: the last XCDs may
+    // get fewer), walked in column bands of 8 row tiles.  False past the XCD's
+    // share, and then for every later i of the block (the grid is a multiple
+    // of 8 or one round).
+    const int share = (tiles + 7) / 8;
     auto tile_origin = [&](int i, int& m0, int& n0) {
-        int t = i;
-        if (tiles % 8 == 0) t = (t % 8) * (tiles / 8) + t / 8;
+        const int t = (i % 8) * share + i / 8;
+        if (i / 8 >= share || t >= tiles) return false;
         constexpr int GROUP = 8;
         const int band = t / (GROUP * tiles_n);
         const int first_m = band * GROUP;
@@ -944,6 +954,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
         const int in_band = t - band * GROUP * tiles_n;
         m0 = (first_m + in_band % gm) * BM;
         n0 = (in_band / gm) * BN_OUT;
+        return true;
     };
 
     const int KT = (K + BK - 1) / BK;
@@ -1011,7 +1022,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
         int8_t* const st = smem + slot(kk);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            if (i == PER - 1 && REM != 0 && g != 0) continue;
+            if (i == PER - 1 && !full_share) continue;
             const int8_t* p;
             if ((XT && wave + NW * i < XB) || (WT && wave + NW * i >= XB)) {
                 // a tiled block: K step kstep is the row group's kstep-th
@@ -1029,13 +1040,13 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     // wait until this wave's loads of every step before `later` more of its
     // own load batches are complete
     auto wait_batches = [&](int later) {
-        if (g == 0) {
-            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * PER0));
-            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER0));
+        if (full_share) {
+            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * PER));
+            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER));
             else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         } else {
-            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * PER1));
-            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER1));
+            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * (PER - 1)));
+            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER - 1));
             else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         }
     };
@@ -1061,7 +1072,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     };
     auto put_scales = [&](int buf) {
         if constexpr (STAGED) {
-            float* d = reinterpret_cast<float*>(smem + RING + buf * SCALE_BYTES);
+            float* d = reinterpret_cast<float*>(smem + SCALES + buf * SCALE_BYTES);
 #pragma unroll
             for (int i = 0; i < SPT; ++i) {
                 const int idx = threadIdx.x + 512 * i;
@@ -1097,7 +1108,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     };
     auto epilogue = [&](int m0, int n0, int buf) {
         if constexpr (STAGED) {
-            const float* sc = reinterpret_cast<const float*>(smem + RING + buf * SCALE_BYTES);
+            const float* sc = reinterpret_cast<const float*>(smem + SCALES + buf * SCALE_BYTES);
             const float* xr = sc + wm * WM + (lane & 15);
             typename Epi::Col ccol[TN];
 #pragma unroll
@@ -1111,7 +1122,8 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
             // staged through the slot of the tile's last step (the other
             // three hold the next tile's first steps)
             staged_store<TM, TN, WN_OUT, Epi, 1>(epi_w, acc, [&](int b) { return xr[16 * b]; }, ccol,
-                                                 smem + slot(KT - 1) + wave * (16 * 256),
+                                                 smem + (STG_OWN ? RING : slot(KT - 1)) +
+                                                     wave * (16 * 256),
                                                  m0 + wm * WM, n0 + wn * WN_OUT, M, N, lane);
         } else {
             const int mrow = m0 + wm * WM + (lane & 15);
@@ -1130,16 +1142,15 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     };
 
     int ti = blockIdx.x;
-    if (ti >= tiles) return;
+    int m0, n0;
+    if (!tile_origin(ti, m0, n0)) return;
     if constexpr (WIN_BYTES > 0) {
         // the window, read once per block (visible after the first barrier)
-        uint16_t* w = reinterpret_cast<uint16_t*>(smem + RING + 2 * SCALE_BYTES);
+        uint16_t* w = reinterpret_cast<uint16_t*>(smem + SCALES + 2 * SCALE_BYTES);
         const uint16_t* t = epi.tab + size_t(Epi::kWinTab) * kTabSize;
         for (int i = threadIdx.x; i < kWinSize; i += 512) w[i] = t[win_bits(i)];
         epi_w.win = lds_addr(w);
     }
-    int m0, n0;
-    tile_origin(ti, m0, n0);
     setup(m0, n0);
     // first tile: its operands, steps 0 .. S-2 requested, step 0 complete
     fetch_scales(m0, n0);
@@ -1154,9 +1165,8 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
 #pragma unroll
             for (int b = 0; b < TM; ++b) acc[a][b] = v4i{0, 0, 0, 0};
         const int tnext = ti + int(gridDim.x);
-        const bool more = tnext < tiles;
         int m0n = 0, n0n = 0;
-        if (more) tile_origin(tnext, m0n, n0n);
+        const bool more = tile_origin(tnext, m0n, n0n);
         // With a next tile (and K steps enough), the loads of its steps 0-2
         // go out in this tile's last three steps, in the ring positions where
         // steps KT..KT+2 would go: the loop's loads never stop at the tile
@@ -1592,14 +1602,17 @@ hipError_t launch_splitk(hipStream_t st, const int8_t* X, int64_t ldx, const int
                          int64_t ldw, int M, int N, int K, const Epi& epi) {
     constexpr int S = 4;                        // 2 x 4 x 18 KB of LDS
     const int tm = (M + 127) / 128, tn = (N + 159) / 160;
-    if (K % 64 == 0)
-        hipLaunchKernelGGL((gemm_i8_splitk_kernel<S, false, WNN, Epi, XT, WT>),
-                           dim3(unsigned(tm * tn)), dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm,
-                           tn, epi);
-    else
-        hipLaunchKernelGGL((gemm_i8_splitk_kernel<S, true, WNN, Epi, XT, WT>),
-                           dim3(unsigned(tm * tn)), dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm,
-                           tn, epi);
+    if constexpr (!(XT && WT)) {                // packed weights hold zeros past K
+        if (K % 64 != 0) {
+            hipLaunchKernelGGL((gemm_i8_splitk_kernel<S, true, WNN, Epi, XT, WT>),
+                               dim3(unsigned(tm * tn)), dim3(512), 0, st, X, ldx, W, ldw, M, N, K,
+                               tm, tn, epi);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((gemm_i8_splitk_kernel<S, false, WNN, Epi, XT, WT>),
+                       dim3(unsigned(tm * tn)), dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm, tn,
+                       epi);
     return hipGetLastError();
 }
 
@@ -1836,21 +1849,107 @@ hipError_t launch_skinny(hipStream_t st, const int8_t* X, int64_t ldx, const int
 // ping-pong tile (as 4 x 2 waves) or the large one.
 constexpr int kSkinnyPairedM = 256;
 
-// The persistent ping-pong kernel over 256 x 320 tiles, one block per CU (X
-// row-major with row stride ldx, or XT: in the MFMA block layout).
-template <bool XT, bool WT = false, class Epi>
+// The persistent kernel's grid: one block per CU, or one round of blocks (each
+// XCD's share rounded up) when there are fewer tiles
+inline unsigned pp_grid(int64_t tiles) {
+    return unsigned(std::min<int64_t>((tiles + 7) / 8 * 8, device_cus() / 8 * 8));
+}
+
+// The persistent ping-pong kernel over BM x BN tiles, one block per CU (X
+// row-major with row stride ldx, or XT: in the MFMA block layout; WT: the
+// packed weight).  K past the last whole step matters to row-major operands
+// only: in the packed weight those bytes are zeros.
+template <bool XT, bool WT = false, int BM = 256, int BN = 320, int WGM = 0, class Epi>
 hipError_t launch_pp(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t* W, int64_t ldw,
                      int M, int N, int K, const Epi& epi) {
-    constexpr int WGM = Epi::kPaired ? 4 : 2, WGN = 8 / WGM;
-    const int tm = (M + 255) / 256, tn = Epi::kPaired ? (N + 159) / 160 : (N + 319) / 320;
-    const dim3 grid(unsigned(std::min<int64_t>(int64_t(tm) * tn, device_cus())));
-    if (K % 64 == 0)
-        hipLaunchKernelGGL((gemm_i8_pp_kernel<256, 320, WGM, WGN, 4, false, Epi, XT, WT>), grid,
-                           dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm, tn, epi);
-    else
-        hipLaunchKernelGGL((gemm_i8_pp_kernel<256, 320, WGM, WGN, 4, true, Epi, XT, WT>), grid,
-                           dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm, tn, epi);
+    constexpr int GM = WGM ? WGM : (Epi::kPaired ? 4 : 2), GN = 8 / GM;
+    constexpr int BN_OUT = Epi::kPaired ? BN / 2 : BN;
+    const int tm = (M + BM - 1) / BM, tn = (N + BN_OUT - 1) / BN_OUT;
+    const dim3 grid(pp_grid(int64_t(tm) * tn));
+    if constexpr (!(XT && WT)) {
+        if (K % 64 != 0) {
+            hipLaunchKernelGGL((gemm_i8_pp_kernel<BM, BN, GM, GN, 4, true, Epi, XT, WT>), grid,
+                               dim3(512), 0, st, X, ldx, W, ldw, M, N, K, tm, tn, epi);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((gemm_i8_pp_kernel<BM, BN, GM, GN, 4, false, Epi, XT, WT>), grid, dim3(512),
+                       0, st, X, ldx, W, ldw, M, N, K, tm, tn, epi);
     return hipGetLastError();
+}
+
+// The ping-pong kernel's tile for a product of two block-layout operands: the
+// one with the least predicted time.  A block runs ceil(share / CUs per XCD)
+// rounds of tiles; a K step of a BM x BN tile takes 0.0546 us per 10^4
+// outputs (the matrix cores and the LDS reads that feed them) plus 0.21 us
+// (barriers, waits, load issue), a tile's epilogue 0.99 us per 10^4 outputs,
+// both less when the last round leaves CUs (and so memory bandwidth) free.
+// Fitted to 15 tile shapes on 170 products of 3-260 GOP, M 65-4096, N 256-10240,
+// K 256-8192 (the times' scatter about it is 3.5%); choosing among these five by
+// it is 0.3% off the fastest of the fifteen on average (11% at worst).  Against
+// the kernels that took those products before (256 x 160 and 128 x 128 tiles of
+// row-major operands, split K), cold weights and activations rotating:
+//   3974 x 3072 x 3072 (M, N, K)  51.2 -> 34.7 us (192 x 256: 252 tiles)
+//   3952 x 3072 x 8192            135.5 -> 82.0 us
+//   1388 x 9376 x 2816            53.7 -> 37.1 us
+//   2048 x 5120 x 1280            25.0 -> 17.7 us
+//   4096 x 1280 x 1280            14.4 -> 12.2 us (128 x 192, against split K)
+// Long contractions of narrow outputs stay with the split-K kernel, whose four
+// waves per team read 12% fewer LDS bytes per MFMA than 128 x 192's eight and
+// whose steps cost less (0.29 us of 128 x 160 x 64; its exchange and epilogue 5.6 us a
+// round; fitted to the same products, scatter 3.7%): at 4096 x 1280 x 5120, in a
+// training step, 30.4 us against 32.5; at 4096 x 1280 x 1280 14.2 against 12.2.
+// It is taken where it is predicted 3% faster.
+struct PpTile {
+    int bm, bn;
+};
+constexpr PpTile kPpTiles[] = {{256, 320}, {192, 320}, {192, 256}, {192, 192}, {128, 192}};
+
+inline double pp_time(int bm, int bn, int64_t M, int64_t N, int K) {
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), cus = device_cus();
+    const int64_t rounds = ((tiles + 7) / 8 + cus / 8 - 1) / (cus / 8);
+    const double area = 1e-4 * bm * bn, fill = double(tiles) / double(cus * rounds);
+    const double steps = (K + 63) / 64;
+    return 3.8 + double(rounds) * (steps * (0.0546 * area + 0.206) * (0.84 + 0.16 * fill) +
+                                   0.994 * area * (0.615 + 0.385 * fill));
+}
+
+inline double splitk_time(int64_t M, int64_t N, int K) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 159) / 160), cus = device_cus();
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    const double fill = double(tiles) / double(cus * rounds), steps = (K + 63) / 64;
+    return 2.9 + double(rounds) * (steps * 0.287 * (0.82 + 0.18 * fill) +
+                                   5.62 * (0.8 + 0.2 * fill));
+}
+
+inline int pp_tile(int64_t M, int64_t N, int K, double* time) {
+    int best = 0;
+    double t = 0;
+    for (int i = 0; i < int(sizeof(kPpTiles) / sizeof(kPpTiles[0])); ++i) {
+        const double c = pp_time(kPpTiles[i].bm, kPpTiles[i].bn, M, N, K);
+        if (i == 0 || c < t) best = i, t = c;
+    }
+    *time = t;
+    return best;
+}
+
+// X and W both in the block layout, unpaired epilogues
+template <class Epi>
+hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N, int K,
+                          const Epi& epi) {
+    double t = 0;
+    const int tile = pp_tile(M, N, K, &t);
+    if constexpr (Epi::kStaged) {
+        if (1.03 * splitk_time(M, N, K) < t)
+            return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
+    }
+    switch (tile) {
+        case 0: return launch_pp<true, true, 256, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 1: return launch_pp<true, true, 192, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 2: return launch_pp<true, true, 192, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 3: return launch_pp<true, true, 192, 192, 4>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        default: return launch_pp<true, true, 128, 192>(st, Xt, 0, Wp, 0, M, N, K, epi);
+    }
 }
 
 template <class Epi>
@@ -2183,20 +2282,27 @@ hipError_t gemm_dequant_nn(hipStream_t st, const int8_t* A, int64_t lda, const i
 
 hipError_t gemm_dequant_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                            void* out, int64_t ldo, const float* xs, const float* ws,
-                           const float* bias, const uint16_t* bias16, int M, int N, int K,
-                           bool packed) {
+                           const float* bias, const uint16_t* bias16, int M, int N, int K) {
     const EpiDequant epi{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16};
-    if (packed) return launch_splitk<false, EpiDequant, true, true>(st, At, 0, B, 0, M, N, K, epi);
-    return launch_splitk<false, EpiDequant, true>(st, At, 0, B, ldb, M, N, K, epi);
+    if (splitk_applies(M, N, K))
+        return launch_splitk<false, EpiDequant, true>(st, At, 0, B, ldb, M, N, K, epi);
+    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, epi);
 }
 
-hipError_t gemm_dequant_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
-                              void* out, int64_t ldo, const float* xs, const float* ws,
-                              const float* bias, const uint16_t* bias16, int M, int N, int K,
-                              bool packed) {
-    const EpiDequant epi{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16};
-    if (packed) return launch_pp<true, true>(st, At, 0, B, 0, M, N, K, epi);
-    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, epi);
+bool xt_applies(int M, int N, int K) { return splitk_applies(M, N, K) || pp_applies(M, N, K, false); }
+
+template <class Epi>
+static hipError_t packed_gemm(hipStream_t st, const int8_t* At, const int8_t* Bp, int M, int N,
+                              int K, const Epi& epi) {
+    if (M <= 64) return launch_skinny<1, Epi, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
+    return launch_tiles(st, At, Bp, M, N, K, epi);
+}
+
+hipError_t gemm_dequant_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
+                               int64_t ldo, const float* xs, const float* ws, const float* bias,
+                               const uint16_t* bias16, int M, int N, int K) {
+    return packed_gemm(st, At, Bp, M, N, K,
+                       EpiDequant{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16});
 }
 
 template <int ACT>
@@ -2220,13 +2326,6 @@ hipError_t gemm_act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int
 }
 
 bool skinny_applies(int M, bool paired) { return M <= (paired ? kSkinnyPairedM : 64); }
-
-hipError_t gemm_dequant_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
-                                  int64_t ldo, const float* xs, const float* ws, const float* bias,
-                                  const uint16_t* bias16, int M, int N, int K) {
-    const EpiDequant epi{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16};
-    return launch_skinny<1, EpiDequant, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
-}
 
 hipError_t gemm_act_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
                               int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
@@ -2252,47 +2351,54 @@ hipError_t gemm_dequant_nn_xt(hipStream_t st, const int8_t* At, const int8_t* Bk
     return launch_splitk<true, EpiDequant, true>(st, At, 0, Bkn, ldb, M, N, K, epi);
 }
 
-hipError_t gemm_dequant_residual(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B,
-                                 int64_t ldb, void* out, int64_t ldo, const float* xs,
-                                 const float* ws, const float* bias, const uint16_t* bias16,
-                                 const void* res, int64_t ldr, const void* rscale, int M, int N,
-                                 int K) {
+static EpiDequantRes residual_epi(void* out, int64_t ldo, const float* xs, const float* ws,
+                                  const float* bias, const uint16_t* bias16, const void* res,
+                                  int64_t ldr, const void* rscale) {
     EpiDequantRes e;
     static_cast<EpiDequant&>(e) =
         EpiDequant{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16};
     e.res = static_cast<const uint16_t*>(res);
     e.ldr = ldr;
     e.rscale = static_cast<const uint16_t*>(rscale);
-    return launch_gemm(st, A, lda, B, ldb, M, N, K, e);
+    return e;
+}
+
+hipError_t gemm_dequant_residual(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B,
+                                 int64_t ldb, void* out, int64_t ldo, const float* xs,
+                                 const float* ws, const float* bias, const uint16_t* bias16,
+                                 const void* res, int64_t ldr, const void* rscale, int M, int N,
+                                 int K) {
+    return launch_gemm(st, A, lda, B, ldb, M, N, K,
+                       residual_epi(out, ldo, xs, ws, bias, bias16, res, ldr, rscale));
 }
 
 hipError_t gemm_dequant_residual_xt(hipStream_t st, const int8_t* At, const int8_t* B,
                                     int64_t ldb, void* out, int64_t ldo, const float* xs,
                                     const float* ws, const float* bias, const uint16_t* bias16,
                                     const void* res, int64_t ldr, const void* rscale, int M, int N,
-                                    int K, bool packed) {
-    EpiDequantRes e;
-    static_cast<EpiDequant&>(e) =
-        EpiDequant{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16};
-    e.res = static_cast<const uint16_t*>(res);
-    e.ldr = ldr;
-    e.rscale = static_cast<const uint16_t*>(rscale);
-    if (pp_applies(M, N, K, false)) {
-        if (packed) return launch_pp<true, true>(st, At, 0, B, 0, M, N, K, e);
-        return launch_pp<true>(st, At, 0, B, ldb, M, N, K, e);
-    }
-    if (splitk_applies(M, N, K)) {
-        if (packed) return launch_splitk<false, EpiDequantRes, true, true>(st, At, 0, B, 0, M, N, K, e);
+                                    int K) {
+    const EpiDequantRes e = residual_epi(out, ldo, xs, ws, bias, bias16, res, ldr, rscale);
+    if (splitk_applies(M, N, K))
         return launch_splitk<false, EpiDequantRes, true>(st, At, 0, B, ldb, M, N, K, e);
-    }
-    return hipErrorInvalidValue;
+    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, e);
+}
+
+hipError_t gemm_dequant_residual_packed(hipStream_t st, const int8_t* At, const int8_t* Bp,
+                                        void* out, int64_t ldo, const float* xs, const float* ws,
+                                        const float* bias, const uint16_t* bias16, const void* res,
+                                        int64_t ldr, const void* rscale, int M, int N, int K) {
+    return packed_gemm(st, At, Bp, M, N, K,
+                       residual_epi(out, ldo, xs, ws, bias, bias16, res, ldr, rscale));
 }
 
 hipError_t gemm_i32_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
-                          int32_t* C, int64_t ldc, int M, int N, int K, bool packed) {
-    const EpiI32 epi{C, ldc};
-    if (packed) return launch_pp<true, true>(st, At, 0, B, 0, M, N, K, epi);
-    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, epi);
+                          int32_t* C, int64_t ldc, int M, int N, int K) {
+    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, EpiI32{C, ldc});
+}
+
+hipError_t gemm_i32_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, int32_t* C,
+                           int64_t ldc, int M, int N, int K) {
+    return packed_gemm(st, At, Bp, M, N, K, EpiI32{C, ldc});
 }
 
 hipError_t gemm_act(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,

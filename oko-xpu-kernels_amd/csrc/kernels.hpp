@@ -66,24 +66,26 @@ hipError_t gemm_dequant_nn(hipStream_t st, const int8_t* A, int64_t lda, const i
 // form (gemm_dequant_nn) with B stored [K, N] at row stride ldb
 bool splitk_applies(int M, int N, int K);
 bool splitk_nn_applies(int M, int N, int K, int64_t ldb);
-// the split-K dequant GEMMs with A in the MFMA block layout (tiled_offset);
-// callers check splitk_applies first.  packed: B is pack_weight's copy of the
-// weight (the block layout too; ldb unused)
+// The dequant GEMMs with A in the MFMA block layout (tiled_offset) and B
+// row-major, on the split-K or the persistent kernel (callers check xt_applies)
+bool xt_applies(int M, int N, int K);
 hipError_t gemm_dequant_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                            void* out, int64_t ldo, const float* xs, const float* ws,
-                           const float* bias, const uint16_t* bias16, int M, int N, int K,
-                           bool packed = false);
+                           const float* bias, const uint16_t* bias16, int M, int N, int K);
+// and with B pack_weight's copy of the weight (the block layout too), any
+// shape: the kernel and tile are chosen by it
+hipError_t gemm_dequant_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
+                               int64_t ldo, const float* xs, const float* ws, const float* bias,
+                               const uint16_t* bias16, int M, int N, int K);
+// the NN split-K GEMM (splitk_nn_applies) with A in the block layout; packed:
+// B is pack_weight_nn's copy of the weight
 hipError_t gemm_dequant_nn_xt(hipStream_t st, const int8_t* At, const int8_t* Bkn, int64_t ldb,
                               void* out, int64_t ldo, const float* xs, int M, int N, int K,
                               bool packed = false);
 // whether the persistent ping-pong kernel takes the dequant GEMM (paired:
-// the FFN's up-projection) of this shape, and those GEMMs with A in the MFMA
-// block layout on that kernel
+// the FFN's up-projection) of this shape, and the up-projection with A in the
+// MFMA block layout on that kernel (packed: B is pack_weight's copy)
 bool pp_applies(int M, int N, int K, bool paired);
-hipError_t gemm_dequant_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
-                              void* out, int64_t ldo, const float* xs, const float* ws,
-                              const float* bias, const uint16_t* bias16, int M, int N, int K,
-                              bool packed = false);
 hipError_t gemm_act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                           void* out, int64_t ldo, const float* xs, const float* ws, int M, int N,
                           int K, int act, bool packed = false);
@@ -102,29 +104,31 @@ hipError_t gemm_dequant_residual(hipStream_t st, const int8_t* A, int64_t lda, c
                                  const float* ws, const float* bias, const uint16_t* bias16,
                                  const void* res, int64_t ldr, const void* rscale, int M, int N,
                                  int K);
-// the same two GEMMs with A in the MFMA block layout (packed: B is pack_weight's
-// copy): the residual epilogue on the persistent or the split-K kernel (callers
-// check pp_applies / splitk_applies; other shapes are refused), and the int32
-// product on the persistent kernel (callers check pp_applies)
+// the residual GEMM and the int32 product with A in the MFMA block layout: B
+// row-major (callers check xt_applies, and pp_applies for the int32 one), or
+// pack_weight's copy (any shape)
 hipError_t gemm_dequant_residual_xt(hipStream_t st, const int8_t* At, const int8_t* B,
                                     int64_t ldb, void* out, int64_t ldo, const float* xs,
                                     const float* ws, const float* bias, const uint16_t* bias16,
                                     const void* res, int64_t ldr, const void* rscale, int M, int N,
-                                    int K, bool packed);
+                                    int K);
+hipError_t gemm_dequant_residual_packed(hipStream_t st, const int8_t* At, const int8_t* Bp,
+                                        void* out, int64_t ldo, const float* xs, const float* ws,
+                                        const float* bias, const uint16_t* bias16, const void* res,
+                                        int64_t ldr, const void* rscale, int M, int N, int K);
 hipError_t gemm_i32_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
-                          int32_t* C, int64_t ldc, int M, int N, int K, bool packed);
+                          int32_t* C, int64_t ldc, int M, int N, int K);
+hipError_t gemm_i32_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, int32_t* C,
+                           int64_t ldc, int M, int N, int K);
 // out[m, n] = act(bf16(acc(n) * ws[n] * xs[m]), bf16(acc(N + n) * ws[N + n] * xs[m])) for the
 // paired activations 3 (situ) and 4 (GEGLU), whose B has 2N rows; act 5 (GELU) takes N rows
 hipError_t gemm_act(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,
                     void* out, int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
                     int act, const int8_t* Bp = nullptr);
-// The skinny kernel with x in the MFMA block layout (At) and the packed weight
-// (Bp), for the batches launch_gemm gives it (skinny_applies: M <= 64; paired
-// activations 3 and 4, M <= 256); a linear's callers check gemm_slices first
+// The FFN's up-projection on the skinny kernel with x in the MFMA block layout
+// (At) and the packed weight (Bp), for the batches launch_gemm gives it
+// (skinny_applies: M <= 64; paired activations 3 and 4, M <= 256)
 bool skinny_applies(int M, bool paired);
-hipError_t gemm_dequant_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
-                                  int64_t ldo, const float* xs, const float* ws, const float* bias,
-                                  const uint16_t* bias16, int M, int N, int K);
 hipError_t gemm_act_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
                               int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
                               int act);

@@ -1,0 +1,48 @@
+"""The tiles that products of two block-layout operands take (the packed
+weight): each tile of the persistent kernel at its edges -- ragged rows and
+columns, the shortest K, one round of tiles and several -- with the dequant,
+residual and int32 epilogues.  The reference is the exact integer product in
+float64 and the epilogue's fp32 operations one by one in torch, so the results
+are equal bit for bit."""
+
+import pytest
+import torch
+
+from gpu_util import activation, weight
+from xpu_kernels import int8
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(x, w8, ws, bias, res=None, rscale=None):
+    """(int32 product, bf16 output) from the library's own quantizer (checked
+    against the oracle elsewhere) and plain torch."""
+    q, xs = int8.quantize(x)
+    acc = (q.double() @ w8.double().t()).to(torch.int32)
+    y = acc.float() * (ws[None, :] * xs[:, None])
+    y = (y + bias.float()).to(torch.bfloat16)
+    return acc, y if res is None else torch.addcmul(res, y, rscale)
+
+
+# (M, N, K): 256x320 (one round), 192x320 (one and two rounds), 192x256 (one and
+# two), 192x192 (one, a long K; two), 128x192 (one tile; a lone row group and column
+# block past a tile; several rounds; K = 256), split K (a long K)
+PP_SHAPES = [(4090, 5104, 2048), (1050, 10912, 256), (3000, 10240, 1280), (3974, 3072, 3072),
+             (1355, 6160, 256), (2060, 9232, 1280), (920, 6224, 256), (1541, 3856, 5120),
+             (2323, 6144, 256), (65, 16, 256), (129, 208, 256), (400, 1936, 2048),
+             (2147, 11024, 256), (700, 2064, 6144), (2100, 1296, 5120)]
+
+
+@pytest.mark.parametrize("m,n,k", PP_SHAPES)
+def test_packed_tiles_exact(dev, m, n, k):
+    w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
+    x = activation(m, k, seed=m + k).to(dev)
+    bias = weight(1, n, seed=3, std=0.01)[0].to(dev)
+    res = activation(m, n, seed=m, n_out=0).to(dev)
+    rscale = weight(1, n, seed=4, std=0.5)[0].to(dev)
+    acc, y = reference(x, w8, ws, bias)
+    assert torch.equal(int8.linear(x, w8, ws, bias), y)
+    got, xs = int8.linear_acc(x, w8, ws)
+    assert torch.equal(got, acc)
+    _, yr = reference(x, w8, ws, bias, res, rscale)
+    assert torch.equal(int8.linear(x, w8, ws, bias, residual=res, residual_scale=rscale), yr)
