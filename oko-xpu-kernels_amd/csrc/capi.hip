@@ -243,8 +243,7 @@ size_t linear_work_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 // quantize + GEMM + dequant of xpuint8_linear_stream on checked arguments.
-// wp (optional): pack_weight's copy of w8, read instead of w8 wherever the
-// product is not split in K across blocks.
+// wp (optional): pack_weight's copy of w8, read instead of w8.
 int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_scale,
                const void* bias, int32_t bias_bf16, void* out, int64_t M, int64_t N, int64_t K,
                void* work, const int8_t* wp = nullptr) {
@@ -252,6 +251,13 @@ int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_s
     float* xs = reinterpret_cast<float*>(static_cast<char*>(work) + linear_work_q_bytes(M, K));
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
+    // the packed weight: q in the MFMA block layout too, for every shape
+    if (wp && rowquant_can_tile(int(K))) {
+        XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
+        return launched(gemm_dequant_packed(st, q, wp, out, N, xs, w_scale, b32, b16, int(M),
+                                            int(N), int(K)),
+                        "linear (gemm)");
+    }
     // too few output tiles for the chip: the product split in K across
     // blocks, each slice's int32 partial sums in the workspace, then one pass
     // that adds them and applies the dequant
@@ -264,14 +270,9 @@ int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_s
         return launched(dequant_slices(st, part, N, nsl, M * N, out, xs, w_scale, b32, b16, M, N),
                         "linear (dequant)");
     }
-    // q in the MFMA block layout: for every kernel that reads the packed weight,
-    // and for the split-K and persistent kernels on the row-major one
-    if (rowquant_can_tile(int(K)) && (wp || xt_applies(int(M), int(N), int(K)))) {
+    // the split-K and persistent kernels read q in the MFMA block layout too
+    if (rowquant_can_tile(int(K)) && xt_applies(int(M), int(N), int(K))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
-        if (wp)
-            return launched(gemm_dequant_packed(st, q, wp, out, N, xs, w_scale, b32, b16, int(M),
-                                                int(N), int(K)),
-                            "linear (gemm)");
         return launched(gemm_dequant_xt(st, q, w8, K, out, N, xs, w_scale, b32, b16, int(M),
                                         int(N), int(K)),
                         "linear (gemm)");

@@ -1836,6 +1836,206 @@ hipError_t launch_skinny(hipStream_t st, const int8_t* X, int64_t ldx, const int
     return hipGetLastError();
 }
 
+// ------------------------------------------------------ K split over waves
+// Products too small to fill the chip with LDS-staged tiles: a block of NW
+// waves owns a (16 MB) x (16 NB) tile and its waves take every NW-th 64-byte
+// K step, each holding the whole tile's accumulators.  Both operands come in
+// the MFMA block layout (x from the quantizer, the packed weight), so a
+// fragment of 16 rows is one contiguous 1 KB load straight into registers in
+// the MFMA's own order: no LDS ring, no barrier and no shared pace in the K
+// loop, D steps of MB + NB loads in flight per wave.  What such a product waits
+// for is latency (a chain of K steps behind each other's barriers in the
+// 128 x 128 kernel); here the chain is K / (64 NW) steps long and four
+// to eight of them are in flight at once.  The price is operand traffic: a
+// step loads (MB + NB) KB per MB * NB MFMAs through the CU's 64 bytes per
+// clock, half the matrix cores' rate at 64 x 64, which is why large products stay
+// with the LDS kernels.  Against the kernels that took these products before
+// (the 128 x 128 kernel, or K slices across blocks and a pass that adds them), GEMM
+// alone, us:
+//   1024 x 1280 x 1280 (M, N, K)  19.4 -> 6.3     438 x 496 x 1024   15.2 -> 3.3
+//   1024 x 1280 x 5120            23.0 -> 16.2    135 x 992 x 3840   15.2 -> 4.5
+//   2501 x 880 x 1792             22.4 -> 11.9    128 x 4096 x 4096  16.3 -> 7.7
+//
+// The NW partial sums meet in LDS (exact integer sums).  Each thread then adds
+// and converts eight consecutive columns of one row (lanes l, l + 16, ..: the
+// row's next eight), so a wave's stores leave as 16-byte pieces, 64 bytes of
+// each of 16 rows.
+//
+// Blocks are dealt to the 8 XCDs round robin (block b on XCD b % 8): XCD x
+// takes the rectangle of lm x ln tiles at (x % gx, x / gx) of the tile grid, so
+// that its L2 holds few operand rows (the host picks gx; blocks past the
+// grid's edge leave at once).
+//
+// Paired epilogues: the tile's NB weight blocks are NB/2 column blocks of the
+// first half and the same of the second (epi.half rows further).
+template <int MB, int NB, int NW, int D, class Epi>
+__global__ __launch_bounds__(NW * 64) void gemm_i8_wavek_kernel(
+    const int8_t* __restrict__ X, const int8_t* __restrict__ W, int M, int N, int KB, int tiles_m,
+    int tiles_n, int gx_log2, int lm, int ln, Epi epi) {
+    constexpr bool PAIRED = Epi::kPaired;
+    constexpr int NC = PAIRED ? NB / 2 : NB;                 // output column blocks
+    static_assert(!PAIRED || NB % 2 == 0, "a paired epilogue takes both halves of each block");
+    static_assert(NC % 2 == 0 || NC == 1, "column blocks leave in pairs");
+    static_assert(NW * NB * MB <= 160, "the partial sums fit in the CU's 160 KB of LDS");
+    __shared__ v4i part[NW][NB * MB][64];
+    const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+    const int sq = seq / lm;
+    const int tmi = (xcd & ((1 << gx_log2) - 1)) * lm + (seq - sq * lm);
+    const int tni = (xcd >> gx_log2) * ln + sq;
+    if (tmi >= tiles_m || tni >= tiles_n) return;
+    const int m0 = tmi * 16 * MB, n0 = tni * 16 * NC;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // this lane's chunk of a 1 KB block: row l%16, chunk l/16
+    const uint32_t lo = (lane & 15) * 64 + swz(lane & 15, lane >> 4) * 16;
+    const int64_t kbytes = int64_t(KB) * 1024;
+    const int8_t* xbase[MB];
+    const int8_t* wbase[NB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b)                    // row blocks past M: the last one
+        xbase[b] = X + int64_t(min(m0 / 16 + b, (M - 1) / 16)) * kbytes;
+#pragma unroll
+    for (int p = 0; p < NB; ++p)                    // column blocks past N: the last one
+        wbase[p] = W + int64_t(min(n0 / 16 + (p % NC), (N - 1) / 16) +
+                               (p >= NC ? pair_offset(epi) / 16 : 0)) * kbytes;
+    v4i wbuf[D][NB], xbuf[D][MB];
+    auto load = [&](int slot, int t) {
+        const int64_t k = int64_t(wave + NW * t) * 1024;
+#pragma unroll
+        for (int p = 0; p < NB; ++p)
+            wbuf[slot][p] = *reinterpret_cast<const v4i*>(wbase[p] + k + uint64_t(lo));
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+            xbuf[slot][b] = *reinterpret_cast<const v4i*>(xbase[b] + k + uint64_t(lo));
+    };
+    v4i acc[NB][MB];
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[p][b] = v4i{0, 0, 0, 0};
+    auto mfma = [&](int slot) {
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int p = 0; p < NB; ++p)
+                acc[p][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wbuf[slot][p], xbuf[slot][b],
+                                                                  acc[p][b], 0, 0, 0);
+    };
+    const int n = wave < KB ? (KB - wave + NW - 1) / NW : 0;    // this wave's steps
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+        if (j < n) load(j, j);
+    int t = 0;
+    for (; t + 2 * D <= n; t += D) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            mfma(j);
+            load(j, t + D + j);
+        }
+    }
+    // the last steps: up to D more loads, then none
+#pragma unroll
+    for (int j = 0; j < 2 * D - 1; ++j) {
+        if (t + j < n) {
+            mfma(j % D);
+            if (j < D && t + D + j < n) load(j, t + D + j);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) part[wave][p * MB + b][lane] = acc[p][b];
+    __syncthreads();
+    // item i: row i%16 of m-block mb, its columns 8c..8c+7 (c the chunk); lane l
+    // of a block holds rows 4*(l/16)+i of the weight block (n) for x row l%16 (m)
+    constexpr int CH = NC == 1 ? 2 : 4;             // chunks of a wave's 64 items
+    constexpr int ITEMS = 16 * MB * 2 * NC, STEP = NW * 64;
+#pragma unroll
+    for (int i0 = 0; i0 < ITEMS; i0 += STEP) {
+        const int i = i0 + threadIdx.x;
+        if (ITEMS % STEP != 0 && i >= ITEMS) break;
+        const int row = i & 15, c4 = (i >> 4) & (CH - 1), g = i / (16 * CH);
+        const int mb = g % MB, c = (g / MB) * CH + c4;       // 16-column block c/2, half c%2
+        const int blk = (c >> 1) * MB + mb, l0 = row + 32 * (c & 1);
+        v4i a = part[0][blk][l0], b = part[0][blk][l0 + 16];
+        v4i a2, b2;
+        if constexpr (PAIRED) {
+            a2 = part[0][NC * MB + blk][l0];
+            b2 = part[0][NC * MB + blk][l0 + 16];
+        }
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            a += part[w][blk][l0];
+            b += part[w][blk][l0 + 16];
+            if constexpr (PAIRED) {
+                a2 += part[w][NC * MB + blk][l0];
+                b2 += part[w][NC * MB + blk][l0 + 16];
+            }
+        }
+        const int m = m0 + 16 * mb + row, nn = n0 + 8 * c;
+        if (m >= M || nn >= N) continue;
+        if constexpr (!Epi::kStaged) {
+            epi(m, nn, a);
+            epi(m, nn + 4, b);
+        } else {
+            const float x = epi.row(m);
+            uint2 lo2, hi2;
+            if constexpr (PAIRED) {
+                lo2 = epi.convert2(a, a2, x, epi.col(nn), epi.col(epi.half + nn));
+                hi2 = epi.convert2(b, b2, x, epi.col(nn + 4), epi.col(epi.half + nn + 4));
+            } else {
+                lo2 = epi.convert(a, x, epi.col(nn));
+                hi2 = epi.convert(b, x, epi.col(nn + 4));
+            }
+            epi.store16(m, nn, make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
+        }
+    }
+}
+
+// The kernel's tiles: 16 MB x 16 NB outputs, NW waves, and the blocks of one
+// that a CU holds at once (LDS, registers)
+struct WavekTile {
+    int mb, nb, nw, d, per_cu;
+};
+constexpr WavekTile kWavekTiles[] = {
+    {1, 1, 8, 4, 2}, {1, 2, 4, 4, 6}, {2, 2, 4, 4, 4}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
+
+// Predicted time in us: the fullest CU's operand loads (0.68 us per 100 KB),
+// the chain of each round's K steps (D at a time; 0.2 us each), its reductions
+// (0.28 us per 16 KB of partial sums), and the product's bytes (12 TB/s: caches).  Fitted to 16
+// tiles on 390 products of up to 260 GOP, scatter 10%; the tile it picks of
+// these five is 2% off the fastest of the sixteen on average.
+inline double wavek_time(const WavekTile& t, int64_t M, int64_t N, int K) {
+    const int64_t blocks = ((M + 16 * t.mb - 1) / (16 * t.mb)) * ((N + 16 * t.nb - 1) / (16 * t.nb));
+    const int64_t cus = device_cus(), per = (blocks + cus - 1) / cus;
+    const int64_t rounds = (blocks + cus * t.per_cu - 1) / (cus * t.per_cu);
+    const int KB = (K + 63) / 64, chain = (KB + t.nw * t.d - 1) / (t.nw * t.d);
+    const double bytes = double(M) * K + double(N) * K + 2.0 * double(M) * double(N);
+    return 2.25 + 0.0068 * double(per) * (t.mb + t.nb) * KB + 0.2 * double(rounds) * chain +
+           0.277 / 16 * double(per) * (t.mb * t.nb * t.nw) + 0.082e-6 * bytes;
+}
+
+template <int MB, int NB, int NW, int D, class Epi>
+hipError_t launch_wavek(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N, int K,
+                        const Epi& epi) {
+    constexpr int NC = Epi::kPaired ? NB / 2 : NB;
+    const int tm = (M + 16 * MB - 1) / (16 * MB), tn = (N + 16 * NC - 1) / (16 * NC);
+    // the XCD grid gx x (8 / gx): fewest tiles on the fullest XCD, then fewest
+    // operand rows read by one
+    int best = 0;
+    int64_t cost = 0;
+    for (int g = 0; g < 4; ++g) {
+        const int64_t lm = (tm + (1 << g) - 1) >> g, ln = (tn + (8 >> g) - 1) / (8 >> g);
+        const int64_t c = lm * ln * 4096 + lm * MB + ln * NB;
+        if (g == 0 || c < cost) best = g, cost = c;
+    }
+    const int lm = (tm + (1 << best) - 1) >> best, ln = (tn + (8 >> best) - 1) / (8 >> best);
+    hipLaunchKernelGGL((gemm_i8_wavek_kernel<MB, NB, NW, D, Epi>), dim3(unsigned(8 * lm * ln)),
+                       dim3(NW * 64), 0, st, Xt, Wp, M, N, (K + 63) / 64, tm, tn, best, lm, ln,
+                       epi);
+    return hipGetLastError();
+}
+
 // Tile choice: the 256 x 320 ping-pong tile when it gives at least one tile
 // per CU (8-12% faster than the two-block 256 x 160 kernel at M=4096, K=1280
 // and 2560, N=5120 and 10240, interleaved A/B timing); else the large tile
@@ -1939,9 +2139,28 @@ hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int 
                           const Epi& epi) {
     double t = 0;
     const int tile = pp_tile(M, N, K, &t);
+    bool splitk = false;
     if constexpr (Epi::kStaged) {
-        if (1.03 * splitk_time(M, N, K) < t)
-            return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        const double ts = 1.03 * splitk_time(M, N, K);
+        if (ts < t) splitk = true, t = ts;
+    }
+    // the K-split-over-waves kernel where it is predicted 6% faster (its
+    // prediction scatters more)
+    int wk = -1;
+    for (int i = 0; i < int(sizeof(kWavekTiles) / sizeof(kWavekTiles[0])); ++i) {
+        const double tw = 1.06 * wavek_time(kWavekTiles[i], M, N, K);
+        if (tw < t) wk = i, t = tw;
+    }
+    switch (wk) {
+        case 0: return launch_wavek<1, 1, 8, 4>(st, Xt, Wp, M, N, K, epi);
+        case 1: return launch_wavek<1, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+        case 2: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+        case 3: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
+        case 4: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
+        default: break;
+    }
+    if constexpr (Epi::kStaged) {
+        if (splitk) return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
     }
     switch (tile) {
         case 0: return launch_pp<true, true, 256, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
@@ -2294,7 +2513,10 @@ bool xt_applies(int M, int N, int K) { return splitk_applies(M, N, K) || pp_appl
 template <class Epi>
 static hipError_t packed_gemm(hipStream_t st, const int8_t* At, const int8_t* Bp, int M, int N,
                               int K, const Epi& epi) {
-    if (M <= 64) return launch_skinny<1, Epi, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
+    // 33-64 rows of a narrow, long product have too few 16-column blocks for the
+    // skinny kernel (those whose row-major form is split in K across blocks)
+    if (M <= 64 && skinny_slices(M, N, K) == 0)
+        return launch_skinny<1, Epi, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
     return launch_tiles(st, At, Bp, M, N, K, epi);
 }
 

@@ -24,16 +24,21 @@ def reference(x, w8, ws, bias, res=None, rscale=None):
     return acc, y if res is None else torch.addcmul(res, y, rscale)
 
 
-# (M, N, K): 256x320 (one round), 192x320 (one and two rounds), 192x256 (one and
-# two), 192x192 (one, a long K; two), 128x192 (one tile; a lone row group and column
-# block past a tile; several rounds; K = 256), split K (a long K)
+# (M, N, K): the persistent kernel's 256x320 (one round), 192x320 (one and two
+# rounds), 192x256 (one and two), 192x192 (one, a long K; two), 128x192 (one; four);
+# split K (a long K)
 PP_SHAPES = [(4090, 5104, 2048), (1050, 10912, 256), (3000, 10240, 1280), (3974, 3072, 3072),
              (1355, 6160, 256), (2060, 9232, 1280), (920, 6224, 256), (1541, 3856, 5120),
-             (2323, 6144, 256), (65, 16, 256), (129, 208, 256), (400, 1936, 2048),
-             (2147, 11024, 256), (700, 2064, 6144), (2100, 1296, 5120)]
+             (2323, 6144, 256), (1251, 4752, 3072), (2147, 11024, 256), (4090, 1264, 6144)]
+# the K-split-over-waves kernel's 16x16 (one row block and one column block past
+# the batch; fewer K steps than waves; a long K at 33 rows), 16x32, 32x32, 32x64
+# and 64x64 tiles, each with ragged rows and columns
+WAVEK_SHAPES = [(65, 16, 256), (129, 208, 256), (35, 320, 5120), (64, 1280, 5120),
+                (525, 976, 2048), (438, 496, 1024), (135, 992, 3840), (1000, 1296, 1280),
+                (700, 2064, 6144), (400, 1936, 2048), (1218, 624, 6400), (449, 1696, 256)]
 
 
-@pytest.mark.parametrize("m,n,k", PP_SHAPES)
+@pytest.mark.parametrize("m,n,k", PP_SHAPES + WAVEK_SHAPES)
 def test_packed_tiles_exact(dev, m, n, k):
     w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
     x = activation(m, k, seed=m + k).to(dev)
