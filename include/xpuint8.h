@@ -440,24 +440,37 @@ int64_t xpuint8_column_sum_workspace_size(int64_t M, int64_t N);
 int xpuint8_linear_dw_stream(const void *stream, const void *dy, const void *x, void *dw,
                              int64_t M, int64_t N, int64_t K);
 
+/* The same with a workspace (may be NULL): an output with too few tiles to fill
+ * the GPU has its contraction split across blocks as far as the fp32 partial
+ * sums fit the work_bytes at `work` (16-byte aligned, no clearing needed), added
+ * in a fixed order and rounded once.  xpuint8_linear_dw_workspace_size: the bytes it
+ * would like, 0 for none, -1 when the shape is not supported (no device
+ * needed).  No reference counterpart. */
+int xpuint8_linear_dw_work_stream(const void *stream, const void *dy, const void *x, void *dw,
+                                  int64_t M, int64_t N, int64_t K, void *work,
+                                  int64_t work_bytes);
+int64_t xpuint8_linear_dw_workspace_size(int64_t M, int64_t N, int64_t K);
+
 /* The activation gradient of a linear with a bf16 weight (the dense-mode
  * backward): dx[m,k] = sum_n dy[m,n] * w[n,k], dy bf16 [M,N], w bf16 [N,K]
  * (the unrotated weight, e.g. from xpuint8_dequant_weight_stream), dx bf16
  * [M,K]; fp32 accumulation, one RNE rounding.  N % 16 == 0, K % 16 == 0.
- * `work` may be NULL.  A small batch, whose [M,K] output has too few tiles to
- * fill the GPU, with a `work` of xpuint8_linear_dx_workspace_size(M, N, K)
- * bytes (16-byte aligned; no clearing needed) has the contraction split
- * across blocks: their fp32 partial sums are added in a fixed order, then
- * rounded once, so the result is as above up to the order of the fp32 sum.
+ * `work` may be NULL.  A product whose [M,K] output has too few tiles to fill
+ * the GPU has its contraction split across blocks, as far as the fp32 partial
+ * sums fit the work_bytes at `work` (16-byte aligned; no clearing needed):
+ * they are added in a fixed order, then rounded once, so the result is as
+ * above up to the order of the fp32 sum.
  * Replaces the torch matmul dy @ w of linear_dx
  * (python/xpu_kernels/int8/ops.py:194-204). */
 int xpuint8_linear_dx_stream(const void *stream, const void *dy, const void *w, void *dx,
                              int64_t M, int64_t N, int64_t K, void *work, int64_t work_bytes);
 
-/* The workspace xpuint8_linear_dx_stream uses for this shape, in bytes: 0
- * when the contraction is not split, -1 when the shape is not supported.  No
- * device needed.  A helper of the entry point above (no reference
- * counterpart). */
+/* A workspace for xpuint8_linear_dx_stream, in bytes: fp32 partial sums of a
+ * few slices for a small batch, 0 for others, -1 when the shape is not
+ * supported.  The split_ form gives what the entry point would use if it could
+ * choose (0 when the contraction is best left whole).  No device needed.
+ * Helpers of the entry point above (no reference counterpart). */
+int64_t xpuint8_linear_dx_split_workspace_size(int64_t M, int64_t N, int64_t K);
 int64_t xpuint8_linear_dx_workspace_size(int64_t M, int64_t N, int64_t K);
 
 /* RMSNorm + rotary embedding of q or k read straight from the int32

@@ -917,22 +917,32 @@ int xpuint8_linear_dx_int8_noalloc_stream(const void* stream, const void* dy,
     return dx_chain(as_stream(stream), dy, w_scale, w8, dx, M, N, K, g_scratch[dev]);
 }
 
-int xpuint8_linear_dw_stream(const void* stream, const void* dy, const void* x, void* dw,
-                             int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return fail(2, "M, N and K must be positive");
-    if (N % 16 != 0 || K % 16 != 0) return fail(2, "N and K must be multiples of 16");
-    if (M > kMaxDim || N > kMaxDim || K > kMaxDim) return fail(4, "M, N and K must be < 2^31");
-    XPU_NONNULL(dy); XPU_NONNULL(x); XPU_NONNULL(dw);
-    XPU_TRY(ensure_device());
-    return launched(gemm_bf16_tn(as_stream(stream), dy, N, x, K, dw, K, int(M), int(N), int(K)),
-                    "linear_dw");
-}
-
 static int check_linear_dx(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0) return fail(2, "M, N and K must be positive");
     if (N % 16 != 0 || K % 16 != 0) return fail(2, "N and K must be multiples of 16");
     if (M > kMaxDim || N > kMaxDim || K > kMaxDim) return fail(4, "M, N and K must be < 2^31");
     return 0;
+}
+
+int64_t xpuint8_linear_dw_workspace_size(int64_t M, int64_t N, int64_t K) {
+    if (check_linear_dx(M, N, K) != 0) return -1;
+    return bf16_dw_work_bytes(int(M), int(N), int(K));
+}
+
+int xpuint8_linear_dw_work_stream(const void* stream, const void* dy, const void* x, void* dw,
+                                  int64_t M, int64_t N, int64_t K, void* work,
+                                  int64_t work_bytes) {
+    XPU_TRY(check_linear_dx(M, N, K));
+    XPU_NONNULL(dy); XPU_NONNULL(x); XPU_NONNULL(dw); XPU_ALIGNED_OPT(work);
+    XPU_TRY(ensure_device());
+    return launched(gemm_bf16_tn(as_stream(stream), dy, N, x, K, dw, K, int(M), int(N), int(K),
+                                 static_cast<float*>(work), work_bytes),
+                    "linear_dw");
+}
+
+int xpuint8_linear_dw_stream(const void* stream, const void* dy, const void* x, void* dw,
+                             int64_t M, int64_t N, int64_t K) {
+    return xpuint8_linear_dw_work_stream(stream, dy, x, dw, M, N, K, nullptr, 0);
 }
 
 int64_t xpuint8_linear_dx_workspace_size(int64_t M, int64_t N, int64_t K) {
@@ -941,18 +951,18 @@ int64_t xpuint8_linear_dx_workspace_size(int64_t M, int64_t N, int64_t K) {
     return nsl > 0 ? int64_t(nsl) * M * K * 4 : 0;
 }
 
+int64_t xpuint8_linear_dx_split_workspace_size(int64_t M, int64_t N, int64_t K) {
+    if (check_linear_dx(M, N, K) != 0) return -1;
+    return bf16_dx_work_bytes(int(M), int(N), int(K));
+}
+
 int xpuint8_linear_dx_stream(const void* stream, const void* dy, const void* w, void* dx,
                              int64_t M, int64_t N, int64_t K, void* work, int64_t work_bytes) {
     XPU_TRY(check_linear_dx(M, N, K));
     XPU_NONNULL(dy); XPU_NONNULL(w); XPU_NONNULL(dx); XPU_ALIGNED_OPT(work);
     XPU_TRY(ensure_device());
-    // a small batch with a workspace: the contraction split across blocks
-    const int nsl = bf16_nn_slices(int(M), int(N), int(K));
-    if (nsl > 0 && work != nullptr && work_bytes >= int64_t(nsl) * M * K * 4)
-        return launched(gemm_bf16_nn_slices(as_stream(stream), dy, N, w, K, dx, K, int(M), int(N),
-                                            int(K), static_cast<float*>(work), nsl),
-                        "linear_dx");
-    return launched(gemm_bf16_nn(as_stream(stream), dy, N, w, K, dx, K, int(M), int(N), int(K)),
+    return launched(gemm_bf16_nn(as_stream(stream), dy, N, w, K, dx, K, int(M), int(N), int(K),
+                                 static_cast<float*>(work), work_bytes),
                     "linear_dx");
 }
 
@@ -968,8 +978,7 @@ static DenseBwdWork dense_bwd_layout(int64_t M, int64_t N, int64_t K) {
     w.wd = 0;
     w.colsum = up(2 * N * K);
     w.part = w.colsum + up(colsum_work_bytes(M, N));
-    const int nsl = bf16_nn_slices(int(M), int(N), int(K));
-    w.total = w.part + (nsl > 0 ? size_t(nsl) * size_t(M) * size_t(K) * 4 : 0);
+    w.total = w.part + size_t(bf16_dx_work_bytes(int(M), int(N), int(K)));
     return w;
 }
 
@@ -1000,11 +1009,9 @@ int xpuint8_linear_backward_dense_stream(const void* stream, const void* dy, con
     void* wd = w + L.wd;
     XPU_TRY(launched(dequant_weight(st, w8, w_scale, wd, N, int(K)),
                      "linear_backward_dense (dequant_weight)"));
-    if (const int nsl = bf16_nn_slices(int(M), int(N), int(K)))
-        return launched(gemm_bf16_nn_slices(st, dy, N, wd, K, dx, K, int(M), int(N), int(K),
-                                            reinterpret_cast<float*>(w + L.part), nsl),
-                        "linear_backward_dense (gemm)");
-    return launched(gemm_bf16_nn(st, dy, N, wd, K, dx, K, int(M), int(N), int(K)),
+    return launched(gemm_bf16_nn(st, dy, N, wd, K, dx, K, int(M), int(N), int(K),
+                                 reinterpret_cast<float*>(w + L.part),
+                                 int64_t(L.total - L.part)),
                     "linear_backward_dense (gemm)");
 }
 

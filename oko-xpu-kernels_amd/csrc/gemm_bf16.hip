@@ -20,6 +20,8 @@
 // D = A * B with A from x (D rows = k) and B from dy (D columns = n), so lane
 // l of a 16x16 block holds D[4(l/16)+i][l%16]: four consecutive k of one dw
 // row, stored as one 8-byte write.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -37,15 +39,6 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 __device__ __attribute__((aligned(16))) int8_t g_zero_line[16];
 
 constexpr int kStepRows = 32;                // reduction rows per MFMA step
-constexpr int kRegion = kStepRows * 256;     // 32 rows x 128 bf16 columns = 8 KB
-
-// A region row is 256 bytes = 16 chunks of 16 bytes, i.e. one pass over the
-// 64 four-byte LDS banks; chunk c of row r sits at position c ^ swz(r).  A
-// transposing read touches 16 rows, 8g + 4h + q (g, q = 0..3), and two
-// adjacent chunks (8 banks) in each: swz takes 8 distinct even values over
-// (q, g & 1), so the rows' chunk pairs cover all 64 banks twice -- the
-// minimum two cycles for the read's 512 bytes.
-__device__ __forceinline__ int swz(int r) { return 2 * ((r & 3) | (((r >> 3) & 1) << 2)); }
 
 __device__ __forceinline__ void dma16(const int8_t* gsrc, int8_t* ldst) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -59,14 +52,16 @@ __device__ __forceinline__ void dma16(const int8_t* gsrc, int8_t* ldst) {
 // load writes, and waits for *all* outstanding loads before it -- including
 // the stage just issued, which removes the pipelining.  Here the ring's own
 // vmcnt waits (before each barrier) order the loads; the reads' completion is
-// awaited by lds_wait() below before any fragment is used.
+// awaited (lgkmcnt) before any fragment is used.
 __device__ __forceinline__ uint32_t lds_addr(const int8_t* p) {
     return static_cast<uint32_t>(
         reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const int8_t*)p));
 }
-__device__ __forceinline__ v4s tr_read(uint32_t addr) {
+template <int OFF>
+__device__ __forceinline__ v4s tr_read_at(uint32_t addr) {
+    static_assert(OFF >= 0 && OFF < 65536, "ds offset field");
     v4s r;
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
     return r;
 }
 
@@ -79,300 +74,11 @@ __host__ __device__ constexpr int vmcnt_imm(int n) {
     return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8);
 }
 
-// One 128 (k) x 128 (n) tile per block of 4 waves (2 x 2, 64 x 64 each); the
-// reduction runs in steps of 32 rows through a ring of STAGES LDS stages (x
-// region, then dy region), filled STAGES-1 steps ahead.
-template <int STAGES>
-__global__ __launch_bounds__(256, 2) void gemm_bf16_tn_kernel(
-    const uint16_t* __restrict__ X, int64_t ldx, const uint16_t* __restrict__ Y, int64_t ldy,
-    uint16_t* __restrict__ out, int64_t ldo, int R, int K, int N, int tiles_k, int tiles_n) {
-    constexpr int BKD = 128, BND = 128;                 // D rows (k), D columns (n) per tile
-    constexpr int TM = 4, TN = 4;                       // 16x16 blocks per wave
-    constexpr int STAGE = 2 * kRegion;
-    __shared__ __attribute__((aligned(1024))) int8_t smem[STAGES * STAGE];
-
-    const int tiles = tiles_k * tiles_n;
-    int t = blockIdx.x;
-    if (tiles % 8 == 0) t = (t % 8) * (tiles / 8) + t / 8;   // each XCD a contiguous range
-    const int k0 = (t % tiles_k) * BKD, n0 = (t / tiles_k) * BND;
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-
-    // DMA: a stage is 16 blocks of 1 KB (4 rows x 256 bytes): blocks 0..7 the
-    // x region, 8..15 the dy region; wave w brings blocks w, w+4, w+8, w+12.
-    // Lane l fills row r = 4*(b%8) + l/16, position l%16, i.e. source chunk
-    // (l%16) ^ swz(r).  Columns past K / N repeat a valid chunk (their results
-    // are not stored); rows past R read zeros.
-    const int8_t* src[4];
-    int srow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int b = wave + 4 * i;
-        srow[i] = 4 * (b & 7) + (lane >> 4);
-        const int dchunk = (lane & 15) ^ swz(srow[i]);
-        if (i < 2) {
-            const int col = min(k0 + dchunk * 8, K - 8);
-            src[i] = reinterpret_cast<const int8_t*>(X + col);
-        } else {
-            const int col = min(n0 + dchunk * 8, N - 8);
-            src[i] = reinterpret_cast<const int8_t*>(Y + col);
-        }
-    }
-    auto issue = [&](int buf, int step) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = step * kStepRows + srow[i];
-            const int64_t ld = i < 2 ? ldx : ldy;
-            const int8_t* p = row < R ? src[i] + int64_t(row) * ld * 2 : g_zero_line;
-            dma16(p, smem + buf * STAGE + (wave + 4 * i) * 1024);
-        }
-    };
-
-    // transposing-read offsets: lane l (group g, index j) reads row
-    // 8g + 4h + j/4 (h = 0, 1), 8 bytes at column 16*blk + 4*(j%4)
-    const int g = lane >> 4, j = lane & 15;
-    uint32_t roff[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) roff[h] = (8 * g + 4 * h + (j >> 2)) * 256 + 8 * (j & 1);
-    const int cpair = (j & 3) >> 1;             // chunk within the block's two
-    const int rs = swz(8 * g + (j >> 2));       // swz of the rows read (h does not change it)
-    const uint32_t sbase = lds_addr(smem);
-    // fragment halves: lo = reduction rows +0..3, hi = +4..7 of the lane's 8
-    auto frag_read = [&](uint32_t region, int blk, v4s& lo, v4s& hi) {
-        const uint32_t pos = ((2 * blk + cpair) ^ rs) * 16;
-        lo = tr_read(region + roff[0] + pos);
-        hi = tr_read(region + roff[1] + pos);
-    };
-    auto join = [](const v4s& lo, const v4s& hi) {
-        const v8s v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        return __builtin_bit_cast(v8bf, v);
-    };
-
-    v4f acc[TN][TM];
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    const int RS = (R + kStepRows - 1) / kStepRows;
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-        if (s < RS) issue(s, s);
-#pragma clang loop unroll(disable)
-    for (int st = 0; st < RS; ++st) {
-        const int later = min(RS - 1 - st, STAGES - 2);
-        if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(8));
-        else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(4));
-        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __builtin_amdgcn_s_barrier();
-        // the buffer refilled now was read at step st-1, before this barrier
-        if (st + STAGES - 1 < RS) issue((st + STAGES - 1) % STAGES, st + STAGES - 1);
-        const uint32_t sb = sbase + (st % STAGES) * STAGE;
-        v4s al[TM], ah[TM], bl[TN], bh[TN];
-#pragma unroll
-        for (int b = 0; b < TM; ++b) frag_read(sb, wm * TM + b, al[b], ah[b]);
-#pragma unroll
-        for (int a = 0; a < TN; ++a) frag_read(sb + kRegion, wn * TN + a, bl[a], bh[a]);
-        // every read has landed before any fragment is used (the operands tie
-        // the fragments to this wait, so no use can be scheduled above it)
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(al[0]), "+v"(al[1]), "+v"(al[2]), "+v"(al[3]), "+v"(ah[0]),
-                       "+v"(ah[1]), "+v"(ah[2]), "+v"(ah[3]), "+v"(bl[0]), "+v"(bl[1]),
-                       "+v"(bl[2]), "+v"(bl[3]), "+v"(bh[0]), "+v"(bh[1]), "+v"(bh[2]),
-                       "+v"(bh[3]));
-        v8bf af[TM], bf[TN];
-#pragma unroll
-        for (int b = 0; b < TM; ++b) af[b] = join(al[b], ah[b]);
-#pragma unroll
-        for (int a = 0; a < TN; ++a) bf[a] = join(bl[a], bh[a]);
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b], bf[a], acc[a][b], 0, 0, 0);
-    }
-
-    // lane l of block (a, b): dw row n = n0 + 64 wn + 16a + l%16,
-    // columns k = k0 + 64 wm + 16b + 4(l/16) .. +3
-#pragma unroll
-    for (int a = 0; a < TN; ++a) {
-        const int n = n0 + wn * 64 + 16 * a + (lane & 15);
-        if (n >= N) continue;
-#pragma unroll
-        for (int b = 0; b < TM; ++b) {
-            const int k = k0 + wm * 64 + 16 * b + 4 * (lane >> 4);
-            if (k < K) {
-                const v4f v = acc[a][b];
-                *reinterpret_cast<uint2*>(out + int64_t(n) * ldo + k) =
-                    make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
-            }
-        }
-    }
-}
-
-// The activation gradient of a linear with a bf16 weight, the dense-mode dx:
-//
-//   out[m, k] = sum_n dy[m, n] * w[n, k]      dy bf16 [M, N], w bf16 [N, K]
-//
-// (python/xpu_kernels/int8/ops.py:194-204, dy @ w).  The weight is contracted
-// along its rows, like both operands above, and goes through the same x
-// region and transposing reads (D rows = k).  dy is contracted along its
-// contiguous dimension: its region holds 128 rows (m) of one 32-element
-// (64-byte) step, and lane l's B fragment, dy[m][8(l/16)..+7] of row
-// m = l%16 of a block, is one plain 16-byte read.  Chunk c of region row r
-// sits at position c ^ swz_dy(r); the 16 rows a read touches then cover the
-// 64 banks exactly once.  Lane l of a 16x16 block holds D[4(l/16)+i][l%16]:
-// four consecutive k of one output row, one 8-byte store.
-__device__ __forceinline__ int swz_dy(int r) { return (r >> 2) & 3; }
-
-__device__ __forceinline__ v8bf plain_read(uint32_t addr) {
-    v8s r;
-    asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr));
-    return __builtin_bit_cast(v8bf, r);
-}
-
-template <int STAGES>
-__global__ __launch_bounds__(256, 2) void gemm_bf16_nn_kernel(
-    const uint16_t* __restrict__ W, int64_t ldw, const uint16_t* __restrict__ Y, int64_t ldy,
-    uint16_t* __restrict__ out, int64_t ldo, int R, int K, int M, int tiles_k, int tiles_m) {
-    constexpr int BKD = 128, BMD = 128;                 // D rows (k), D columns (m) per tile
-    constexpr int TM = 4, TN = 4;                       // 16x16 blocks per wave
-    constexpr int STAGE = 2 * kRegion;
-    __shared__ __attribute__((aligned(1024))) int8_t smem[STAGES * STAGE];
-
-    const int tiles = tiles_k * tiles_m;
-    int t = blockIdx.x;
-    if (tiles % 8 == 0) t = (t % 8) * (tiles / 8) + t / 8;   // each XCD a contiguous range
-    const int k0 = (t % tiles_k) * BKD, m0 = (t / tiles_k) * BMD;
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-
-    // DMA: blocks 0..7 of a stage are the weight region (as in the TN kernel:
-    // 4 rows x 256 bytes each), blocks 8..15 the dy region (16 rows x 64
-    // bytes each).  Lane l of a dy block fills row r = 16*(b-8) + l/4,
-    // position l%4, i.e. chunk (l%4) ^ swz_dy(r) of the step: columns past R
-    // read zeros, rows past M repeat the last row (not stored).
-    const int8_t* src[4];
-    int srow[4];
-    int scol[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int b = wave + 4 * i;
-        if (i < 2) {
-            srow[i] = 4 * (b & 7) + (lane >> 4);
-            const int dchunk = (lane & 15) ^ swz(srow[i]);
-            const int col = min(k0 + dchunk * 8, K - 8);
-            src[i] = reinterpret_cast<const int8_t*>(W + col);
-            scol[i] = 0;
-        } else {
-            const int r = 16 * (b - 8) + (lane >> 2);
-            srow[i] = r;
-            const int m = min(m0 + r, M - 1);
-            src[i] = reinterpret_cast<const int8_t*>(Y + int64_t(m) * ldy);
-            scol[i] = 8 * ((lane & 3) ^ swz_dy(r));
-        }
-    }
-    auto issue = [&](int buf, int step) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int8_t* p;
-            if (i < 2) {
-                const int row = step * kStepRows + srow[i];
-                p = row < R ? src[i] + int64_t(row) * ldw * 2 : g_zero_line;
-            } else {
-                const int col = step * kStepRows + scol[i];
-                p = col < R ? src[i] + int64_t(col) * 2 : g_zero_line;
-            }
-            dma16(p, smem + buf * STAGE + (wave + 4 * i) * 1024);
-        }
-    };
-
-    // weight fragments: the TN kernel's transposing reads
-    const int g = lane >> 4, j = lane & 15;
-    uint32_t roff[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) roff[h] = (8 * g + 4 * h + (j >> 2)) * 256 + 8 * (j & 1);
-    const int cpair = (j & 3) >> 1;
-    const int rs = swz(8 * g + (j >> 2));
-    const uint32_t sbase = lds_addr(smem);
-    auto frag_read = [&](uint32_t region, int blk, v4s& lo, v4s& hi) {
-        const uint32_t pos = ((2 * blk + cpair) ^ rs) * 16;
-        lo = tr_read(region + roff[0] + pos);
-        hi = tr_read(region + roff[1] + pos);
-    };
-    auto join = [](const v4s& lo, const v4s& hi) {
-        const v8s v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        return __builtin_bit_cast(v8bf, v);
-    };
-    // dy fragments: row 16*blk + j of the region, chunk g
-    const uint32_t dyoff = j * 64 + ((g ^ swz_dy(j)) * 16);
-
-    v4f acc[TN][TM];
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    const int RS = (R + kStepRows - 1) / kStepRows;
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-        if (s < RS) issue(s, s);
-#pragma clang loop unroll(disable)
-    for (int st = 0; st < RS; ++st) {
-        const int later = min(RS - 1 - st, STAGES - 2);
-        if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(8));
-        else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(4));
-        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __builtin_amdgcn_s_barrier();
-        if (st + STAGES - 1 < RS) issue((st + STAGES - 1) % STAGES, st + STAGES - 1);
-        const uint32_t sb = sbase + (st % STAGES) * STAGE;
-        v4s al[TM], ah[TM];
-        v8bf bf[TN];
-#pragma unroll
-        for (int b = 0; b < TM; ++b) frag_read(sb, wm * TM + b, al[b], ah[b]);
-#pragma unroll
-        for (int a = 0; a < TN; ++a) bf[a] = plain_read(sb + kRegion + (wn * TN + a) * 1024 + dyoff);
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(al[0]), "+v"(al[1]), "+v"(al[2]), "+v"(al[3]), "+v"(ah[0]),
-                       "+v"(ah[1]), "+v"(ah[2]), "+v"(ah[3]), "+v"(bf[0]), "+v"(bf[1]),
-                       "+v"(bf[2]), "+v"(bf[3]));
-        v8bf af[TM];
-#pragma unroll
-        for (int b = 0; b < TM; ++b) af[b] = join(al[b], ah[b]);
-#pragma unroll
-        for (int a = 0; a < TN; ++a)
-#pragma unroll
-            for (int b = 0; b < TM; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[b], bf[a], acc[a][b], 0, 0, 0);
-    }
-
-    // lane l of block (a, b): output row m = m0 + 64 wn + 16a + l%16,
-    // columns k = k0 + 64 wm + 16b + 4(l/16) .. +3
-#pragma unroll
-    for (int a = 0; a < TN; ++a) {
-        const int m = m0 + wn * 64 + 16 * a + (lane & 15);
-        if (m >= M) continue;
-#pragma unroll
-        for (int b = 0; b < TM; ++b) {
-            const int k = k0 + wm * 64 + 16 * b + 4 * (lane >> 4);
-            if (k < K) {
-                const v4f v = acc[a][b];
-                *reinterpret_cast<uint2*>(out + int64_t(m) * ldo + k) =
-                    make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
-            }
-        }
-    }
-}
-
 // ---------------------------------------------------------------- split K
 // Narrow outputs with a long contraction: the dense dx (C5: M = 4096 rows,
 // K = 1280 outputs, R = 5120 contraction rows) and dW (N = 5120 rows, K = 1280,
-// R = 4096).  There the 128 x 128 tiles above make 320 (400) blocks for 256
-// CUs, and the CUs that run two of them set the time.  Here one block of 8
+// R = 4096), where 128 x 192 tiles of the persistent kernel below leave CUs idle
+// (66.9 against 58.8 us for the dx, 61.9 against 54.9 for dW).  One block of 8
 // waves owns a BB x 160 tile of out[b, k] (256 tiles at C5 for both), in two
 // teams of 4 (2 x 2 waves of BB/2 x 80): team t owns half of the 32-row
 // contraction steps through its own ring of S LDS stages, and the teams
@@ -407,13 +113,6 @@ __device__ __forceinline__ int swz_y(int r, int c) { return c ^ ((r >> 1) & 3); 
 __device__ __forceinline__ int chunk_at(int r, int c) { return 4 * r + (c ^ ((r >> 2) & 2)); }
 
 template <int OFF>
-__device__ __forceinline__ v4s tr_read_at(uint32_t addr) {
-    static_assert(OFF >= 0 && OFF < 65536, "ds offset field");
-    v4s r;
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
-    return r;
-}
-template <int OFF>
 __device__ __forceinline__ v8s plain_read_at(uint32_t addr) {
     static_assert(OFF >= 0 && OFF < 65536, "ds offset field");
     v8s r;
@@ -421,20 +120,10 @@ __device__ __forceinline__ v8s plain_read_at(uint32_t addr) {
     return r;
 }
 
-// SL: contraction slice blockIdx.y of a split across blocks (dense dx only):
-// R is the slice's length, A's rows and Y's columns are offset to it, and the
-// slice's fp32 partial sums go to (float*)out + blockIdx.y * sl_stride
-// instead of the bf16 output.
-template <int S, bool YT, bool SL = false>
+template <int S, bool YT>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_splitk_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ Y, int64_t ldy,
-    uint16_t* __restrict__ out, int64_t ldo, int R, int K, int NBR, int tiles_b, int tiles_k,
-    int64_t sl_stride = 0) {
-    static_assert(!SL || !YT, "contraction slices for the dense dx");
-    if constexpr (SL) {
-        A += int64_t(blockIdx.y) * R * lda;
-        Y += int64_t(blockIdx.y) * R;
-    }
+    uint16_t* __restrict__ out, int64_t ldo, int R, int K, int NBR, int tiles_b, int tiles_k) {
     constexpr int BK = 160, TK = 5;                     // A side: k columns, blocks per wave
     constexpr int TB = YT ? 5 : 4, BB = 32 * TB;        // B side: blocks per wave, tile rows
     constexpr int AB = BK / 16, YB = BB / 16, NB = AB + YB;
@@ -701,19 +390,380 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_splitk_kernel(
                 const int k = k0 + wk * 80 + 16 * a + 4 * (lane >> 4);
                 if (k < K) {
                     const v4f v = acc[a][b];
-                    if constexpr (SL)
-                        *reinterpret_cast<v4f*>(reinterpret_cast<float*>(out) +
-                                                int64_t(blockIdx.y) * sl_stride +
-                                                int64_t(row) * ldo + k) = v;
-                    else
-                        *reinterpret_cast<uint2*>(out + int64_t(row) * ldo + k) =
-                            make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
+                    *reinterpret_cast<uint2*>(out + int64_t(row) * ldo + k) =
+                        make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
                 }
             }
         }
     };
     if (team == 0) finish(std::integral_constant<int, 0>{});
     else finish(std::integral_constant<int, 1>{});
+}
+
+// ------------------------------------------------------------ large outputs
+// Products with at least a round of large tiles: the persistent ping-pong
+// scheme of the int8 GEMM in bf16, one block of 8 waves per CU over BB x BC
+// tiles of out[b, c], in two groups of 4 waves (the tile's row halves) that
+// alternate between MFMAs and data movement every half step, through a ring of
+// four LDS slots of one 32-row contraction step that runs on from tile to tile.
+//   phase A(s): group 0 runs step s's MFMAs; group 1 reads step s's fragments
+//               and issues its loads for step s + 3
+//   phase B(s): group 1 runs step s's MFMAs; group 0 reads step s + 1's
+//               fragments and issues its loads for step s + 3
+// A slot is refilled only after its last reader's phase, a step is complete
+// (each wave waits for its own loads, then the barrier) before its first.
+//
+// The split-K kernel above gives a 128 x 160 tile 18 KB of operands per 32-row
+// step for 320 clocks of MFMA per SIMD, more than the direct-to-LDS path
+// moves (32-40 bytes per clock for row segments); a 256 x 320 tile needs 36 KB for
+// 1280 clocks.  A wave's accumulators are the same 160 registers at
+// 128 x 80 as there the whole block's.
+//
+// Operands in a slot (1 KB blocks, one direct-to-LDS load each):
+//   contracted along its rows (a; y too with YT): 8 rows x 64 columns, so that
+//     a load is 8 whole cache lines (16 x 64 bytes: 16 halves); block 4cg + rb
+//     holds rows 8rb.. of columns 64cg..; the 32-byte chunk pair p of row r at
+//     pair p ^ (2 ((r >> 1) & 1) + (rb & 1)), which puts the 8 row pieces that half a
+//     wave's transposing read touches on distinct banks;
+//   contracted along its columns (y of the dx): 16 rows x 64 bytes as in the
+//     split-K kernel.
+// Rows of the contraction past R are read as zeros from both operands.
+//
+// SL: contraction slice blockIdx.y of a split across blocks, `slice` (a multiple
+// of 32) long but the last: a and y are offset to it, and its fp32 sums go to
+// (float*)out + blockIdx.y * sl_stride instead of the bf16 output.
+// Off: the lanes' byte offsets from a block's first row, at most 15 rows
+// (uint32_t; uint64_t for leading dimensions past 2^27).
+// fragments b = 0 .. COUNT-1 of a plainly read operand, 1 KB apart
+template <int COUNT, int I = 0, int NF>
+__device__ __forceinline__ void plain_read_frags(v8s (&f)[NF], uint32_t addr) {
+    if constexpr (I < COUNT) {
+        f[I] = plain_read_at<I * 1024>(addr);
+        plain_read_frags<COUNT, I + 1>(f, addr);
+    }
+}
+
+template <int BB, int BC, int WGM, bool YT, bool SL, class Off = uint32_t>
+__global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(
+    const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ Y, int64_t ldy,
+    uint16_t* __restrict__ out, int64_t ldo, int R, int NC, int NBR, int tiles_b, int tiles_c,
+    int slice, int64_t sl_stride) {
+    if constexpr (SL) {
+        const int64_t r0 = int64_t(blockIdx.y) * slice;
+        A += r0 * lda;
+        Y += YT ? r0 * ldy : r0;
+        R = min(slice, R - int(r0));
+    }
+    constexpr int NW = 8, WGN = NW / WGM, S = 4;
+    static_assert(WGM % 2 == 0 && WGM * WGN == NW, "two groups of four waves (row halves)");
+    constexpr int WB = BB / WGM, WC = BC / WGN, TB = WB / 16, TC = WC / 16;
+    static_assert(BC % 64 == 0 && (!YT || BB % 64 == 0), "whole 64-column blocks");
+    constexpr int YB = BB / 16, CB = BC / 16, NB = YB + CB;    // 1 KB blocks per slot
+    constexpr int PER = (NB + NW - 1) / NW, REM = NB % NW;
+    static_assert(REM == 0 || REM == 4, "group 0 issues PER, group 1 PER or PER - 1");
+    constexpr int STAGE = NB * 1024, RING = S * STAGE;
+    // the epilogue's staging (16 rows x 256 bytes per wave): the slot of the
+    // tile's last step, or an area of its own where a slot is smaller
+    constexpr int STG = NW * 16 * 256, STG_OWN = STG > STAGE ? STG : 0;
+    static_assert(RING + STG_OWN <= 160 * 1024, "LDS");
+    static_assert(WC <= 128, "staged rows of at most 256 bytes");
+    __shared__ __attribute__((aligned(1024))) int8_t smem[RING + STG_OWN];
+
+    const int tiles = tiles_b * tiles_c;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wb = wave / WGN, wc = wave % WGN;
+    const int grp = wb / (WGM / 2);
+    const bool full_share = REM == 0 || grp == 0;
+
+    // tile origin of sequence number i: XCD i % 8 takes a contiguous eighth of
+    // the tiles (rounded up), in bands of 8 row tiles; false past its share
+    const int share = (tiles + 7) / 8;
+    auto tile_origin = [&](int i, int& b0, int& c0) {
+        const int t = (i % 8) * share + i / 8;
+        if (i / 8 >= share || t >= tiles) return false;
+        constexpr int GROUP = 8;
+        const int band = t / (GROUP * tiles_c);
+        const int first = band * GROUP;
+        const int gm = min(tiles_b - first, GROUP);
+        const int in_band = t - band * GROUP * tiles_c;
+        b0 = (first + in_band % gm) * BB;
+        c0 = (in_band / gm) * BC;
+        return true;
+    };
+
+    const int ST = (R - 1) / kStepRows + 1;
+    const int8_t* base[PER];
+    Off off[PER];
+    auto setup = [&](int b0, int c0) {
+        int ln;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int j = min(wave + NW * i, NB - 1);
+            if (!YT && j < YB) {
+                const int r = ln >> 2, c = swz_y(r, ln & 3);
+                // (blocks past the last row repeat it)
+                const int r0 = min(b0 + 16 * j, NBR - 1);
+                base[i] = reinterpret_cast<const int8_t*>(Y + int64_t(r0) * ldy);
+                off[i] = Off(min(r, NBR - 1 - r0)) * Off(ldy) * 2u + 16 * c;
+            } else {
+                const bool isy = j < YB;
+                const int jj = isy ? j : j - YB, cg = jj >> 2, rb = jj & 3;
+                const int r = ln >> 3, p = ln & 7;
+                const int c = 2 * ((p >> 1) ^ (2 * ((r >> 1) & 1) + (rb & 1))) + (p & 1);
+                const int o0 = isy ? b0 : c0, lim = isy ? NBR : NC;
+                const int64_t ld = isy ? ldy : lda;
+                base[i] = reinterpret_cast<const int8_t*>((isy ? Y : A) + o0 + 8 * rb * ld);
+                off[i] = Off(r) * Off(ld) * 2u + Off(min(o0 + 64 * cg + 8 * c, lim - 8) - o0) * 2u;
+            }
+        }
+    };
+    int ring0 = 0;                              // number of the tile's first step, mod S
+    auto slot = [&](int s) { return ((ring0 + s + 1) & (S - 1)) * STAGE; };
+    // this wave's loads of step `step` of the tile set up last, into ring position s
+    auto issue_at = [&](int s, int step) {
+        int8_t* const st = smem + slot(s);
+        const int64_t arow = int64_t(step) * kStepRows * lda * 2;
+        const int64_t yrow = YT ? int64_t(step) * kStepRows * ldy * 2 : int64_t(step) * 64;
+        const int left = R - step * kStepRows;  // rows of the step
+        if (left >= kStepRows) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                if (i == PER - 1 && !full_share) continue;
+                const int j = wave + NW * i;
+                dma16(base[i] + (j < YB ? yrow : arow) + uint64_t(off[i]), st + j * 1024);
+            }
+        } else {
+            // the last, partial step: the lane's contraction index within it (its
+            // row, or the first of its eight columns) past R reads zeros
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                if (i == PER - 1 && !full_share) continue;
+                const int j = wave + NW * i;
+                const int r = !YT && j < YB ? 8 * swz_y(lane >> 2, lane & 3)
+                                            : 8 * ((j < YB ? j : j - YB) & 3) + (lane >> 3);
+                const int8_t* p = base[i] + (j < YB ? yrow : arow) + uint64_t(off[i]);
+                if (r >= left) p = g_zero_line;
+                dma16(p, st + j * 1024);
+            }
+        }
+    };
+    auto wait_batches = [&](int later) {
+        if (full_share) {
+            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * PER));
+            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        } else {
+            if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * (PER - 1)));
+            else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(PER - 1));
+            else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        }
+    };
+
+    // fragment addresses within a slot: transposing reads of the 16-column
+    // block blk of a row-contracted operand whose blocks start at `first`
+    // (+512: the other four rows of each eight); plain 16-byte reads of dy
+    const int g = lane >> 4, jl = lane & 15;
+    auto tr_off = [&](int first, int blk) {
+        const int cg = blk >> 2, sub = blk & 3;
+        const int pair = sub ^ (2 * ((jl >> 3) & 1) + (g & 1));
+        return uint32_t((first + 4 * cg + g) * 1024 + (jl >> 2) * 128 + 32 * pair +
+                        16 * ((jl & 3) >> 1) + 8 * (jl & 1));
+    };
+    uint32_t aoff[TC], ytoff[YT ? TB : 1];
+#pragma unroll
+    for (int a = 0; a < TC; ++a) aoff[a] = tr_off(YB, wc * TC + a);
+    if constexpr (YT) {
+#pragma unroll
+        for (int b = 0; b < TB; ++b) ytoff[b] = tr_off(0, wb * TB + b);
+    }
+    const uint32_t yoff = (wb * TB) * 1024 + jl * 64 + swz_y(jl, g) * 16;
+    const uint32_t sbase = lds_addr(smem);
+
+    v4f acc[TC][TB];
+    v4s al[TC], ah[TC], yl[YT ? TB : 1], yh[YT ? TB : 1];
+    v8s yf[YT ? 1 : TB];
+    auto read_frags = [&](int s) {
+        const uint32_t sb = sbase + slot(s);
+#pragma unroll
+        for (int a = 0; a < TC; ++a) {
+            al[a] = tr_read_at<0>(sb + aoff[a]);
+            ah[a] = tr_read_at<512>(sb + aoff[a]);
+        }
+        if constexpr (YT) {
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                yl[b] = tr_read_at<0>(sb + ytoff[b]);
+                yh[b] = tr_read_at<512>(sb + ytoff[b]);
+            }
+        } else {
+            plain_read_frags<TB>(yf, sb + yoff);
+        }
+    };
+    auto join = [](const v4s& lo, const v4s& hi) {
+        const v8s v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        return __builtin_bit_cast(v8bf, v);
+    };
+    auto compute = [&]() {
+        // every read has landed before any fragment is used: the wait, then an
+        // empty asm per fragment that its uses cannot be scheduled above
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(al[0]));
+#pragma unroll
+        for (int a = 0; a < TC; ++a) asm volatile("" : "+v"(al[a]), "+v"(ah[a]));
+        if constexpr (YT) {
+#pragma unroll
+            for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(yl[b]), "+v"(yh[b]));
+        } else {
+#pragma unroll
+            for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(yf[b]));
+        }
+        v8bf af[TC];
+#pragma unroll
+        for (int a = 0; a < TC; ++a) af[a] = join(al[a], ah[a]);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            v8bf bf;
+            if constexpr (YT) bf = join(yl[b], yh[b]);
+            else bf = __builtin_bit_cast(v8bf, yf[b]);
+#pragma unroll
+            for (int a = 0; a < TC; ++a)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bf, acc[a][b], 0, 0, 0);
+        }
+    };
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // lane l of block (a, b): output row b0 + WB wb + 16b + l%16, columns c0 +
+    // WC wc + 16a + 4(l/16) .. +3; 16 rows per pass through the wave's staging
+    // area, 16-byte chunk c of row r at c ^ r, leaving as contiguous 16-byte stores
+    auto epilogue = [&](int b0, int c0) {
+        if constexpr (SL) {
+            float* const part = reinterpret_cast<float*>(out) + int64_t(blockIdx.y) * sl_stride;
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                const int row = b0 + wb * WB + 16 * b + (lane & 15);
+#pragma unroll
+                for (int a = 0; a < TC; ++a) {
+                    const int col = c0 + wc * WC + 16 * a + 4 * (lane >> 4);
+                    if (row < NBR && col < NC)
+                        *reinterpret_cast<v4f*>(part + int64_t(row) * ldo + col) = acc[a][b];
+                }
+            }
+            return;
+        }
+        int8_t* const stg = smem + (STG_OWN ? RING : slot(ST - 1)) + wave * (16 * 256);
+        constexpr int CH = WC / 8, ITEMS = 16 * CH;
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            const int r = lane & 15;
+#pragma unroll
+            for (int a = 0; a < TC; ++a) {
+                const int c = 16 * a + 4 * (lane >> 4);
+                const v4f v = acc[a][b];
+                *reinterpret_cast<uint2*>(stg + r * 256 + (((c >> 3) ^ r) << 4) + (c & 7) * 2) =
+                    make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0)
+#pragma unroll
+            for (int i = 0; i < (ITEMS + 63) / 64; ++i) {
+                const int flat = i * 64 + lane, rr = flat / CH, c = flat % CH;
+                if (ITEMS % 64 == 0 || flat < ITEMS) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(stg + rr * 256 + ((c ^ rr) << 4));
+                    const int row = b0 + wb * WB + 16 * b + rr, col = c0 + wc * WC + 8 * c;
+                    if (row < NBR && col < NC)
+                        *reinterpret_cast<uint4*>(out + int64_t(row) * ldo + col) = v;
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);                   // reads done before reuse
+        }
+    };
+
+    int ti = blockIdx.x, b0, c0;
+    if (!tile_origin(ti, b0, c0)) return;
+    setup(b0, c0);
+    for (int s = 0; s < S - 1; ++s)
+        if (s < ST) issue_at(s, s);
+    wait_batches(min(S - 2, ST - 1));
+    barrier();
+    for (;;) {
+#pragma unroll
+        for (int a = 0; a < TC; ++a)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
+        const int tnext = ti + int(gridDim.x);
+        int b0n = 0, c0n = 0;
+        const bool more = tile_origin(tnext, b0n, c0n);
+        // with a next tile the loads of its steps 0-2 go out in this tile's last
+        // three steps, so the ring never drains
+        const bool cont = more && ST >= S - 1;
+        const int smain = cont ? ST - (S - 1) : ST;
+        if (grp == 0) {
+            read_frags(0);
+            barrier();
+#pragma clang loop unroll(disable)
+            for (int s = 0; s < smain; ++s) {
+                compute();                                      // A(s)
+                if (s + 1 < ST) wait_batches(min(S - 3, ST - 2 - s));
+                barrier();
+                if (s + 1 < ST) read_frags(s + 1);              // B(s)
+                if (s + S - 1 < ST) issue_at(s + S - 1, s + S - 1);
+                barrier();
+            }
+            if (cont) {
+                setup(b0n, c0n);
+#pragma clang loop unroll(disable)
+                for (int s = smain; s < ST; ++s) {
+                    compute();                                  // A(s)
+                    if (s + 1 < ST) wait_batches(S - 3);
+                    barrier();
+                    if (s + 1 < ST) read_frags(s + 1);          // B(s)
+                    issue_at(s + S - 1, s + S - 1 - ST);
+                    barrier();
+                }
+            }
+        } else {
+            barrier();
+#pragma clang loop unroll(disable)
+            for (int s = 0; s < smain; ++s) {
+                read_frags(s);                                  // A(s)
+                if (s + S - 1 < ST) issue_at(s + S - 1, s + S - 1);
+                if (s + 1 < ST) wait_batches(min(S - 2, ST - 2 - s));
+                barrier();
+                compute();                                      // B(s)
+                barrier();
+            }
+            if (cont) {
+                setup(b0n, c0n);
+#pragma clang loop unroll(disable)
+                for (int s = smain; s < ST; ++s) {
+                    read_frags(s);                              // A(s)
+                    issue_at(s + S - 1, s + S - 1 - ST);
+                    if (s + 1 < ST) wait_batches(S - 2);
+                    barrier();
+                    compute();                                  // B(s)
+                    barrier();
+                }
+            }
+        }
+        // every fragment read has completed; with too few steps for the loop to
+        // have issued the next tile's first loads, they go out here
+        if (more && !cont) {
+            setup(b0n, c0n);
+            for (int s = 0; s < S - 1; ++s)
+                if (s < ST) issue_at(ST + s, s);
+        }
+        epilogue(b0, c0);
+        if (!more) break;
+        __builtin_amdgcn_s_waitcnt(0);                          // stores, loads, LDS all done
+        barrier();
+        ring0 = (ring0 + ST) & (S - 1);
+        ti = tnext;
+        b0 = b0n;
+        c0 = c0n;
+    }
 }
 
 // out[m, k] = bf16(sum over s of part[s][m, k]), the slices added in order in
@@ -741,20 +791,143 @@ __global__ __launch_bounds__(256) void sum_slices_bf16_kernel(const float* __res
 
 // Whether a product takes the split-K kernel: a contraction of whole 32-row
 // steps long enough for two teams, and enough bb x 160 tiles to fill the chip
-// where 128 x 128 tiles would leave a ragged second round.  (The byte offsets
-// of the row-contracted operands, up to R rows, stay below 2^32.)
+// in one round.  (The byte offsets of the row-contracted operands, up to R rows,
+// stay below 2^32.)
 static bool bf16_splitk_applies(int nb, int bb, int R, int K, int64_t lda, int64_t ldy, bool yt) {
     if (nb <= 64 || R % kStepRows || R < 2048 || K % 8 || (yt && nb % 8)) return false;
     if (int64_t(R) * lda * 2 >= (int64_t(1) << 32)) return false;
     if (yt && int64_t(R) * ldy * 2 >= (int64_t(1) << 32)) return false;
+    if (!yt && int64_t(bb) * ldy * 2 >= (int64_t(1) << 32)) return false;
     const int64_t tiles = int64_t((nb + bb - 1) / bb) * ((K + 159) / 160);
     return tiles >= 128 && tiles <= 256;
 }
 
-// Contraction slices of the dense dx (dy [M, N] . w [N, K]) split across
-// blocks, when its 128 x 160 tiles are too few for the split-K kernel (below
-// 128): the fewest power-of-two slices giving at least 192 blocks, each slice
-// a whole number of 32-row steps and at least 1024 rows; 0 when none applies.
+// The persistent kernel's tiles of out[b, c], by index; 256 x 320 is taken for
+// the dx only and 256 x 256 for dW only (whose transposing reads of both
+// operands need the registers), 256 x 320 and 192 x 256 for whole contractions
+// only.
+struct Bf16Tile {
+    int bb, bc;
+};
+constexpr Bf16Tile kBf16Tiles[] = {{256, 320}, {256, 256}, {192, 256},
+                                   {128, 256}, {128, 192}, {128, 128}};
+constexpr int kBf16FirstSliced = 3, kBf16MaxSlices = 8;
+
+struct Bf16Plan {
+    int tile, slices, slice;    // slice: rows of the contraction per slice
+};
+
+// The tile and the contraction slices with the least predicted time.  rounds of
+// tiles, each the slice's 32-row steps (0.066 us per 10^4 outputs for the dx,
+// 0.073 for dW, whose operands both come through transposing reads, plus 0.24 /
+// 0.27 us of barriers, waits and load issue) and an epilogue; slices add their
+// fp32 stores and a pass that reads them back.  Fitted to eight tiles and up to
+// eight slices on 110 products (M 128-4096, N 512-10240, K 512-5120; scatter 6%
+// for the dx, 4% for dW); choosing by it is 0.6% and 0.5% off the fastest of them on
+// average.  Against the 128 x 128 kernels and the power-of-two slices
+// it replaces, us:
+//   dx 4096 x 1280 x 5120 (M, N, K)  83.7 -> 53.0 (256 x 320, one round)
+//   dx 3682 x 3248 x 4864            176.4 -> 104.2
+//   dx 322 x 5648 x 2048             87.9 -> 26.4 (128 x 128, four slices)
+//   dx 205 x 2672 x 768              51.1 -> 14.9 (2672 % 32 kept it unsplit)
+//   dW 2893 x 544 x 768 (M, N, K)    46.0 -> 17.2 (eight slices)
+//   dW 1970 x 672 x 512              32.1 -> 16.3
+// and over all 110 1.69 times as fast (dx) and 1.23 (dW).
+// work: the bytes of fp32 partial sums that may be used.
+static Bf16Plan bf16_plan(int64_t nbr, int64_t nc, int R, bool yt, int64_t work) {
+    const double c0 = yt ? 3.98 : 4.57, mm = yt ? 0.0732 : 0.0658, st = yt ? 0.273 : 0.238,
+                 fs = yt ? 0.97 : 0.947, ep = yt ? 0.92 : 1.26, fe = yt ? 0.18 : 0.0,
+                 s0 = yt ? 4.5 : 2.5, sp = yt ? 0.8e-6 : 0.85e-6, se = yt ? 0.51 : 0.91;
+    const int64_t cus = device_cus();
+    Bf16Plan best{5, 1, R};
+    double time = 0;
+    for (int i = 0; i < int(sizeof(kBf16Tiles) / sizeof(kBf16Tiles[0])); ++i) {
+        if (i == (yt ? 0 : 1)) continue;
+        const int64_t bb = kBf16Tiles[i].bb, bc = kBf16Tiles[i].bc;
+        const int64_t tiles = ((nbr + bb - 1) / bb) * ((nc + bc - 1) / bc);
+        const double area = 1e-4 * double(bb * bc);
+        for (int n = 1; n <= (i < kBf16FirstSliced ? 1 : kBf16MaxSlices); ++n) {
+            const int len = n == 1 ? R : int((int64_t(R) + n - 1) / n + 31) / 32 * 32;
+            if (n > 1 && (len < 128 || (R - 1) / len + 1 != n || n * nbr * nc * 4 > work)) continue;
+            const int64_t rounds = ((tiles + 7) / 8 * n + cus / 8 - 1) / (cus / 8);
+            const double fill = double(tiles * n) / double(cus * rounds);
+            double t = c0 + double(rounds) * (((len - 1) / 32 + 1) * (mm * area + st) *
+                                                  (fs + (1 - fs) * fill) +
+                                              ep * area * (fe + (1 - fe) * fill));
+            if (n > 1) t += s0 + sp * double(nbr) * double(nc) * n + double(rounds) * se * area;
+            if (time == 0 || t < time) best = Bf16Plan{i, n, len}, time = t;
+        }
+    }
+    return best;
+}
+
+int64_t bf16_dx_work_bytes(int M, int N, int K) {
+    if (bf16_splitk_applies(M, 128, N, K, K, N, false)) return 0;
+    const int n = bf16_plan(M, K, N, false, int64_t(1) << 62).slices;
+    return n > 1 ? int64_t(n) * M * K * 4 : 0;
+}
+int64_t bf16_dw_work_bytes(int R, int N, int K) {
+    if (bf16_splitk_applies(N, 160, R, K, K, N, true)) return 0;
+    const int n = bf16_plan(N, K, R, true, int64_t(1) << 62).slices;
+    return n > 1 ? int64_t(n) * N * K * 4 : 0;
+}
+
+// out[b, c] = sum over r of a[r, c] * y (y[b, r], or y[r, b] with YT) on the
+// persistent kernel by the plan
+template <bool YT>
+static hipError_t launch_bf16_pp(hipStream_t st, const uint16_t* a, int64_t lda, const uint16_t* y,
+                                 int64_t ldy, uint16_t* out, int64_t ldo, int R, int nc, int nbr,
+                                 float* part, int64_t part_bytes) {
+    const bool wide = std::max(lda, ldy) >= (int64_t(1) << 27);
+    const Bf16Plan p =
+        wide ? Bf16Plan{5, 1, R} : bf16_plan(nbr, nc, R, YT, part ? part_bytes : 0);
+    const int bb = kBf16Tiles[p.tile].bb, bc = kBf16Tiles[p.tile].bc;
+    const int tb = (nbr + bb - 1) / bb, tc = (nc + bc - 1) / bc;
+    const int64_t tiles = int64_t(tb) * tc;
+    const dim3 grid(unsigned(std::min<int64_t>((tiles + 7) / 8 * 8, device_cus() / 8 * 8)),
+                    unsigned(p.slices));
+    const int64_t stride = int64_t(nbr) * nc;
+#define XPU_BF16_PP(BB, BC, WGM, SL, ...)                                                         \
+    hipLaunchKernelGGL((gemm_bf16_pp_kernel<BB, BC, WGM, YT, SL, ##__VA_ARGS__>), grid,          \
+                       dim3(512), 0, st, a, lda, y, ldy,                                           \
+                       SL ? reinterpret_cast<uint16_t*>(part) : out, SL ? int64_t(nc) : ldo, R,   \
+                       nc, nbr, tb, tc, p.slice, stride)
+    if (wide) {
+        XPU_BF16_PP(128, 128, 2, false, uint64_t);
+    } else if (p.slices > 1) {
+        switch (p.tile) {
+            case 3: XPU_BF16_PP(128, 256, 2, true); break;
+            case 4: XPU_BF16_PP(128, 192, 2, true); break;
+            default: XPU_BF16_PP(128, 128, 2, true); break;
+        }
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        int64_t blocks = (int64_t(nbr) * (nc / 4) + 255) / 256;
+        if (blocks > (int64_t(1) << 20)) blocks = int64_t(1) << 20;
+        hipLaunchKernelGGL(sum_slices_bf16_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, part,
+                           p.slices, stride, out, ldo, int64_t(nbr), int64_t(nc));
+    } else {
+        switch (p.tile) {
+            case 0:
+                if constexpr (!YT) XPU_BF16_PP(256, 320, 2, false);
+                break;
+            case 1:
+                if constexpr (YT) XPU_BF16_PP(256, 256, 2, false);
+                break;
+            case 2: XPU_BF16_PP(192, 256, 2, false); break;
+            case 3: XPU_BF16_PP(128, 256, 2, false); break;
+            case 4: XPU_BF16_PP(128, 192, 2, false); break;
+            default: XPU_BF16_PP(128, 128, 2, false); break;
+        }
+    }
+#undef XPU_BF16_PP
+    return hipGetLastError();
+}
+
+// The workspace that xpuint8_linear_dx_workspace_size names: fp32 partial sums
+// of the fewest power-of-two slices giving 192 blocks of 128 x 160 tiles where
+// those number below 128 (each slice a whole number of 32-row steps and at least
+// 1024 rows); 0 slices when none applies.  The product splits its contraction as
+// bf16_plan finds best within the workspace it is given.
 int bf16_nn_slices(int M, int N, int K) {
     if (M <= 64 || K % 8 || N % kStepRows) return 0;
     const int64_t tiles = int64_t((M + 127) / 128) * ((K + 159) / 160);
@@ -762,67 +935,41 @@ int bf16_nn_slices(int M, int N, int K) {
     int s = 1;
     while (tiles * s < 192 && (N / kStepRows) % (2 * s) == 0 && N / (2 * s) >= 1024) s *= 2;
     if (s == 1) return 0;
-    // the split-K kernel's 32-bit byte offsets: a slice's rows of w (N / s
-    // rows of K) and a 128-row block of dy (rows of N); beyond them the
-    // unsplit kernel takes the shape
     if (int64_t(N / s) * K * 2 >= (int64_t(1) << 32) || 128 * int64_t(N) * 2 >= (int64_t(1) << 31))
         return 0;
     return s;
 }
 
-hipError_t gemm_bf16_nn_slices(hipStream_t st, const void* dy, int64_t ldy, const void* w,
-                               int64_t ldw, void* out, int64_t ldo, int M, int N, int K,
-                               float* part, int nsl) {
-    const int tm = (M + 127) / 128, tk = (K + 159) / 160;
-    hipLaunchKernelGGL((gemm_bf16_splitk_kernel<4, false, true>),
-                       dim3(unsigned(tm * tk), unsigned(nsl)), dim3(512), 0, st,
-                       static_cast<const uint16_t*>(w), ldw, static_cast<const uint16_t*>(dy), ldy,
-                       reinterpret_cast<uint16_t*>(part), int64_t(K), N / nsl, K, M, tm, tk,
-                       int64_t(M) * K);
-    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    int64_t blocks = (int64_t(M) * (K / 4) + 255) / 256;
-    if (blocks > (int64_t(1) << 20)) blocks = int64_t(1) << 20;
-    hipLaunchKernelGGL(sum_slices_bf16_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, part, nsl,
-                       int64_t(M) * K, static_cast<uint16_t*>(out), ldo, int64_t(M), int64_t(K));
-    return hipGetLastError();
-}
-
 hipError_t gemm_bf16_nn(hipStream_t st, const void* dy, int64_t ldy, const void* w, int64_t ldw,
-                        void* out, int64_t ldo, int M, int N, int K) {
+                        void* out, int64_t ldo, int M, int N, int K, float* part,
+                        int64_t part_bytes) {
+    const uint16_t* a = static_cast<const uint16_t*>(w);
+    const uint16_t* y = static_cast<const uint16_t*>(dy);
     if (bf16_splitk_applies(M, 128, N, K, ldw, ldy, false)) {
         const int tm = (M + 127) / 128, tk = (K + 159) / 160;
         hipLaunchKernelGGL((gemm_bf16_splitk_kernel<4, false>), dim3(unsigned(tm * tk)), dim3(512),
-                           0, st, static_cast<const uint16_t*>(w), ldw,
-                           static_cast<const uint16_t*>(dy), ldy, static_cast<uint16_t*>(out), ldo,
-                           N, K, M, tm, tk);
+                           0, st, a, ldw, y, ldy, static_cast<uint16_t*>(out), ldo, N, K, M, tm, tk);
         return hipGetLastError();
     }
-    const int tiles_k = (K + 127) / 128, tiles_m = (M + 127) / 128;
-    hipLaunchKernelGGL((gemm_bf16_nn_kernel<2>), dim3(unsigned(tiles_k * tiles_m)), dim3(256), 0,
-                       st, static_cast<const uint16_t*>(w), ldw, static_cast<const uint16_t*>(dy),
-                       ldy, static_cast<uint16_t*>(out), ldo, N, K, M, tiles_k, tiles_m);
-    return hipGetLastError();
+    return launch_bf16_pp<false>(st, a, ldw, y, ldy, static_cast<uint16_t*>(out), ldo, N, K, M,
+                                 part, part_bytes);
 }
 
 hipError_t gemm_bf16_tn(hipStream_t st, const void* dy, int64_t ldy, const void* x, int64_t ldx,
-                        void* dw, int64_t ldo, int R, int N, int K) {
+                        void* dw, int64_t ldo, int R, int N, int K, float* part,
+                        int64_t part_bytes) {
     constexpr int STAGES_TN = 4;                // 2 x 4 x 20 KB of LDS
+    const uint16_t* a = static_cast<const uint16_t*>(x);
+    const uint16_t* y = static_cast<const uint16_t*>(dy);
     if (bf16_splitk_applies(N, 160, R, K, ldx, ldy, true)) {
         const int tn = (N + 159) / 160, tk = (K + 159) / 160;
         hipLaunchKernelGGL((gemm_bf16_splitk_kernel<STAGES_TN, true>), dim3(unsigned(tn * tk)),
-                           dim3(512), 0, st, static_cast<const uint16_t*>(x), ldx,
-                           static_cast<const uint16_t*>(dy), ldy, static_cast<uint16_t*>(dw), ldo,
-                           R, K, N, tn, tk);
+                           dim3(512), 0, st, a, ldx, y, ldy, static_cast<uint16_t*>(dw), ldo, R, K,
+                           N, tn, tk);
         return hipGetLastError();
     }
-    const int tiles_k = (K + 127) / 128, tiles_n = (N + 127) / 128;
-    // two stages (one in flight): measured fastest at the C5 shape (75 us vs
-    // 83-86 us for three to five), the smaller LDS footprint leaving room for
-    // more resident blocks per CU
-    hipLaunchKernelGGL((gemm_bf16_tn_kernel<2>), dim3(unsigned(tiles_k * tiles_n)), dim3(256), 0,
-                       st, static_cast<const uint16_t*>(x), ldx, static_cast<const uint16_t*>(dy),
-                       ldy, static_cast<uint16_t*>(dw), ldo, R, K, N, tiles_k, tiles_n);
-    return hipGetLastError();
+    return launch_bf16_pp<true>(st, a, ldx, y, ldy, static_cast<uint16_t*>(dw), ldo, R, K, N, part,
+                                part_bytes);
 }
 
 }  // namespace xpuint8

@@ -288,9 +288,9 @@ def linear_dx(dy, w):
         m = dy2.shape[0]
         dx = torch.empty((m, k), device=dy.device, dtype=torch.bfloat16)
         if m:
-            # a small batch splits the contraction across blocks (fp32
-            # partials in the workspace)
-            need = int(lib.xpuint8_linear_dx_workspace_size(m, n, k))
+            # an output with few tiles splits the contraction across blocks
+            # (fp32 partials in the workspace)
+            need = int(lib.xpuint8_linear_dx_split_workspace_size(m, n, k))
             work = torch.empty(need, device=dy.device, dtype=torch.uint8) if need > 0 else None
             rc = lib.xpuint8_linear_dx_stream(_stream(dy.device), _ptr(dy2), _ptr(w2), _ptr(dx),
                                               m, n, k, _opt(work), max(need, 0))
@@ -320,8 +320,11 @@ def linear_dw(dy, x):
         lib = _lib()
         dy2, x2 = _c(dy2), _c(x2)
         dw = torch.empty((n, k), device=dy2.device, dtype=torch.bfloat16)
-        rc = lib.xpuint8_linear_dw_stream(_stream(dy2.device), _ptr(dy2), _ptr(x2), _ptr(dw),
-                                          dy2.shape[0], n, k)
+        m = dy2.shape[0]
+        need = int(lib.xpuint8_linear_dw_workspace_size(m, n, k))
+        work = torch.empty(need, device=dy2.device, dtype=torch.uint8) if need > 0 else None
+        rc = lib.xpuint8_linear_dw_work_stream(_stream(dy2.device), _ptr(dy2), _ptr(x2), _ptr(dw),
+                                               m, n, k, _opt(work), max(need, 0))
         if rc != 0:
             _err(lib, "linear_dw")
         return dw
