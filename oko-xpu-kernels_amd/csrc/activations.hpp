@@ -72,10 +72,8 @@ __device__ __forceinline__ float activate_pre(const uint16_t* tab, float a, floa
     if constexpr (ACT == 2) {
         return tab_lookup(tab, kTabSilu, a) * b;
     } else if constexpr (ACT == 3) {
-        const float tg = tab_lookup(tab, kTabSituTanhG, b);
-        const float sg = tab_lookup(tab, kTabSigmoid, b);
-        const float th = tab_lookup(tab, kTabSituTanhH, a);
-        return bf16_round(tg * sg) * th;
+        // the gate factor bf16(tanh(b/4) * sigmoid(b)) as one table
+        return tab_lookup(tab, kTabSituGate, b) * tab_lookup(tab, kTabSituTanhH, a);
     } else if constexpr (ACT == 4) {
         return a * tab_lookup(tab, kTabGeluErf, b);
     } else {
@@ -105,12 +103,21 @@ __device__ __forceinline__ float act_combine(float a, float b, const uint32_t* t
 // whose exponent field is in [115, 131) (|x| in [2^-12, 2^4)), where the
 // FFN's activations lie: 2048 positive inputs, then the 2048 negative ones.
 // Input bits b sit at position 2048 * (b >> 15) + (b & 0x7FFF) - (115 << 7);
-// inputs outside read the table in global memory.  Used for the GELU (erf)
-// of the FFN's up-projection epilogue (ids 4 and 5, one lookup per value).
+// inputs outside read the table in global memory.  Used by the FFN's
+// up-projection epilogue: the GELU (erf) of ids 4 and 5 and situ's gate factor.
 constexpr int kWinLo = 115 << 7, kWinHalf = 16 * 128, kWinSize = 2 * kWinHalf;
 template <int ACT>
 __host__ __device__ constexpr int act_window_table() {
-    return (ACT == 4 || ACT == 5) ? kTabGeluErf : -1;
+    return (ACT == 4 || ACT == 5) ? kTabGeluErf : ACT == 3 ? kTabSituGate : -1;
+}
+// Situ's second window, tanh(h/25) of the hidden value: an odd function (the
+// sign is put back on the magnitude's result), so the positive inputs in
+// [2^-10, 2^4) serve both signs, at word (b & 0x7FFF) - (117 << 7).  3.5 KB: with
+// the first window, what the 256 x 320 tile's ring leaves of the LDS.
+constexpr int kWin2Lo = 117 << 7, kWin2Size = 14 * 128;
+template <int ACT>
+__host__ __device__ constexpr int act_window_words() {
+    return act_window_table<ACT>() < 0 ? 0 : kWinSize + (ACT == 3 ? kWin2Size : 0);
 }
 // bf16 input bits of window position w
 __device__ __forceinline__ uint32_t win_bits(int w) {

@@ -318,19 +318,15 @@ int ffn_run(hipStream_t st, const void* x, const int8_t* up_w8, const int8_t* up
     char* region = v + ffn_work_region_offset(M, inner);
     int8_t* xq = reinterpret_cast<int8_t*>(region);
     float* xs = reinterpret_cast<float*>(region + linear_work_q_bytes(M, K));
-    // the persistent up-projection reads xq in the MFMA block layout
-    if (pp_applies(int(M), int(inner), int(K), act_paired(activation)) &&
-        rowquant_can_tile(int(K))) {
+    // xq in the MFMA block layout: with the packed weight, and for the persistent
+    // up-projection from a row-major one
+    if (rowquant_can_tile(int(K)) &&
+        (up_wp || pp_applies(int(M), int(inner), int(K), act_paired(activation)))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, xq, xs, M, int(K)), "ffn (quantize)"));
-        XPU_TRY(launched(gemm_act_pp_xt(st, xq, up_wp ? up_wp : up_w8, K, v, inner, xs, up_scale,
-                                        int(M), int(inner), int(K), activation, up_wp != nullptr),
-                         "ffn (up projection)"));
-    } else if (up_wp && skinny_applies(int(M), act_paired(activation)) &&
-               rowquant_can_tile(int(K))) {
-        // so does the skinny one, given the packed weight
-        XPU_TRY(launched(convrot_quantize_tiled(st, x, xq, xs, M, int(K)), "ffn (quantize)"));
-        XPU_TRY(launched(gemm_act_skinny_xt(st, xq, up_wp, v, inner, xs, up_scale, int(M),
-                                            int(inner), int(K), activation),
+        XPU_TRY(launched(up_wp ? gemm_act_packed(st, xq, up_wp, v, inner, xs, up_scale, int(M),
+                                                 int(inner), int(K), activation)
+                               : gemm_act_pp_xt(st, xq, up_w8, K, v, inner, xs, up_scale, int(M),
+                                                int(inner), int(K), activation),
                          "ffn (up projection)"));
     } else {
         XPU_TRY(launched(convrot_quantize(st, x, xq, xs, M, int(K), 0), "ffn (quantize)"));

@@ -201,8 +201,14 @@ struct EpiAct {
     const float* ws;          // per weight row: [2 * half] paired, [N] otherwise
     int half;                 // row offset of the second half (paired)
     const uint16_t* tab;      // device activation tables
-    uint32_t win = 0;         // LDS address of the table window (0: none)
+    uint32_t win = 0;         // LDS address of the table window(s) (0: none)
     static constexpr int kWinTab = act_window_table<ACT>();
+    static constexpr int kWinWords = act_window_words<ACT>();
+    // table word (16-bit) of word w of the window(s)
+    __device__ __forceinline__ uint16_t win_fill(int w) const {
+        if (w >= kWinSize) return tab[kTabSituTanhH * kTabSize + kWin2Lo + w - kWinSize];
+        return tab[kWinTab * kTabSize + win_bits(w)];
+    }
     struct Col { float4 w; };
     __device__ __forceinline__ float row(int m) const { return xs[m]; }
     __device__ __forceinline__ Col col(int n) const {
@@ -275,16 +281,55 @@ struct EpiAct {
             asm volatile("ds_read_u16 %0, %1" : "=v"(t[2 * j]) : "v"(a0));
             asm volatile("ds_read_u16 %0, %1" : "=v"(t[2 * j + 1]) : "v"(a1));
         }
+        tor &= 0x78007800u;
+        // situ's second lookup, tanh(h/25) of the hidden values: the window of
+        // positive inputs, its word min(|h| - lo, last) clamped with saturating
+        // packed arithmetic, the sign put back afterwards
+        uint32_t hp[2], u[4];
+        if constexpr (ACT == 3) {
+            hp[0] = cvt_pk_bf16(val[0], val[1]);
+            hp[1] = cvt_pk_bf16(val[2], val[3]);
+            const u16x2 last{uint16_t(kWin2Size - 1), uint16_t(kWin2Size - 1)};
+            const uint32_t win2 = win + 2 * kWinSize;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const u16x2 tt = __builtin_bit_cast(u16x2, hp[j] & 0x7FFF7FFFu) -
+                                 u16x2{uint16_t(kWin2Lo), uint16_t(kWin2Lo)};
+                tor |= __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(tt, last));
+                const uint32_t off = __builtin_bit_cast(
+                    uint32_t, u16x2(__builtin_elementwise_min(tt, last) << u16x2{1, 1}));
+                asm volatile("ds_read_u16 %0, %1" : "=v"(u[2 * j]) : "v"(win2 + (off & 0xFFFFu)));
+                asm volatile("ds_read_u16 %0, %1" : "=v"(u[2 * j + 1]) : "v"(win2 + (off >> 16)));
+            }
+        }
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]));
-        if (__builtin_amdgcn_ballot_w64((tor & 0x78007800u) != 0)) {
+        if constexpr (ACT == 3)
+            asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+        if (__builtin_amdgcn_ballot_w64(tor != 0)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t k = (kp[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
                 if (((k - uint32_t(kWinLo)) & 0x7800u) != 0)
                     t[i] = tab[kWinTab * kTabSize + k];
+                if constexpr (ACT == 3) {
+                    const uint32_t h = (hp[i >> 1] >> (16 * (i & 1))) & 0x7FFFu;
+                    if (h - uint32_t(kWin2Lo) >= uint32_t(kWin2Size))
+                        u[i] = tab[kTabSituTanhH * kTabSize + h];
+                }
             }
         }
-        if constexpr (ACT == 4) {
+        if constexpr (ACT == 3) {
+            // tanh(|h|/25) with h's sign, times the gate factor (exact in fp32),
+            // then the packing's rounding
+            float r[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t sign = (i & 1) ? hp[i >> 1] & 0x80000000u
+                                              : (hp[i >> 1] << 16) & 0x80000000u;
+                r[i] = tab_float(t[i]) * __uint_as_float((u[i] << 16) | sign);
+            }
+            return make_uint2(cvt_pk_bf16(r[0], r[1]), cvt_pk_bf16(r[2], r[3]));
+        } else if constexpr (ACT == 4) {
             // the hidden values, rounded to bf16 in pairs, times the table's
             // gelu(gate): each product exact in fp32, then the packing's
             // rounding
@@ -313,7 +358,7 @@ struct EpiAct {
     }
     __device__ __forceinline__ uint2 convert2_w(const v4i& av, const v4i& bv, float x, const Col& ca,
                                                 const Col& cb) const {
-        static_assert(ACT == 4, "the windowed pair form is GEGLU's");
+        static_assert(ACT == 3 || ACT == 4, "the windowed pair form is situ's and GEGLU's");
         const float a[4] = {deq_raw(av[0], ca.w.x, x), deq_raw(av[1], ca.w.y, x),
                             deq_raw(av[2], ca.w.z, x), deq_raw(av[3], ca.w.w, x)};
         const float b[4] = {deq_raw(bv[0], cb.w.x, x), deq_raw(bv[1], cb.w.y, x),
@@ -923,8 +968,9 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     constexpr int SCALE_BYTES = NSCALE * 4;
     constexpr int SPT = (NSCALE + 511) / 512;                   // operand values per thread
     // the activation table's LDS window, for an epilogue that has one
-    constexpr int WIN_BYTES = has_window<Epi>() ? 2 * kWinSize : 0;
-    constexpr int LDS_BYTES = RING + STG_OWN + 2 * SCALE_BYTES + WIN_BYTES + 16;
+    constexpr int WIN_WORDS = [] { if constexpr (has_window<Epi>()) return Epi::kWinWords; else return 0; }();
+    constexpr int WIN_BYTES = 2 * WIN_WORDS;
+    constexpr int LDS_BYTES = RING + STG_OWN + 2 * SCALE_BYTES + WIN_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) int8_t smem[LDS_BYTES];
     constexpr int SCALES = RING + STG_OWN;                      // LDS offset of the operands
@@ -1147,8 +1193,7 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     if constexpr (WIN_BYTES > 0) {
         // the window, read once per block (visible after the first barrier)
         uint16_t* w = reinterpret_cast<uint16_t*>(smem + SCALES + 2 * SCALE_BYTES);
-        const uint16_t* t = epi.tab + size_t(Epi::kWinTab) * kTabSize;
-        for (int i = threadIdx.x; i < kWinSize; i += 512) w[i] = t[win_bits(i)];
+        for (int i = threadIdx.x; i < WIN_WORDS; i += 512) w[i] = epi.win_fill(i);
         epi_w.win = lds_addr(w);
     }
     setup(m0, n0);
@@ -1992,27 +2037,40 @@ __global__ __launch_bounds__(NW * 64) void gemm_i8_wavek_kernel(
     }
 }
 
-// The kernel's tiles: 16 MB x 16 NB outputs, NW waves, and the blocks of one
+// The kernel's tiles: 16 MB x 16 NB weight rows, NW waves, and the blocks of one
 // that a CU holds at once (LDS, registers)
 struct WavekTile {
     int mb, nb, nw, d, per_cu;
 };
-constexpr WavekTile kWavekTiles[] = {
-    {1, 1, 8, 4, 2}, {1, 2, 4, 4, 6}, {2, 2, 4, 4, 4}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
 
-// Predicted time in us: the fullest CU's operand loads (0.68 us per 100 KB),
-// the chain of each round's K steps (D at a time; 0.2 us each), its reductions
-// (0.28 us per 16 KB of partial sums), and the product's bytes (12 TB/s: caches).  Fitted to 16
-// tiles on 390 products of up to 260 GOP, scatter 10%; the tile it picks of
-// these five is 2% off the fastest of the sixteen on average.
-inline double wavek_time(const WavekTile& t, int64_t M, int64_t N, int K) {
+// Predicted time in us: the fullest CU's operand loads (`load` us per KB), the
+// chain of each round's K steps (D at a time; `step` us each), its reductions
+// and epilogues (`red` us per KB of partial sums), and the product's bytes (12
+// TB/s: caches).  N: weight rows; out_cols: output columns.
+struct WavekModel {
+    double c0, load, step, red, byte;
+};
+inline double wavek_time(const WavekModel& w, const WavekTile& t, int64_t M, int64_t N, int K,
+                         int64_t out_cols) {
     const int64_t blocks = ((M + 16 * t.mb - 1) / (16 * t.mb)) * ((N + 16 * t.nb - 1) / (16 * t.nb));
     const int64_t cus = device_cus(), per = (blocks + cus - 1) / cus;
     const int64_t rounds = (blocks + cus * t.per_cu - 1) / (cus * t.per_cu);
     const int KB = (K + 63) / 64, chain = (KB + t.nw * t.d - 1) / (t.nw * t.d);
-    const double bytes = double(M) * K + double(N) * K + 2.0 * double(M) * double(N);
-    return 2.25 + 0.0068 * double(per) * (t.mb + t.nb) * KB + 0.2 * double(rounds) * chain +
-           0.277 / 16 * double(per) * (t.mb * t.nb * t.nw) + 0.082e-6 * bytes;
+    const double bytes = double(M) * K + double(N) * K + 2.0 * double(M) * double(out_cols);
+    return w.c0 + w.load * double(per) * (t.mb + t.nb) * KB + w.step * double(rounds) * chain +
+           w.red * double(per) * (t.mb * t.nb * t.nw) + w.byte * bytes;
+}
+
+// The tile with the least predicted time below `time` (updated), -1 for none
+template <int NT>
+inline int wavek_tile(const WavekModel& w, const WavekTile (&tiles)[NT], double bias, int64_t M,
+                      int64_t N, int K, int64_t out_cols, double* time) {
+    int best = -1;
+    for (int i = 0; i < NT; ++i) {
+        const double t = bias * wavek_time(w, tiles[i], M, N, K, out_cols);
+        if (t < *time) best = i, *time = t;
+    }
+    return best;
 }
 
 template <int MB, int NB, int NW, int D, class Epi>
@@ -2080,15 +2138,43 @@ hipError_t launch_pp(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t*
 
 // The ping-pong kernel's tile for a product of two block-layout operands: the
 // one with the least predicted time.  A block runs ceil(share / CUs per XCD)
-// rounds of tiles; a K step of a BM x BN tile takes 0.0546 us per 10^4
-// outputs (the matrix cores and the LDS reads that feed them) plus 0.21 us
-// (barriers, waits, load issue), a tile's epilogue 0.99 us per 10^4 outputs,
-// both less when the last round leaves CUs (and so memory bandwidth) free.
-// Fitted to 15 tile shapes on 170 products of 3-260 GOP, M 65-4096, N 256-10240,
-// K 256-8192 (the times' scatter about it is 3.5%); choosing among these five by
-// it is 0.3% off the fastest of the fifteen on average (11% at worst).  Against
-// the kernels that took those products before (256 x 160 and 128 x 128 tiles of
-// row-major operands, split K), cold weights and activations rotating:
+// rounds of tiles; a K step of a BM x BN tile takes `mm` us per 10^4 outputs
+// (the matrix cores and the LDS reads that feed them) plus `st` us (barriers,
+// waits, load issue), a tile's epilogue `ep` us per 10^4 outputs, both less when
+// the last round leaves CUs (and so memory bandwidth) free (`fs`, `fe`).
+struct PpTile {
+    int bm, bn;
+};
+struct PpModel {
+    double c0, mm, st, fs, ep, fe;
+};
+// n_tiles: tiles across the output columns
+inline double pp_time(const PpModel& p, int bm, int bn, int64_t M, int64_t n_tiles, int K) {
+    const int64_t tiles = ((M + bm - 1) / bm) * n_tiles, cus = device_cus();
+    const int64_t rounds = ((tiles + 7) / 8 + cus / 8 - 1) / (cus / 8);
+    const double area = 1e-4 * bm * bn, fill = double(tiles) / double(cus * rounds);
+    const double steps = (K + 63) / 64;
+    return p.c0 + double(rounds) * (steps * (p.mm * area + p.st) * (p.fs + (1 - p.fs) * fill) +
+                                    p.ep * area * (p.fe + (1 - p.fe) * fill));
+}
+template <int NT>
+inline int pp_tile(const PpModel& p, const PpTile (&tiles)[NT], bool paired, int64_t M, int64_t N,
+                   int K, double* time) {
+    int best = 0;
+    for (int i = 0; i < NT; ++i) {
+        const int cols = paired ? tiles[i].bn / 2 : tiles[i].bn;
+        const double c = pp_time(p, tiles[i].bm, tiles[i].bn, M, (N + cols - 1) / cols, K);
+        if (i == 0 || c < *time) best = i, *time = c;
+    }
+    return best;
+}
+
+// Unpaired epilogues.  The persistent kernel's model is fitted to 15 tile shapes
+// on 170 products of 3-260 GOP, M 65-4096, N 256-10240, K 256-8192 (the times'
+// scatter about it is 3.5%); choosing among these five by it is 0.3% off the
+// fastest of the fifteen on average (11% at worst).  Against the kernels that took
+// those products before (256 x 160 and 128 x 128 tiles of row-major operands,
+// split K), cold weights and activations rotating:
 //   3974 x 3072 x 3072 (M, N, K)  51.2 -> 34.7 us (192 x 256: 252 tiles)
 //   3952 x 3072 x 8192            135.5 -> 82.0 us
 //   1388 x 9376 x 2816            53.7 -> 37.1 us
@@ -2100,21 +2186,17 @@ hipError_t launch_pp(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t*
 // round; fitted to the same products, scatter 3.7%): at 4096 x 1280 x 5120, in a
 // training step, 30.4 us against 32.5; at 4096 x 1280 x 1280 14.2 against 12.2.
 // It is taken where it is predicted 3% faster.
-struct PpTile {
-    int bm, bn;
-};
+// The model of the kernel that splits K over waves is fitted to 16 tiles on 390
+// products of up to 260 GOP, scatter 10%; the tile it picks of these five is 2%
+// off the fastest of the sixteen on average.  It is taken where it is predicted
+// 6% faster.
 constexpr PpTile kPpTiles[] = {{256, 320}, {192, 320}, {192, 256}, {192, 192}, {128, 192}};
+constexpr PpModel kPpModel = {3.8, 0.0546, 0.206, 0.84, 0.994, 0.615};
+constexpr WavekTile kWavekTiles[] = {
+    {1, 1, 8, 4, 2}, {1, 2, 4, 4, 6}, {2, 2, 4, 4, 4}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
+constexpr WavekModel kWavekModel = {2.25, 0.0068, 0.2, 0.277 / 16, 0.082e-6};
 
-inline double pp_time(int bm, int bn, int64_t M, int64_t N, int K) {
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn), cus = device_cus();
-    const int64_t rounds = ((tiles + 7) / 8 + cus / 8 - 1) / (cus / 8);
-    const double area = 1e-4 * bm * bn, fill = double(tiles) / double(cus * rounds);
-    const double steps = (K + 63) / 64;
-    return 3.8 + double(rounds) * (steps * (0.0546 * area + 0.206) * (0.84 + 0.16 * fill) +
-                                   0.994 * area * (0.615 + 0.385 * fill));
-}
-
-inline double splitk_time(int64_t M, int64_t N, int K) {
+inline double splitk_time(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 159) / 160), cus = device_cus();
     const int64_t rounds = (tiles + cus - 1) / cus;
     const double fill = double(tiles) / double(cus * rounds), steps = (K + 63) / 64;
@@ -2122,36 +2204,25 @@ inline double splitk_time(int64_t M, int64_t N, int K) {
                                    5.62 * (0.8 + 0.2 * fill));
 }
 
-inline int pp_tile(int64_t M, int64_t N, int K, double* time) {
-    int best = 0;
-    double t = 0;
-    for (int i = 0; i < int(sizeof(kPpTiles) / sizeof(kPpTiles[0])); ++i) {
-        const double c = pp_time(kPpTiles[i].bm, kPpTiles[i].bn, M, N, K);
-        if (i == 0 || c < t) best = i, t = c;
-    }
-    *time = t;
-    return best;
-}
+// Whether an epilogue is an activation's (no split-K form)
+template <class Epi, class = void>
+struct IsActEpi : std::false_type {};
+template <class Epi>
+struct IsActEpi<Epi, std::void_t<decltype(Epi::kWinTab)>> : std::true_type {};
 
 // X and W both in the block layout, unpaired epilogues
 template <class Epi>
 hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N, int K,
-                          const Epi& epi) {
+                        const Epi& epi) {
+    constexpr bool kSplitK = Epi::kStaged && !IsActEpi<Epi>::value;
     double t = 0;
-    const int tile = pp_tile(M, N, K, &t);
+    const int tile = pp_tile(kPpModel, kPpTiles, false, M, N, K, &t);
     bool splitk = false;
-    if constexpr (Epi::kStaged) {
+    if constexpr (kSplitK) {
         const double ts = 1.03 * splitk_time(M, N, K);
         if (ts < t) splitk = true, t = ts;
     }
-    // the K-split-over-waves kernel where it is predicted 6% faster (its
-    // prediction scatters more)
-    int wk = -1;
-    for (int i = 0; i < int(sizeof(kWavekTiles) / sizeof(kWavekTiles[0])); ++i) {
-        const double tw = 1.06 * wavek_time(kWavekTiles[i], M, N, K);
-        if (tw < t) wk = i, t = tw;
-    }
-    switch (wk) {
+    switch (wavek_tile(kWavekModel, kWavekTiles, 1.06, M, N, K, N, &t)) {
         case 0: return launch_wavek<1, 1, 8, 4>(st, Xt, Wp, M, N, K, epi);
         case 1: return launch_wavek<1, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
         case 2: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
@@ -2159,7 +2230,7 @@ hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int 
         case 4: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
         default: break;
     }
-    if constexpr (Epi::kStaged) {
+    if constexpr (kSplitK) {
         if (splitk) return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
     }
     switch (tile) {
@@ -2167,6 +2238,46 @@ hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int 
         case 1: return launch_pp<true, true, 192, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 2: return launch_pp<true, true, 192, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 3: return launch_pp<true, true, 192, 192, 4>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        default: return launch_pp<true, true, 128, 192>(st, Xt, 0, Wp, 0, M, N, K, epi);
+    }
+}
+
+// The FFN's paired up-projection (N output columns, 2N weight rows), x and the
+// weight in the block layout.  Models as above, fitted to nine tiles of the
+// persistent kernel (scatter 5%) and seven of the other (10%) on 80 products (M
+// 17-4096, N 1024-8192, K 512-3072, situ and GEGLU, whose epilogues differ); the
+// choice is 1.5% off the fastest of all on average (10% at worst).  Against the
+// 256 x 320, two-block and skinny kernels, us (M, N, K):
+//   situ 3952 x 8192 x 3072   277.6 -> 176.5 (256 x 256, windowed tables)
+//   GEGLU 892 x 5376 x 1536   33.9 -> 20.9 (192 x 256)
+//   situ 1164 x 3072 x 2304   46.1 -> 26.5 (128 x 256)
+//   situ 200 x 5120 x 1280    21.1 -> 11.2 (32 x 64, K over waves)
+//   GEGLU 353 x 2048 x 1792   27.3 -> 8.6 (64 x 64)
+// and 1.95 times as fast over all 80.  Up to 16 rows the skinny kernel stays (one
+// row block: 5.1 against 5.4 us at 16 x 5120 x 1280).
+constexpr PpTile kPairTiles[] = {{256, 320}, {256, 256}, {192, 256}, {128, 256}, {128, 192}};
+constexpr WavekTile kPairWavekTiles[] = {
+    {1, 2, 8, 4, 3}, {2, 2, 4, 4, 5}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
+template <class Epi>
+hipError_t launch_pair_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N,
+                             int K, bool situ, const Epi& epi) {
+    if (M <= 16) return launch_skinny<4, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
+    const PpModel pm = {4.05, 0.0771, 0.1875, 0.76, situ ? 1.76 : 0.85, 0.77};
+    const WavekModel wm = {1.88, 0.0058, 0.42, (situ ? 0.32 : 0.236) / 16, 0.084e-6};
+    double t = 0;
+    const int tile = pp_tile(pm, kPairTiles, true, M, N, K, &t);
+    switch (wavek_tile(wm, kPairWavekTiles, 1.03, M, 2 * int64_t(N), K, N, &t)) {
+        case 0: return launch_wavek<1, 2, 8, 4>(st, Xt, Wp, M, N, K, epi);
+        case 1: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+        case 2: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
+        case 3: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
+        default: break;
+    }
+    switch (tile) {
+        case 0: return launch_pp<true, true, 256, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 1: return launch_pp<true, true, 256, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 2: return launch_pp<true, true, 192, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        case 3: return launch_pp<true, true, 128, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
         default: return launch_pp<true, true, 128, 192>(st, Xt, 0, Wp, 0, M, N, K, epi);
     }
 }
@@ -2527,40 +2638,32 @@ hipError_t gemm_dequant_packed(hipStream_t st, const int8_t* At, const int8_t* B
                        EpiDequant{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16});
 }
 
-template <int ACT>
-static hipError_t act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
-                            const EpiAct<ACT>& epi, int M, int N, int K, bool packed) {
-    if (packed) return launch_pp<true, true>(st, At, 0, B, 0, M, N, K, epi);
-    return launch_pp<true>(st, At, 0, B, ldb, M, N, K, epi);
-}
-
 hipError_t gemm_act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                           void* out, int64_t ldo, const float* xs, const float* ws, int M, int N,
-                          int K, int act, bool packed) {
+                          int K, int act) {
     uint16_t* o = static_cast<uint16_t*>(out);
     const uint16_t* tab = activation_tables();
     switch (act) {
-        case 3: return act_pp_xt(st, At, B, ldb, EpiAct<3>{o, ldo, xs, ws, N, tab}, M, N, K, packed);
-        case 4: return act_pp_xt(st, At, B, ldb, EpiAct<4>{o, ldo, xs, ws, N, tab}, M, N, K, packed);
-        case 5: return act_pp_xt(st, At, B, ldb, EpiAct<5>{o, ldo, xs, ws, N, tab}, M, N, K, packed);
+        case 3: return launch_pp<true>(st, At, 0, B, ldb, M, N, K, EpiAct<3>{o, ldo, xs, ws, N, tab});
+        case 4: return launch_pp<true>(st, At, 0, B, ldb, M, N, K, EpiAct<4>{o, ldo, xs, ws, N, tab});
+        case 5: return launch_pp<true>(st, At, 0, B, ldb, M, N, K, EpiAct<5>{o, ldo, xs, ws, N, tab});
         default: return hipErrorInvalidValue;
     }
 }
 
-bool skinny_applies(int M, bool paired) { return M <= (paired ? kSkinnyPairedM : 64); }
-
-hipError_t gemm_act_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
-                              int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
-                              int act) {
+hipError_t gemm_act_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
+                           int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
+                           int act) {
     uint16_t* o = static_cast<uint16_t*>(out);
     const uint16_t* tab = activation_tables();
     switch (act) {
-        case 3: return launch_skinny<4, EpiAct<3>, true, true>(st, At, 0, Bp, 0, M, N, K,
-                                                              EpiAct<3>{o, ldo, xs, ws, N, tab});
-        case 4: return launch_skinny<4, EpiAct<4>, true, true>(st, At, 0, Bp, 0, M, N, K,
-                                                              EpiAct<4>{o, ldo, xs, ws, N, tab});
-        case 5: return launch_skinny<1, EpiAct<5>, true, true>(st, At, 0, Bp, 0, M, N, K,
-                                                              EpiAct<5>{o, ldo, xs, ws, N, tab});
+        case 3: return launch_pair_tiles(st, At, Bp, M, N, K, true, EpiAct<3>{o, ldo, xs, ws, N, tab});
+        case 4: return launch_pair_tiles(st, At, Bp, M, N, K, false, EpiAct<4>{o, ldo, xs, ws, N, tab});
+        case 5: {
+            const EpiAct<5> epi{o, ldo, xs, ws, N, tab};
+            if (M <= 64) return launch_skinny<1, EpiAct<5>, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
+            return launch_tiles(st, At, Bp, M, N, K, epi);
+        }
         default: return hipErrorInvalidValue;
     }
 }

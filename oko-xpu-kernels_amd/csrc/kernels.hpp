@@ -83,12 +83,17 @@ hipError_t gemm_dequant_nn_xt(hipStream_t st, const int8_t* At, const int8_t* Bk
                               void* out, int64_t ldo, const float* xs, int M, int N, int K,
                               bool packed = false);
 // whether the persistent ping-pong kernel takes the dequant GEMM (paired:
-// the FFN's up-projection) of this shape, and the up-projection with A in the
-// MFMA block layout on that kernel (packed: B is pack_weight's copy)
+// the FFN's up-projection) of this shape from a row-major weight, and the
+// up-projection with A in the MFMA block layout and such a weight on that kernel
 bool pp_applies(int M, int N, int K, bool paired);
 hipError_t gemm_act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                           void* out, int64_t ldo, const float* xs, const float* ws, int M, int N,
-                          int K, int act, bool packed = false);
+                          int K, int act);
+// the up-projection with A in the block layout and B pack_weight's copy, any
+// shape: the kernel and tile are chosen by it
+hipError_t gemm_act_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
+                           int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
+                           int act);
 // w [N, K] int8 (row-major, K % 16 == 0) in the MFMA block layout, the bytes
 // past K zero: the packed weight the GEMMs above read with packed = true
 // (tiled_bytes(N, K) bytes at out)
@@ -125,13 +130,6 @@ hipError_t gemm_i32_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, i
 hipError_t gemm_act(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,
                     void* out, int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
                     int act, const int8_t* Bp = nullptr);
-// The FFN's up-projection on the skinny kernel with x in the MFMA block layout
-// (At) and the packed weight (Bp), for the batches launch_gemm gives it
-// (skinny_applies: M <= 64; paired activations 3 and 4, M <= 256)
-bool skinny_applies(int M, bool paired);
-hipError_t gemm_act_skinny_xt(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,
-                              int64_t ldo, const float* xs, const float* ws, int M, int N, int K,
-                              int act);
 hipError_t dequant_epilogue(hipStream_t st, const int32_t* acc, int64_t acc_ld, void* out,
                             const float* xs, const float* ws, const float* bias, int64_t M,
                             int64_t N);

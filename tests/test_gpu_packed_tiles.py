@@ -51,3 +51,31 @@ def test_packed_tiles_exact(dev, m, n, k):
     assert torch.equal(got, acc)
     _, yr = reference(x, w8, ws, bias, res, rscale)
     assert torch.equal(int8.linear(x, w8, ws, bias, residual=res, residual_scale=rscale), yr)
+
+
+# The FFN's up-projection, (M, inner, K): the paired 256x320 tile (a ragged batch),
+# 256x256, 192x256, 128x256 and 128x192, the wave-split 64x64, 32x64, 32x32 and 16x32,
+# and the skinny kernel's 16 rows
+FFN_SHAPES = [(4090, 5120, 512), (2315, 2560, 256), (892, 5376, 512), (514, 5120, 256),
+              (357, 4608, 256), (304, 1280, 512), (45, 2816, 256), (33, 1536, 256), (19, 512, 256),
+              (16, 1024, 512)]
+
+
+@pytest.mark.parametrize("m,inner,k", FFN_SHAPES)
+@pytest.mark.parametrize("act", ["situ", "geglu_erf", "gelu_erf"])
+def test_ffn_packed_tiles_exact(dev, act, m, inner, k):
+    """Against the library's unfused chain (int32 product, the row kernel that
+    dequantizes, activates and quantizes it, int32 product, dequant), each
+    checked against the oracle elsewhere.  Row magnitudes from 2^-16 to 2^8 put the
+    table lookups inside and on both sides of the epilogue's windows."""
+    up_rows = inner if act == "gelu_erf" else 2 * inner
+    uw8, us = int8.prepare_weight(weight(up_rows, k, seed=inner + k).to(dev))
+    dw8, ds = int8.prepare_weight(weight(k, inner, seed=inner + k + 1).to(dev))
+    mag = torch.exp2(torch.linspace(-16, 8, m))[torch.randperm(m, generator=torch.Generator().manual_seed(m))]
+    x = (activation(m, k, seed=m).float() * mag[:, None]).to(torch.bfloat16).to(dev)
+    bias = weight(1, k, seed=6, std=0.01)[0].to(dev)
+    acc, xs = int8.linear_acc(x, uw8, us)
+    q, s = int8.dequant_act_quantize(acc, xs, us, act)
+    want = int8.dequant(int8.int_mm(q, dw8.t()), s, ds, bias)
+    got = int8.ffn(x, uw8, us, dw8, ds, bias, act=act)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
