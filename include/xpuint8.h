@@ -409,6 +409,12 @@ int xpuint8_linear_dx_int8_noalloc_stream(const void *stream, const void *dy, co
 int xpuint8_prepare_weight_stream(const void *stream, const void *w, int8_t *q, float *scale,
                                   int64_t N, int64_t K);
 
+/* The same with the packed copy of the codes (xpuint8_pack_weight_stream's,
+ * xpuint8_packed_weight_bytes(N, K) bytes at `packed`) written in the same pass.
+ * N % 16 == 0.  No reference counterpart. */
+int xpuint8_prepare_weight_packed_stream(const void *stream, const void *w, int8_t *q,
+                                         int8_t *packed, float *scale, int64_t N, int64_t K);
+
 /* Per-row int8 quantization without rotation (the gradient row quantizer):
  * x bf16 [M,N] -> q int8 [M,N] + scale fp32 [M], bit-identical to
  * quantize_row_torch (python/xpu_kernels/int8/ops.py:320-330).  With a

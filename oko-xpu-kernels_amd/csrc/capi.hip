@@ -1048,6 +1048,19 @@ int xpuint8_prepare_weight_stream(const void* stream, const void* w, int8_t* q, 
     return launched(prepare_weight(as_stream(stream), w, q, scale, N, int(K)), "prepare_weight");
 }
 
+int xpuint8_prepare_weight_packed_stream(const void* stream, const void* w, int8_t* q,
+                                         int8_t* packed, float* scale, int64_t N, int64_t K) {
+    XPU_TRY(check_rows(N, K));
+    if (N % 16 != 0) return fail(2, "prepare_weight_packed: N must be a multiple of 16");
+    XPU_NONNULL(w); XPU_NONNULL(q); XPU_NONNULL(packed); XPU_NONNULL(scale);
+    XPU_TRY(ensure_device());
+    hipStream_t st = as_stream(stream);
+    if (rowquant_can_tile(int(K)))
+        return launched(prepare_weight(st, w, q, scale, N, int(K), packed), "prepare_weight");
+    XPU_TRY(launched(prepare_weight(st, w, q, scale, N, int(K)), "prepare_weight"));
+    return launched(pack_weight(st, q, packed, N, int(K)), "prepare_weight (pack)");
+}
+
 int xpuint8_quantize_row_stream(const void* stream, const void* x, const float* col_scale,
                                 int8_t* q, float* scale, int64_t M, int64_t N) {
     XPU_TRY(check_epilogue(M, N));

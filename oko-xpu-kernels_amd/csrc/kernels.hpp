@@ -32,8 +32,10 @@ hipError_t dequant_act_quantize(hipStream_t st, const int32_t* acc, int64_t acc_
 hipError_t rotate_bf16(hipStream_t st, const void* x, void* out, int64_t M, int K);
 hipError_t dequant_weight(hipStream_t st, const int8_t* w8, const float* scale, void* out,
                           int64_t N, int K);
+// packed (optional; N % 16 == 0 and rowquant_can_tile(K)): the codes in the MFMA
+// block layout too, as pack_weight lays them out
 hipError_t prepare_weight(hipStream_t st, const void* w, int8_t* q, float* scale, int64_t N,
-                          int K);
+                          int K, int8_t* packed = nullptr);
 hipError_t quantize_row(hipStream_t st, const void* x, const float* colscale, int8_t* q,
                         float* scale, int64_t M, int N, bool tiled = false);
 // the quantizers above (rotating with act 0, and quantize_row) can write q in

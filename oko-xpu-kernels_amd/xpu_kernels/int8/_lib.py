@@ -98,6 +98,7 @@ def _signatures():
         "xpuint8_linear_dx_int8_workspace_size": ([i64] * 3, i64),
         "xpuint8_linear_dx_int8_noalloc_stream": ([vp] * 5 + [i64] * 3, c_int),
         "xpuint8_prepare_weight_stream": ([vp] * 4 + [i64] * 2, c_int),
+        "xpuint8_prepare_weight_packed_stream": ([vp] * 5 + [i64] * 2, c_int),
         "xpuint8_quantize_row_stream": ([vp] * 5 + [i64] * 2, c_int),
         "xpuint8_linear_dw_stream": ([vp] * 4 + [i64] * 3, c_int),
         "xpuint8_linear_dw_work_stream": ([vp] * 4 + [i64] * 3 + [vp, i64], c_int),

@@ -17,6 +17,7 @@ bf16 GPU tensor (an fp32 training model) or a dimension is not a multiple of
 
 from __future__ import annotations
 
+import weakref
 from typing import Optional
 
 import torch
@@ -92,7 +93,6 @@ def pack_weight(w8):
         raise RuntimeError("pack_weight() allocates and writes the packed copy of a weight; "
                            "inside a device-graph capture it would be recomputed on every "
                            "replay. Call it before capturing.")
-    import weakref
     lib = _lib()
     n, k = w8.shape
     need = lib.xpuint8_packed_weight_bytes(n, k)
@@ -102,6 +102,13 @@ def pack_weight(w8):
     rc = lib.xpuint8_pack_weight_stream(_stream(w8.device), _ptr(w8), _ptr(packed), n, k)
     if rc != 0:
         _err(lib, "pack_weight")
+    _attach_packed(w8, key, packed)
+    return True
+
+
+def _attach_packed(w8, key, packed):
+    """Enter ``packed`` as the packed copy of ``w8`` (key: ``_pack_key(w8)``)."""
+    n, k = w8.shape
     st = w8.untyped_storage()
     old = _PACKED.get(key)
     if old is not None and old[0]() is st:
@@ -110,7 +117,6 @@ def pack_weight(w8):
         ref = weakref.ref(st)
         weakref.finalize(st, _drop_packed, key, ref)
     _PACKED[key] = [ref, w8._version, (n, k), packed, None]
-    return True
 
 
 def _packed_entry(w8):
@@ -218,11 +224,19 @@ def prepare_weight(w, group: int = 256, *, pack: bool = True):
     n, k = w2.shape
     q = torch.empty((n, k), device=w.device, dtype=torch.int8)
     scale = torch.empty((n,), device=w.device, dtype=torch.float32)
-    rc = lib.xpuint8_prepare_weight_stream(_stream(w.device), _ptr(w2), _ptr(q), _ptr(scale), n, k)
+    key = _pack_key(q) if pack and not is_capturing() else None
+    if key is not None:
+        # the codes and their packed copy (N, K multiples of 16: N*K bytes) in one pass
+        packed = torch.empty(n * ((k + 63) // 64 * 64), device=w.device, dtype=torch.int8)
+        rc = lib.xpuint8_prepare_weight_packed_stream(_stream(w.device), _ptr(w2), _ptr(q),
+                                                      _ptr(packed), _ptr(scale), n, k)
+    else:
+        rc = lib.xpuint8_prepare_weight_stream(_stream(w.device), _ptr(w2), _ptr(q), _ptr(scale),
+                                               n, k)
     if rc != 0:
         _err(lib, "prepare_weight")
-    if pack and not is_capturing():
-        pack_weight(q)
+    if key is not None:
+        _attach_packed(q, key, packed)
     return q, scale
 
 

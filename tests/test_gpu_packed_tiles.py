@@ -79,3 +79,21 @@ def test_ffn_packed_tiles_exact(dev, act, m, inner, k):
     want = int8.dequant(int8.int_mm(q, dw8.t()), s, ds, bias)
     got = int8.ffn(x, uw8, us, dw8, ds, bias, act=act)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# one row group of one 256-group; rows per block that do not divide N; two groups
+# per lane (K > 16384); longer than the one-pass kernel takes
+@pytest.mark.parametrize("n,k", [(16, 256), (10240, 1280), (48, 5120), (1040, 768), (32, 16896),
+                                 (16, 33024)])
+def test_prepare_weight_packed_exact(dev, n, k):
+    """prepare_weight's one-pass codes, scales and packed copy against the two
+    separate passes."""
+    from xpu_kernels.int8 import _lib as L, ops
+    w = weight(n, k, seed=n + k).to(dev)
+    w8, ws = int8.prepare_weight(w)
+    w8r, wsr = int8.prepare_weight(w, pack=False)
+    assert torch.equal(w8, w8r) and torch.equal(ws, wsr)
+    packed = torch.empty(n * k, device=dev, dtype=torch.int8)
+    assert L._lib().xpuint8_pack_weight_stream(L._stream(dev), L._ptr(w8r), L._ptr(packed), n,
+                                               k) == 0
+    assert torch.equal(ops._packed_for(w8), packed)
