@@ -26,6 +26,24 @@ _LOCK = threading.Lock()
 
 LIBNAME = "libxpuint8.so"
 
+#: the hot calls' host path in native code (csrc/host_ops.cpp) once the library
+#: is loaded, else None; every caller has a Python path beside it
+HOST = None
+#: the packed-weight registry (ops.py): storage data_ptr -> [weakref to the
+#: storage, version, shape, packed, packed_nn]
+PACKED = {}
+
+#: the library's entry points that HOST calls, in its order
+_HOST_ENTRIES = (
+    "xpuint8_last_error", "xpuint8_linear_workspace_size", "xpuint8_linear_packed_stream",
+    "xpuint8_ffn_workspace_size", "xpuint8_ffn_packed_stream",
+    "xpuint8_linear_backward_int8_workspace_size", "xpuint8_linear_backward_int8_stream",
+    "xpuint8_linear_backward_dense_workspace_size", "xpuint8_linear_backward_dense_stream",
+    "xpuint8_linear_dx_split_workspace_size", "xpuint8_linear_dx_stream",
+    "xpuint8_linear_dw_workspace_size", "xpuint8_linear_dw_work_stream",
+    "xpuint8_column_sum_workspace_size", "xpuint8_column_sum_stream",
+    "xpuint8_convrot_quantize_stream", "xpuint8_linear_acc_packed_stream")
+
 
 def _candidate_paths():
     for var in ("XPU_KERNELS_LIB", "XPU_INT8_LIB"):
@@ -132,9 +150,29 @@ def library_path() -> Optional[str]:
     return None
 
 
+# torch's accessor of the current stream's raw handle (0.1 us against 2 us for
+# building a torch.cuda.Stream per call; a private name, so the public form
+# stays as the fallback)
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _bind_host(lib):
+    """The native host path bound to the loaded library, or None: not built, built
+    for another torch, or torch without the raw stream accessor."""
+    if _RAW_STREAM is None:
+        return None
+    try:
+        from . import _host
+    except ImportError:
+        return None
+    _host.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _HOST_ENTRIES),
+               _RAW_STREAM, PACKED)
+    return _host
+
+
 def load():
     """Load, bind and initialise the library.  Returns the ctypes handle or None."""
-    global _LIB, _TRIED, _PATH, _ERR
+    global _LIB, _TRIED, _PATH, _ERR, HOST
     if _LIB is not None or _TRIED:
         return _LIB
     with _LOCK:
@@ -152,6 +190,7 @@ def load():
             if lib.xpuint8_init() != 0:
                 _ERR = f"{path}: {lib.xpuint8_last_error()!r}"
                 continue
+            HOST = _bind_host(lib)
             _LIB, _PATH = lib, path
             return lib
         if _ERR is None:
@@ -183,12 +222,6 @@ def _lib():
 
 def _err(lib, what):
     raise RuntimeError(f"{what}: {lib.xpuint8_last_error()!r}")
-
-
-# torch's accessor of the current stream's raw handle (0.1 us against 2 us for
-# building a torch.cuda.Stream per call; a private name, so the public form
-# stays as the fallback)
-_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(device):

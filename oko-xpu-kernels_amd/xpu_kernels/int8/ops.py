@@ -17,14 +17,17 @@ bf16 GPU tensor (an fp32 training model) or a dimension is not a multiple of
 
 from __future__ import annotations
 
+import functools
 import weakref
 from typing import Optional
 
 import torch
 
 from .._capture import is_capturing
+from . import _lib as _L
 from ._lib import (
     ACTIVATIONS,
+    PACKED as _PACKED,
     PAIRED_ACTIVATIONS,
     _c,
     _err,
@@ -51,9 +54,9 @@ def _opt(t):
 # version counter holds the value it was packed at, and it is dropped when
 # the storage is.  Writes the version counter does not see (through
 # ``.data``, DLPack or raw pointers) need a new :func:`pack_weight`.
-# storage data_ptr -> [weakref to the storage, version, shape, packed, packed_nn]
-# (packed_nn: the form linear_dx_int8's product reads, made at its first use)
-_PACKED = {}
+# _PACKED: storage data_ptr -> [weakref to the storage, version, shape, packed,
+# packed_nn] (packed_nn: the form linear_dx_int8's product reads, made at its
+# first use); csrc/host_ops.cpp reads it by the same rules
 
 
 def _pack_key(w8):
@@ -72,6 +75,7 @@ def _pack_key(w8):
 
 
 def _drop_packed(key, ref):
+    """Called when the storage behind ``ref`` is freed."""
     e = _PACKED.get(key)
     if e is not None and e[0] is ref:
         del _PACKED[key]
@@ -114,8 +118,7 @@ def _attach_packed(w8, key, packed):
     if old is not None and old[0]() is st:
         ref = old[0]
     else:
-        ref = weakref.ref(st)
-        weakref.finalize(st, _drop_packed, key, ref)
+        ref = weakref.ref(st, functools.partial(_drop_packed, key))
     _PACKED[key] = [ref, w8._version, (n, k), packed, None]
 
 
@@ -176,6 +179,10 @@ def quantize(x):
     """Rotate and quantize an activation: bf16 [.., K] -> (int8 [.., K], fp32 [..])
     (ops.py:40-52)."""
     lib = _lib()
+    if _L.HOST is not None:
+        r = _L.HOST.quantize(x)
+        if r is not None:
+            return r
     x2, shape = _flat2d(x)
     m, k = x2.shape
     q = torch.empty((m, k), device=x.device, dtype=torch.int8)
@@ -292,6 +299,10 @@ def linear_dx(dy, w):
     kernel (fp32 accumulation, one rounding, like the matmul it replaces);
     other dtypes and shapes are torch's matmul in their dtype, the
     reference's own computation."""
+    if _L.HOST is not None:
+        r = _L.HOST.linear_dx(dy, w)
+        if r is not None:
+            return r
     if dy.shape[-1] != w.shape[0]:
         raise ValueError(f"dy has {dy.shape[-1]} columns but w has {w.shape[0]} rows")
     n, k = int(w.shape[0]), int(w.shape[1])
@@ -320,6 +331,10 @@ def linear_dw(dy, x):
     The contraction runs over the batch (token) dimension, so the batch dims
     must agree.
     """
+    if _L.HOST is not None:
+        r = _L.HOST.linear_dw(dy, x)
+        if r is not None:
+            return r
     if dy.shape[-2] != x.shape[-2]:
         raise ValueError(
             f"dy has {dy.shape[-2]} rows but x has {x.shape[-2]}: the batch "
@@ -352,6 +367,10 @@ def column_sum(dy):
     16) takes one HIP column-sum pass (fp32 sums of 32-row chunks in row
     order, then the chunks in order, one bf16 rounding) instead of torch's
     reduction, whose order is its own; anything else is torch's sum."""
+    if _L.HOST is not None:
+        r = _L.HOST.column_sum(dy)
+        if r is not None:
+            return r
     if (isinstance(dy, torch.Tensor) and dy.dim() == 2 and dy.dtype == torch.bfloat16
             and dy.is_cuda and dy.shape[0] > 0 and dy.shape[1] % 16 == 0):
         lib = _lib()
@@ -390,6 +409,11 @@ def _linear_backward(dy, w8, w_scale, want_dbias, bias_dtype, mode):
     autograd's cast would give) or bf16; otherwise bf16, which autograd casts
     as before."""
     lib = _lib()
+    if _L.HOST is not None:
+        r = _L.HOST.backward(dy, w8, w_scale, want_dbias, bias_dtype == torch.float32,
+                             mode == "dense")
+        if r is not None:
+            return r
     m, n = int(dy.shape[0]), int(dy.shape[1])
     k = int(w8.shape[1])
     d2 = _c(dy)
@@ -713,6 +737,10 @@ def dequant_act_quantize(acc, x_scale, w_scale, activation="situ"):
 def linear_acc(x, w8, w_scale, act: Optional[str] = None):
     """The GEMM without the output dequant: ``(int32 [M, N], fp32 [M])``
     (ops.py:571-588)."""
+    if act is None and _L.HOST is not None:
+        r = _L.HOST.linear_acc(x, w8)
+        if r is not None:
+            return r
     if act is None and _acc_one_call(x, w8):
         x2 = _c(x.reshape(-1, x.shape[-1]))
         return _linear_acc_bf16(_lib(), x2, _c(w8), x2.shape[0], w8.shape[0], w8.shape[1])
@@ -786,6 +814,10 @@ def linear(x, w8, w_scale, bias=None, act: Optional[str] = None, residual=None,
     ``residual``/``residual_scale`` apply ``residual + residual_scale * out``;
     ``return_acc`` returns ``(int32 [M, N], fp32 [M], fp32 [N])`` instead.
     """
+    if act is None and residual is None and not return_acc and _L.HOST is not None:
+        y = _L.HOST.linear(x, w8, w_scale, bias)
+        if y is not None:
+            return y
     reason = unsupported_reason(x, w8, w_scale, act)
     if reason is not None:
         raise TypeError(reason)
@@ -819,7 +851,8 @@ def linear(x, w8, w_scale, bias=None, act: Optional[str] = None, residual=None,
         out = _linear_residual_bf16(lib, x2, w8c, ws, b, b16, res, rs, m, n, k)
         return out.reshape(*x.shape[:-1], n)
     if act is None and return_acc:
-        acc, xs = _linear_acc_bf16(lib, x2, w8c, m, n, k)
+        r = _L.HOST.linear_acc(x2, w8c) if _L.HOST is not None else None
+        acc, xs = _linear_acc_bf16(lib, x2, w8c, m, n, k) if r is None else r
         return acc, xs, expand_scale(w_scale, n, acc.device)
     if act is None:
         xq, xs = quantize(x2)
@@ -930,6 +963,10 @@ def ffn(x, up_w8, up_scale, down_w8, down_scale, down_bias=None, act="situ"):
     if act not in ("situ", "geglu_erf", "gelu_erf"):
         raise TypeError(f"the fused FFN supports situ, geglu_erf and gelu_erf, "
                         f"not {act!r}")
+    if _L.HOST is not None:
+        y = _L.HOST.ffn(x, up_w8, up_scale, down_w8, down_scale, down_bias, ACTIVATIONS[act])
+        if y is not None:
+            return y
     paired = act in PAIRED_ACTIVATIONS
     reason = unsupported_reason(x, up_w8, up_scale, None)
     if reason is not None:

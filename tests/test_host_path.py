@@ -1,0 +1,225 @@
+"""The native host path (csrc/host_ops.cpp, ``int8._lib.HOST``): the same results
+and the same errors as the Python path beside it, over the argument forms both
+may see -- dtypes, strides, offsets, scales and biases of every accepted kind,
+batch dims, empty batches, refused shapes, active torch modes -- and the packed
+copy's rules."""
+
+import importlib
+
+import pytest
+import torch
+
+from xpu_kernels import int8
+from xpu_kernels.int8 import _lib as L, ops
+
+
+def test_module_is_built_and_answers_none_unbound():
+    """Built beside the library; CPU tensors (and an unbound module) are left to
+    the Python path."""
+    host = importlib.import_module("xpu_kernels.int8._host")
+    x = torch.zeros(2, 256, dtype=torch.bfloat16)
+    w8 = torch.zeros(16, 256, dtype=torch.int8)
+    assert host.linear(x, w8, torch.ones(16), None) is None
+    assert host.quantize(x) is None and host.column_sum(x) is None
+    with pytest.raises(TypeError):
+        host.linear(x, w8)
+    with pytest.raises(TypeError):
+        host.bind((), None, {})
+
+
+def _outcome(fn):
+    try:
+        r = fn()
+    except Exception as e:  # noqa: BLE001 - the error is the outcome
+        return type(e).__name__, str(e)
+    return [None if t is None else (tuple(t.shape), t.dtype, t.detach().cpu().clone())
+            for t in (r if isinstance(r, tuple) else (r,))]
+
+
+def _same(a, b):
+    if isinstance(a, tuple) or isinstance(b, tuple):
+        return a == b
+    return len(a) == len(b) and all(
+        (p is None and q is None) or (p[:2] == q[:2] and torch.equal(p[2], q[2]))
+        for p, q in zip(a, b))
+
+
+def _both(monkeypatch, fn):
+    assert L.HOST is not None
+    fast = _outcome(fn)
+    monkeypatch.setattr(L, "HOST", None)
+    slow = _outcome(fn)
+    monkeypatch.undo()
+    assert _same(fast, slow), (fast, slow)
+    return fast
+
+
+def _bf(*shape, dev, seed=0):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=dev).to(torch.bfloat16)
+
+
+def _x_forms(dev, m, k):
+    x = _bf(m, k, dev=dev)
+    yield "plain", x
+    yield "batched", x.reshape(1, m, k)
+    yield "vector", x[0]
+    yield "column slice", _bf(m, 2 * k, dev=dev)[:, :k]
+    yield "transposed", _bf(k, m, dev=dev).t()
+    yield "row slice", _bf(m + 3, k, dev=dev)[3:]
+    yield "misaligned", torch.cat([x.reshape(-1), x[0, :8]])[1:1 + m * k].reshape(m, k)
+    yield "fp32", x.float()
+    yield "fp16", x.half()
+    yield "cpu", x.cpu()
+    yield "empty", x[:0]
+    yield "wrong columns", x[:, : k - 16].contiguous()
+    yield "needs grad", x.clone().requires_grad_(True)
+    yield "parameter", torch.nn.Parameter(x)
+
+
+@pytest.mark.gpu
+def test_linear_same_over_inputs(dev, monkeypatch):
+    w8, ws = int8.prepare_weight(_bf(48, 512, dev=dev, seed=1))
+    for name, x in _x_forms(dev, 21, 512):
+        for call in (lambda: int8.linear(x, w8, ws), lambda: int8.linear_acc(x, w8),
+                     lambda: int8.linear(x, w8, ws, return_acc=True), lambda: int8.quantize(x)):
+            _both(monkeypatch, call)
+
+
+@pytest.mark.gpu
+def test_linear_same_over_weights_scales_and_biases(dev, monkeypatch):
+    x = _bf(21, 512, dev=dev)
+    w = _bf(48, 512, dev=dev, seed=1)
+    w8, ws = int8.prepare_weight(w)
+    w8r, _ = int8.prepare_weight(w, pack=False)
+    wide = torch.zeros(48, 1024, device=dev, dtype=torch.int8)
+    wide[:, :512] = w8
+    weights = {"packed": w8, "plain": w8r, "alias": w8.detach(), "column slice": wide[:, :512],
+               "row slice": w8[16:], "bf16": w, "cpu": w8.cpu(), "3-d": w8.reshape(1, 48, 512),
+               "K % 256": torch.zeros(48, 272, device=dev, dtype=torch.int8),
+               "N % 16": w8[:40].contiguous()}
+    scales = {"plain": ws, "column": ws.reshape(48, 1), "scalar tensor": ws[:1], "float": 0.5,
+              "bf16": ws.to(torch.bfloat16), "cpu": ws.cpu(), "strided": ws.repeat(2)[::2],
+              "wrong length": ws[:47], "misaligned": torch.cat([ws, ws])[1:49], "int": 3,
+              "int tensor": torch.ones(48, device=dev, dtype=torch.int32)}
+    bias = _bf(48, dev=dev, seed=2)
+    biases = {"none": None, "bf16": bias, "fp32": bias.float(), "fp16": bias.half(),
+              "strided": _bf(96, dev=dev)[::2], "misaligned": _bf(64, dev=dev)[1:49],
+              "cpu": bias.cpu(), "row": bias.reshape(1, 48), "scalar": bias[:1],
+              "wrong length": bias[:32]}
+    for w_ in weights.values():
+        _both(monkeypatch, lambda: int8.linear(x, w_, ws))
+    for s in scales.values():
+        _both(monkeypatch, lambda: int8.linear(x, w8, s))
+    for b in biases.values():
+        _both(monkeypatch, lambda: int8.linear(x, w8, ws, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["situ", "geglu_erf", "gelu_erf"])
+def test_ffn_same(dev, monkeypatch, act):
+    rows = 512 if act == "gelu_erf" else 1024
+    up, us = int8.prepare_weight(_bf(rows, 256, dev=dev, seed=3))
+    dn, ds = int8.prepare_weight(_bf(256, 512, dev=dev, seed=4))
+    bias = _bf(256, dev=dev, seed=5)
+    for name, x in _x_forms(dev, 5, 256):
+        _both(monkeypatch, lambda: int8.ffn(x, up, us, dn, ds, bias, act=act))
+    x = _bf(5, 256, dev=dev)
+    for d in (dn, dn.t(), dn[:, :256], up):
+        _both(monkeypatch, lambda: int8.ffn(x, up, us, d, ds, act=act))
+    for s in (ds, ds[:1], 0.25, ds.double(), ds.reshape(256, 1)):
+        _both(monkeypatch, lambda: int8.ffn(x, up, us, dn, s, bias.float(), act=act))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["int8", "dense"])
+@pytest.mark.parametrize("pack", [True, False])
+def test_backward_same(dev, monkeypatch, mode, pack):
+    w8, ws = int8.prepare_weight(_bf(48, 512, dev=dev, seed=1), pack=pack)
+    for x_dtype in (torch.bfloat16, torch.float32):
+        for bias in (None, _bf(48, dev=dev), _bf(48, dev=dev).float()):
+            for expanded in (False, True):
+                def step():
+                    x = _bf(21, 512, dev=dev).to(x_dtype).requires_grad_(True)
+                    b = None if bias is None else bias.clone().requires_grad_(True)
+                    y = int8.int8_linear(x, w8, ws, b, mode=mode)
+                    y.backward(torch.ones((), device=dev, dtype=y.dtype).expand_as(y) if expanded
+                               else _bf(21, 48, dev=dev, seed=7).to(y.dtype))
+                    return y, x.grad, None if b is None else b.grad
+                _both(monkeypatch, step)
+
+
+@pytest.mark.gpu
+def test_products_same(dev, monkeypatch):
+    dy, w, x = _bf(37, 48, dev=dev), _bf(48, 80, dev=dev, seed=1), _bf(37, 80, dev=dev, seed=2)
+    for d in (dy, dy.reshape(1, 37, 48), _bf(48, 37, dev=dev).t(), dy.float(), dy[:, :40], dy[:0]):
+        _both(monkeypatch, lambda: int8.linear_dx(d, w))
+        _both(monkeypatch, lambda: int8.linear_dw(d, x))
+        _both(monkeypatch, lambda: ops.column_sum(d))
+    for w_ in (w.t(), w.float(), w[:, :72], w.cpu()):
+        _both(monkeypatch, lambda: int8.linear_dx(dy, w_))
+
+
+@pytest.mark.gpu
+def test_packed_rules_same(dev, monkeypatch):
+    """The packed copy is read while it is valid, and the row-major codes again
+    after an in-place write, on both paths."""
+    x = _bf(70, 512, dev=dev)
+    w8, ws = int8.prepare_weight(_bf(48, 512, dev=dev, seed=1))
+    _both(monkeypatch, lambda: int8.linear(x, w8, ws))
+    w8[3] = 5
+    stale = _both(monkeypatch, lambda: int8.linear(x, w8, ws))
+    want = int8.linear(x, w8.clone(), ws)
+    assert torch.equal(stale[0][2], want.cpu())
+    # a stale copy that is used would show: poison it
+    w8b, wsb = int8.prepare_weight(_bf(48, 512, dev=dev, seed=1))
+    ops._packed_entry(w8b)[3].zero_()
+    assert int8.linear(x, w8b, wsb).abs().max() == 0
+    w8b.add_(0)
+    assert int8.linear(x, w8b, wsb).abs().max() > 0
+
+
+@pytest.mark.gpu
+def test_modes_take_the_python_path(dev):
+    """A torch-function or dispatch mode sees the call's torch operations."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    w8, ws = int8.prepare_weight(_bf(48, 512, dev=dev, seed=1))
+    x = _bf(4, 512, dev=dev)
+    want, seen = int8.linear(x, w8, ws), []
+
+    class Fn(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Disp(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    for mode in (Fn, Disp):
+        seen.clear()
+        with mode():
+            y = int8.linear(x, w8, ws)
+        assert seen and torch.equal(y, want)
+
+
+@pytest.mark.gpu
+def test_streams_and_threads(dev):
+    """The call runs on the caller's current stream, from any thread."""
+    import threading
+    w8, ws = int8.prepare_weight(_bf(1024, 512, dev=dev, seed=1))
+    x = _bf(300, 512, dev=dev)
+    want, got = int8.linear(x, w8, ws), {}
+    torch.cuda.synchronize()
+
+    def work(i):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for _ in range(20):
+                got[i] = int8.linear(x, w8, ws)
+        st.synchronize()
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert len(got) == 4 and all(torch.equal(y, want) for y in got.values())
