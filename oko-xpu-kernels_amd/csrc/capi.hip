@@ -180,10 +180,14 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
     float* a = reinterpret_cast<float*>(work + L.a);
     int8_t* wt = reinterpret_cast<int8_t*>(work + L.wt);
     void* pre = work + L.pre;
-    // the split-K kernel reads w8 [N, K] as it is stored (transposing LDS
-    // reads) and q in the MFMA block layout, written so by the quantizer;
-    // other shapes take a row-major q, the transposed copy and the NT kernels
-    if (splitk_nn_applies(int(M), int(K), int(N), K) && rowquant_can_tile(int(N))) {
+    // one round of the split-K kernel's 128 x 160 tiles: it reads w8 [N, K] as
+    // it is stored (transposing LDS reads) and q in the MFMA block layout,
+    // written so by the quantizer.  (More than one round: the tiles below are
+    // faster, whole chain 73.3 -> 57.3 us at M=2263, N=5216, K=2560, 288 tiles, 59.5
+    // -> 51.6 at 3522 x 3584 x 2048, 364 tiles; at 252 tiles, 1527 x 4672 x 3328,
+    // 43.7 against 48.1 there, at 128, 984 x 5136 x 2560, 40.6 against 43.1.)
+    const bool one_round = ((M + 127) / 128) * ((K + 159) / 160) <= device_cus();
+    if (one_round && splitk_nn_applies(int(M), int(K), int(N), K) && rowquant_can_tile(int(N))) {
         XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N), true),
                          "linear_dx_int8 (quantize_row)"));
         XPU_TRY(launched(gemm_dequant_nn_xt(st, q, wnn ? wnn : w8, K, pre, K, a, int(M), int(K),
@@ -191,6 +195,26 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
                          "linear_dx_int8 (gemm)"));
         return launched(rotate_bf16(st, pre, dx, M, int(K)), "linear_dx_int8 (rotate)");
     }
+    // otherwise w8^T is written in the MFMA block layout, as a packed weight: the
+    // forward's kernels and tiles, at every size (the transpose moves the same
+    // bytes as a row-major one).  Against row-major operands, whole chain, us
+    // (M, N, K): 547 x 7632 x 1536 82.2 -> 32.1, 2002 x 5552 x 4608 124.4 -> 76.1,
+    // 586 x 1504 x 768 30.1 -> 15.5, 4096 x 1280 x 5120 59.0 -> 56.1, 10 x 5328 x 3840
+    // 23.0 -> 23.2; over 50 products 1.4 times as fast.  Its rows are padded to whole 64-byte steps, up to
+    // 48 K bytes more than N * K, so it may run on into the product's region:
+    // the product goes to dx, where the rotation takes each 256-column group
+    // through registers in place.
+    if (rowquant_can_tile(int(N)) && tiled_bytes(K, N) <= int64_t(L.part - L.wt)) {
+        XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N), true),
+                         "linear_dx_int8 (quantize_row)"));
+        XPU_TRY(launched(transpose_i8(st, w8, wt, N, K, true), "linear_dx_int8 (transpose)"));
+        XPU_TRY(launched(gemm_dequant_packed(st, q, wt, dx, K, a, nullptr, nullptr, nullptr, int(M),
+                                             int(K), int(N)),
+                         "linear_dx_int8 (gemm)"));
+        return launched(rotate_bf16(st, dx, dx, M, int(K)), "linear_dx_int8 (rotate)");
+    }
+    // rows of dy that the quantizer cannot write so (N > 32768), or a few rows with
+    // N % 64 != 0: row-major operands.
     // too few output tiles for the chip: the contraction split across blocks,
     // the slices' int32 partial sums added by the dequant pass (unit column
     // scale, row scale a)

@@ -2422,6 +2422,10 @@ __global__ __launch_bounds__(T) void dequant_kernel(const int32_t* __restrict__ 
 //    4*(t/8) .. +3: sixteen dword reads, a 4 x 4 byte register transpose per
 //    four rows, and four 16-byte stores, 8 lanes per 128-byte output segment.
 // Tiles past R or C are masked per 16-byte chunk.
+// TILED: out is the transposed matrix in the MFMA block layout (tiled_offset of
+// row c, byte r), the bytes past R in its last blocks zero, so that the product
+// with it takes the packed weight's kernels; a lane's four rows then leave as
+// 64-byte row pieces of 1 KB blocks.  The same bytes moved either way.
 __device__ __forceinline__ void transpose4x4(const uint32_t (&w)[4], uint32_t (&o)[4]) {
     // w[i] = bytes (row i, columns 0..3); o[j] = bytes (column j, rows 0..3)
     const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);
@@ -2434,6 +2438,7 @@ __device__ __forceinline__ void transpose4x4(const uint32_t (&w)[4], uint32_t (&
     o[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
 }
 
+template <bool TILED>
 __global__ __launch_bounds__(256) void transpose_i8_kernel(const int8_t* __restrict__ in,
                                                           int8_t* __restrict__ out, int64_t R,
                                                           int64_t C) {
@@ -2470,9 +2475,14 @@ __global__ __launch_bounds__(256) void transpose_i8_kernel(const int8_t* __restr
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int64_t c = c0 + 4 * cg + j;
-        if (c < C && r < R)
-            *reinterpret_cast<uint4*>(out + c * R + r) =
-                make_uint4(col[j][0], col[j][1], col[j][2], col[j][3]);
+        const uint4 v = make_uint4(col[j][0], col[j][1], col[j][2], col[j][3]);
+        if constexpr (TILED) {
+            const int KB = int((R + 63) / 64);
+            if (c < C && r < int64_t(KB) * 64)          // (rows past R read as zeros)
+                *reinterpret_cast<uint4*>(out + tiled_offset(c, int(r), KB)) = v;
+        } else {
+            if (c < C && r < R) *reinterpret_cast<uint4*>(out + c * R + r) = v;
+        }
     }
 }
 
@@ -2762,9 +2772,11 @@ hipError_t dequant_slices(hipStream_t st, const int32_t* acc, int64_t acc_ld, in
     return hipGetLastError();
 }
 
-hipError_t transpose_i8(hipStream_t st, const int8_t* in, int8_t* out, int64_t R, int64_t C) {
+hipError_t transpose_i8(hipStream_t st, const int8_t* in, int8_t* out, int64_t R, int64_t C,
+                        bool tiled) {
     const dim3 grid(unsigned((C + 127) / 128), unsigned((R + 127) / 128));
-    hipLaunchKernelGGL(transpose_i8_kernel, grid, dim3(256), 0, st, in, out, R, C);
+    if (tiled) hipLaunchKernelGGL(transpose_i8_kernel<true>, grid, dim3(256), 0, st, in, out, R, C);
+    else hipLaunchKernelGGL(transpose_i8_kernel<false>, grid, dim3(256), 0, st, in, out, R, C);
     return hipGetLastError();
 }
 

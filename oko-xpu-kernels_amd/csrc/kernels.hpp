@@ -150,7 +150,10 @@ hipError_t gemm_i32_slices(hipStream_t st, const int8_t* X, int64_t ldx, const i
 hipError_t gemm_i32_slices_nn(hipStream_t st, const int8_t* X, int64_t ldx, const int8_t* Bkn,
                               int64_t ldb, int32_t* part, int M, int N, int K, int nsl);
 bool slices_need_nt(int M);
-hipError_t transpose_i8(hipStream_t st, const int8_t* in, int8_t* out, int64_t R, int64_t C);
+// out = in [R, C] transposed (R, C multiples of 16), row-major or (tiled) in the
+// MFMA block layout, the bytes past R zero (tiled_bytes(C, R) bytes)
+hipError_t transpose_i8(hipStream_t st, const int8_t* in, int8_t* out, int64_t R, int64_t C,
+                        bool tiled = false);
 
 // gemm_bf16.hip: dw[n, k] = sum_m dy[m, n] * x[m, k] and out[m, k] = sum_n
 // dy[m, n] * w[n, k] (bf16, fp32 accumulate).  part (optional): part_bytes of

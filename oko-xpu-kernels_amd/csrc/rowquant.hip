@@ -809,10 +809,12 @@ hipError_t launch_rowquant(hipStream_t st, const Loader& ld, int8_t* q, float* s
 // ------------------------------------------------------------ rotate only
 // Every 256-group is independent, so the tensor is a flat list of M*K/256
 // groups (K % 256 == 0); a 16-lane segment rotates one group at a time, a
-// block's 16 segments take 16 consecutive groups per grid-stride step.
+// block's 16 segments take 16 consecutive groups per grid-stride step.  out may
+// be the loader's own bf16 input: a group's values are all in registers (and
+// exchanged between the segment's lanes) before any of them is stored.
 template <class Loader>
-__global__ __launch_bounds__(256) void rotate_kernel(Loader load, uint16_t* __restrict__ out,
-                                                     int64_t M, int K) {
+__global__ __launch_bounds__(256) void rotate_kernel(Loader load, uint16_t* out, int64_t M,
+                                                     int K) {
     const int sl = threadIdx.x & 15;
     const XlaneSigns sgn = xlane_signs(sl);
     const int w_out = lane_w_rot(sl);

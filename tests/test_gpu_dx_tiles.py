@@ -1,0 +1,45 @@
+"""linear_dx_int8's kernels by shape: one round of the split-K kernel on the weight
+as stored, else the transposed weight in the block layout with the packed
+products' tiles (a contraction that ends inside a 64-byte step, whose padded
+copy runs into the product's region; one and two row blocks; a batch just large
+enough for that region), else, for a few rows of such a contraction or rows of
+dy too long to be quantized into the layout, row-major operands.  Bit for bit
+the oracle's, twice in a row through one workspace that the first call left full."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from gpu_util import bits, mismatch, npy, weight
+from xpu_kernels import int8
+from xpu_kernels.int8 import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+# (M, N, K)
+SHAPES = [(2060, 2064, 1280), (2180, 1104, 2560),                # split K; 16 * 16 + 16 tiles more
+          (33, 528, 256), (65, 1040, 512), (130, 48, 256), (300, 2608, 768), (1273, 528, 512),
+          (24, 16, 256), (23, 16, 256), (1, 16, 512), (7, 1296, 256), (16, 64, 256),
+          (3, 32784, 256), (70, 33024, 256)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_dx_int8_by_shape_exact(dev, m, n, k):
+    lib = L._lib()
+    w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
+    g = torch.Generator().manual_seed(m + n)
+    need = lib.xpuint8_linear_dx_int8_workspace_size(m, n, k)
+    work = torch.full((need,), 0x55, device=dev, dtype=torch.uint8)
+    guard = torch.full((m * k + 4096,), 7.0, device=dev, dtype=torch.bfloat16)
+    for _ in range(2):
+        dy = (torch.randn(m, n, generator=g) * 1e-3).to(torch.bfloat16)
+        dx = dy.to(dev)
+        rc = lib.xpuint8_linear_dx_int8_stream(L._stream(dev), L._ptr(dx), L._ptr(ws), L._ptr(w8),
+                                               L._ptr(guard), m, n, k, L._ptr(work), need)
+        assert rc == 0, lib.xpuint8_last_error()
+        got = bits(guard[: m * k].view(m, k))
+        want = O.linear_dx_int8(bits(dy), npy(w8), npy(ws))
+        assert np.array_equal(got, want), mismatch(got, want)
+        assert bool((guard[m * k:] == 7.0).all())
