@@ -2051,9 +2051,9 @@ struct WavekModel {
     double c0, load, step, red, byte;
 };
 inline double wavek_time(const WavekModel& w, const WavekTile& t, int64_t M, int64_t N, int K,
-                         int64_t out_cols) {
+                         int64_t out_cols, int64_t cus) {
     const int64_t blocks = ((M + 16 * t.mb - 1) / (16 * t.mb)) * ((N + 16 * t.nb - 1) / (16 * t.nb));
-    const int64_t cus = device_cus(), per = (blocks + cus - 1) / cus;
+    const int64_t per = (blocks + cus - 1) / cus;
     const int64_t rounds = (blocks + cus * t.per_cu - 1) / (cus * t.per_cu);
     const int KB = (K + 63) / 64, chain = (KB + t.nw * t.d - 1) / (t.nw * t.d);
     const double bytes = double(M) * K + double(N) * K + 2.0 * double(M) * double(out_cols);
@@ -2064,10 +2064,11 @@ inline double wavek_time(const WavekModel& w, const WavekTile& t, int64_t M, int
 // The tile with the least predicted time below `time` (updated), -1 for none
 template <int NT>
 inline int wavek_tile(const WavekModel& w, const WavekTile (&tiles)[NT], double bias, int64_t M,
-                      int64_t N, int K, int64_t out_cols, double* time) {
+                      int64_t N, int K, int64_t out_cols, int64_t cus, double* time) {
     int best = -1;
+#pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const double t = bias * wavek_time(w, tiles[i], M, N, K, out_cols);
+        const double t = bias * wavek_time(w, tiles[i], M, N, K, out_cols, cus);
         if (t < *time) best = i, *time = t;
     }
     return best;
@@ -2148,9 +2149,11 @@ struct PpTile {
 struct PpModel {
     double c0, mm, st, fs, ep, fe;
 };
-// n_tiles: tiles across the output columns
-inline double pp_time(const PpModel& p, int bm, int bn, int64_t M, int64_t n_tiles, int K) {
-    const int64_t tiles = ((M + bm - 1) / bm) * n_tiles, cus = device_cus();
+// n_tiles: tiles across the output columns; cus: device_cus(), which asks the
+// runtime for the current device, once per product (once per tile cost 1.3 us a call)
+inline double pp_time(const PpModel& p, int bm, int bn, int64_t M, int64_t n_tiles, int K,
+                      int64_t cus) {
+    const int64_t tiles = ((M + bm - 1) / bm) * n_tiles;
     const int64_t rounds = ((tiles + 7) / 8 + cus / 8 - 1) / (cus / 8);
     const double area = 1e-4 * bm * bn, fill = double(tiles) / double(cus * rounds);
     const double steps = (K + 63) / 64;
@@ -2159,11 +2162,12 @@ inline double pp_time(const PpModel& p, int bm, int bn, int64_t M, int64_t n_til
 }
 template <int NT>
 inline int pp_tile(const PpModel& p, const PpTile (&tiles)[NT], bool paired, int64_t M, int64_t N,
-                   int K, double* time) {
+                   int K, int64_t cus, double* time) {
     int best = 0;
+#pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int cols = paired ? tiles[i].bn / 2 : tiles[i].bn;
-        const double c = pp_time(p, tiles[i].bm, tiles[i].bn, M, (N + cols - 1) / cols, K);
+        const double c = pp_time(p, tiles[i].bm, tiles[i].bn, M, (N + cols - 1) / cols, K, cus);
         if (i == 0 || c < *time) best = i, *time = c;
     }
     return best;
@@ -2196,8 +2200,8 @@ constexpr WavekTile kWavekTiles[] = {
     {1, 1, 8, 4, 2}, {1, 2, 4, 4, 6}, {2, 2, 4, 4, 4}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
 constexpr WavekModel kWavekModel = {2.25, 0.0068, 0.2, 0.277 / 16, 0.082e-6};
 
-inline double splitk_time(int64_t M, int64_t N, int64_t K) {
-    const int64_t tiles = ((M + 127) / 128) * ((N + 159) / 160), cus = device_cus();
+inline double splitk_time(int64_t M, int64_t N, int64_t K, int64_t cus) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 159) / 160);
     const int64_t rounds = (tiles + cus - 1) / cus;
     const double fill = double(tiles) / double(cus * rounds), steps = (K + 63) / 64;
     return 2.9 + double(rounds) * (steps * 0.287 * (0.82 + 0.18 * fill) +
@@ -2215,14 +2219,15 @@ template <class Epi>
 hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N, int K,
                         const Epi& epi) {
     constexpr bool kSplitK = Epi::kStaged && !IsActEpi<Epi>::value;
+    const int64_t cus = device_cus();
     double t = 0;
-    const int tile = pp_tile(kPpModel, kPpTiles, false, M, N, K, &t);
+    const int tile = pp_tile(kPpModel, kPpTiles, false, M, N, K, cus, &t);
     bool splitk = false;
     if constexpr (kSplitK) {
-        const double ts = 1.03 * splitk_time(M, N, K);
+        const double ts = 1.03 * splitk_time(M, N, K, cus);
         if (ts < t) splitk = true, t = ts;
     }
-    switch (wavek_tile(kWavekModel, kWavekTiles, 1.06, M, N, K, N, &t)) {
+    switch (wavek_tile(kWavekModel, kWavekTiles, 1.06, M, N, K, N, cus, &t)) {
         case 0: return launch_wavek<1, 1, 8, 4>(st, Xt, Wp, M, N, K, epi);
         case 1: return launch_wavek<1, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
         case 2: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
@@ -2264,9 +2269,10 @@ hipError_t launch_pair_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp,
     if (M <= 16) return launch_skinny<4, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
     const PpModel pm = {4.05, 0.0771, 0.1875, 0.76, situ ? 1.76 : 0.85, 0.77};
     const WavekModel wm = {1.88, 0.0058, 0.42, (situ ? 0.32 : 0.236) / 16, 0.084e-6};
+    const int64_t cus = device_cus();
     double t = 0;
-    const int tile = pp_tile(pm, kPairTiles, true, M, N, K, &t);
-    switch (wavek_tile(wm, kPairWavekTiles, 1.03, M, 2 * int64_t(N), K, N, &t)) {
+    const int tile = pp_tile(pm, kPairTiles, true, M, N, K, cus, &t);
+    switch (wavek_tile(wm, kPairWavekTiles, 1.03, M, 2 * int64_t(N), K, N, cus, &t)) {
         case 0: return launch_wavek<1, 2, 8, 4>(st, Xt, Wp, M, N, K, epi);
         case 1: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
         case 2: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);

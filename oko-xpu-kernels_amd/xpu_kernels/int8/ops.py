@@ -814,7 +814,8 @@ def linear(x, w8, w_scale, bias=None, act: Optional[str] = None, residual=None,
     ``residual``/``residual_scale`` apply ``residual + residual_scale * out``;
     ``return_acc`` returns ``(int32 [M, N], fp32 [M], fp32 [N])`` instead.
     """
-    if act is None and residual is None and not return_acc and _L.HOST is not None:
+    if (act is None and residual is None and not return_acc and _L.HOST is not None
+            and getattr(x, "dtype", None) is torch.bfloat16):
         y = _L.HOST.linear(x, w8, w_scale, bias)
         if y is not None:
             return y
