@@ -266,6 +266,15 @@ size_t linear_work_bytes(int64_t M, int64_t N, int64_t K) {
     return linear_work_q_bytes(M, K) + 4 * size_t(M);
 }
 
+// Whether a product with a packed weight quantizes x in its own launch: few enough
+// values of x, and nothing of it where the product writes (the blocks read x
+// while others already store; two launches allow it)
+bool rowq_takes(const void* x, int64_t M, int64_t K, const void* out, int64_t out_bytes) {
+    if (M > 16 || !rowq_applies(int(M), int(K))) return false;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(out);
+    return a + uintptr_t(2 * M * K) <= b || b + uintptr_t(out_bytes) <= a;
+}
+
 // quantize + GEMM + dequant of xpuint8_linear_stream on checked arguments.
 // wp (optional): pack_weight's copy of w8, read instead of w8.
 int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_scale,
@@ -275,6 +284,10 @@ int linear_run(hipStream_t st, const void* x, const int8_t* w8, const float* w_s
     float* xs = reinterpret_cast<float*>(static_cast<char*>(work) + linear_work_q_bytes(M, K));
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
+    if (wp && rowq_takes(x, M, K, out, 2 * M * N))
+        return launched(gemm_dequant_rowq(st, x, wp, out, N, w_scale, b32, b16, int(M), int(N),
+                                          int(K)),
+                        "linear (quantize and gemm)");
     // the packed weight: q in the MFMA block layout too, for every shape
     if (wp && rowquant_can_tile(int(K))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)), "linear (quantize)"));
@@ -344,7 +357,11 @@ int ffn_run(hipStream_t st, const void* x, const int8_t* up_w8, const int8_t* up
     float* xs = reinterpret_cast<float*>(region + linear_work_q_bytes(M, K));
     // xq in the MFMA block layout: with the packed weight, and for the persistent
     // up-projection from a row-major one
-    if (rowquant_can_tile(int(K)) &&
+    if (up_wp && rowq_takes(x, M, K, v, 2 * M * inner)) {
+        XPU_TRY(launched(gemm_act_rowq(st, x, up_wp, v, inner, up_scale, int(M), int(inner), int(K),
+                                       activation),
+                         "ffn (quantize and up projection)"));
+    } else if (rowquant_can_tile(int(K)) &&
         (up_wp || pp_applies(int(M), int(inner), int(K), act_paired(activation)))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, xq, xs, M, int(K)), "ffn (quantize)"));
         XPU_TRY(launched(up_wp ? gemm_act_packed(st, xq, up_wp, v, inner, xs, up_scale, int(M),
@@ -681,6 +698,11 @@ int xpuint8_linear_residual_packed_stream(const void* stream, const void* x, con
     float* xs = reinterpret_cast<float*>(static_cast<char*>(work) + linear_work_q_bytes(M, K));
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
+    if (w8_packed && rowq_takes(x, M, K, out, 2 * M * N))
+        return launched(gemm_dequant_residual_rowq(st, x, w8_packed, out, N, w_scale, b32, b16,
+                                                   residual, N, residual_scale, int(M), int(N),
+                                                   int(K)),
+                        "linear_residual (quantize and gemm)");
     // the kernels that read x in the MFMA block layout
     if (rowquant_can_tile(int(K)) && (w8_packed || xt_applies(int(M), int(N), int(K)))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, xs, M, int(K)),
@@ -714,6 +736,9 @@ int xpuint8_linear_acc_packed_stream(const void* stream, const void* x, const in
     XPU_TRY(ensure_device());
     hipStream_t st = as_stream(stream);
     int8_t* q = static_cast<int8_t*>(work);
+    if (w8_packed && rowq_takes(x, M, K, acc, 4 * M * N) && rowq_takes(x, M, K, x_scale, 4 * M))
+        return launched(gemm_i32_rowq(st, x, w8_packed, acc, N, x_scale, int(M), int(N), int(K)),
+                        "linear_acc (quantize and gemm)");
     if (rowquant_can_tile(int(K)) && (w8_packed || pp_applies(int(M), int(N), int(K), false))) {
         XPU_TRY(launched(convrot_quantize_tiled(st, x, q, x_scale, M, int(K)),
                          "linear_acc (quantize)"));

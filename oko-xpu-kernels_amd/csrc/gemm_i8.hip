@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "activations.hpp"
+#include "quantizer.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -1881,6 +1882,180 @@ hipError_t launch_skinny(hipStream_t st, const int8_t* X, int64_t ldx, const int
     return hipGetLastError();
 }
 
+// ------------------------------------------------------ few rows, one launch
+// At most 16 rows, quantized by the product's own blocks: each block rotates and
+// quantizes all of x (a 16-lane segment takes P of the M * K/256 groups, with the row
+// kernels' arithmetic, so their codes and scales) into LDS while its first
+// weight steps are on their way to registers, then runs the skinny kernel's loop
+// on it.  Bound by latency: a separate quantizer is a launch, a load, a store and
+// the wait for it before the weight is asked for; repeating it in every block
+// costs M * K bf16 from L2 per block and arithmetic that the weight's latency
+// covers in part.
+// W: the packed weight.  x's codes lie in LDS by 64-byte step, row and swizzled
+// chunk; lanes of rows past M read row M - 1 (never stored).
+template <class E, class = void>
+struct HasRowScale : std::false_type {};
+template <class E>
+struct HasRowScale<E, std::void_t<decltype(E::xs)>> : std::true_type {};
+
+template <int NW, int P, int NB, class Epi>
+__global__ __launch_bounds__(NW * 64) void gemm_i8_rowq_kernel(const uint16_t* __restrict__ x,
+                                                               const int8_t* __restrict__ W,
+                                                               float* __restrict__ xs_out, int M,
+                                                               int N, int K, Epi epi) {
+    constexpr bool PAIRED = Epi::kPaired;
+    constexpr int NC = PAIRED ? NB / 2 : NB, D = NW >= 16 ? 4 / NB : 8 / NB;
+    static_assert(D >= 1 && (!PAIRED || NB % 2 == 0), "steps in flight; both halves");
+    __shared__ __attribute__((aligned(16))) int8_t qx[NW * P * 1024];
+    __shared__ v4i part[NW][NB][64];
+    __shared__ uint32_t row_max[16];
+    __shared__ float row_sc[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n0 = blockIdx.x * 16 * NC;
+
+    // x first: the waits for it leave the weight's loads in flight
+    const int sl = threadIdx.x & 15, G = K / kGroup, T = M * G;
+    int row[P], col[P];
+    u32x4 ra[P], rb[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int t = min(int(threadIdx.x >> 4) + 4 * NW * p, T - 1);
+        row[p] = int(unsigned(t) / unsigned(G));
+        col[p] = (t - row[p] * G) * kGroup;
+        const uint16_t* xp = x + row[p] * K + col[p] + 16 * lane_w(sl);
+        ra[p] = load16(xp);
+        rb[p] = load16(xp + 8);
+    }
+    const int8_t* wrow[NB];
+    const int chunk = (((lane >> 4) ^ (lane >> 1)) & 3) << 4;     // of row lane % 16
+#pragma unroll
+    for (int p = 0; p < NB; ++p) {
+        const int nb = min(n0 / 16 + (p % NC), (N - 1) / 16) + (p >= NC ? pair_offset(epi) / 16 : 0);
+        wrow[p] = W + int64_t(nb) * (K / 64) * 1024 + (lane & 15) * 64 + chunk;
+    }
+    const int S = K / 64;
+    v4i wbuf[D][NB];
+    auto load = [&](int slot, int step) {
+        if (step >= S) return;
+#pragma unroll
+        for (int p = 0; p < NB; ++p)
+            wbuf[slot][p] = *reinterpret_cast<const v4i*>(wrow[p] + int64_t(step) * 1024);
+    };
+#pragma unroll
+    for (int j = 0; j < D; ++j) load(j, wave + NW * j);
+
+    // quantize
+    if (threadIdx.x < 16) row_max[threadIdx.x] = 0u;
+    lds_barrier();
+    float v[P][16];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const uint32_t w[8] = {ra[p].x, ra[p].y, ra[p].z, ra[p].w,
+                               rb[p].x, rb[p].y, rb[p].z, rb[p].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[p][2 * j] = bf16lo(w[j]), v[p][2 * j + 1] = bf16hi(w[j]);
+    }
+    const float dom = rotate_groups<P>(v, xlane_signs(sl));
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        // (the segments past T repeat the last group: the same maximum)
+        const uint32_t mb = segment_max_bits(__float_as_uint(absmax16(v[p], 0.f) * dom));
+        if (sl == 0) atomicMax(&row_max[row[p]], mb);
+    }
+    lds_barrier();
+    const int kst = 16 * lane_w_rot(sl);          // the register a lane holds now
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const float sc = row_scale(kRecip, __uint_as_float(row_max[row[p]]));
+        const uint4 q = quant16<true, kRecip>(v[p], sc, rcp_rn(sc), dom);
+        const int k = col[p] + kst, r = row[p];
+        *reinterpret_cast<uint4*>(qx + (k >> 6) * (M * 64) + r * 64 +
+                                  ((((k >> 4) ^ (r >> 1)) & 3) << 4)) = q;
+    }
+    if (threadIdx.x < M) {
+        const float sc = row_scale(kRecip, __uint_as_float(row_max[threadIdx.x]));
+        row_sc[threadIdx.x] = sc;
+        if (xs_out && blockIdx.x == 0) xs_out[threadIdx.x] = sc;
+    }
+    if constexpr (HasRowScale<Epi>::value) epi.xs = row_sc;
+    lds_barrier();
+
+    // the product: wave w takes steps w, w + NW, ...
+    const int xr = min(lane & 15, M - 1);
+    const int8_t* const xq = qx + xr * 64 + ((((lane >> 4) ^ (xr >> 1)) & 3) << 4);
+    v4i acc[NB];
+#pragma unroll
+    for (int p = 0; p < NB; ++p) acc[p] = v4i{0, 0, 0, 0};
+    for (int s0 = wave; s0 < S; s0 += NW * D) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            const int step = s0 + NW * j;
+            if (step < S) {
+                const v4i xf = *reinterpret_cast<const v4i*>(xq + step * (M * 64));
+#pragma unroll
+                for (int p = 0; p < NB; ++p)
+                    acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wbuf[j][p], xf, acc[p], 0, 0, 0);
+            }
+            load(j, step + NW * D);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < NB; ++p) part[wave][p][lane] = acc[p];
+    __syncthreads();
+    // lane l holds rows 4*(l/16)+i of a weight block (n) for x row l%16 (m)
+    if (wave >= NC) return;
+    v4i a = part[0][wave][lane], b = v4i{0, 0, 0, 0};
+    if constexpr (PAIRED) b = part[0][NC + wave][lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+        a += part[w][wave][lane];
+        if constexpr (PAIRED) b += part[w][NC + wave][lane];
+    }
+    const int m = lane & 15, n = n0 + 16 * wave + 4 * (lane >> 4);
+    if (m < M && n < N) {
+        if constexpr (PAIRED) epi.pair(m, n, a, b);
+        else epi(m, n, a);
+    }
+}
+
+// By the number of 256-column groups of x, one 16-lane segment each: 4, 8 or 16
+// waves up to 16, 32 and 64 of them (above 512 column blocks of 16, and for pairs, 8
+// waves of two groups: 16-wave blocks hold x's redundant work to two blocks a
+// CU, 12.2 against 14.4 us at 4 x 10240 x 4096 with two weight blocks), and two
+// weight blocks a block where one would give more than 512.  Above 64 groups the
+// separate quantizer stays: 6.6 us for both launches at 16 x 1280 x 1280 (80
+// groups) against 6.5-6.8, 9.4 at 8 x 4096 x 4096 (128) against 9.4, 13.5 at 8 x
+// 10240 x 2560 (80) against 16.0.
+// Both launches before -> one, cold weights, us (M, N, K):
+//   1 x 1280 x 1280    5.76 -> 4.40      4 x 4096 x 4096    9.15 -> 8.01
+//   1 x 10240 x 4096   15.39 -> 10.18    16 x 4096 x 512    5.58 -> 4.58
+//   1 x 1280 x 8192    10.75 -> 7.61     2 x 10240 x 5120   18.79 -> 14.11
+constexpr int kRowqGroups = 64;
+template <class Epi>
+hipError_t launch_rowq(hipStream_t st, const void* x, const int8_t* Wp, float* xs_out, int M,
+                       int N, int K, const Epi& epi) {
+    constexpr int NB = Epi::kPaired ? 2 : 1;        // one output column block
+    const int T = M * (K / kGroup), blocks = (N + 15) / 16;
+    const bool wide = !Epi::kPaired && blocks > 2 * device_cus();
+    const uint16_t* xb = static_cast<const uint16_t*>(x);
+#define XPU_ROWQ(NW, P, NB)                                                                     \
+    hipLaunchKernelGGL((gemm_i8_rowq_kernel<NW, P, NB, Epi>),                                  \
+                       dim3(unsigned(Epi::kPaired ? blocks : (blocks + NB - 1) / NB)),         \
+                       dim3(NW * 64), 0, st, xb, Wp, xs_out, M, N, K, epi)
+    if (T <= 16) {
+        XPU_ROWQ(4, 1, NB);
+    } else if (T <= 32) {
+        if (wide) XPU_ROWQ(8, 1, 2);
+        else XPU_ROWQ(8, 1, NB);
+    } else if (Epi::kPaired || wide) {
+        XPU_ROWQ(8, 2, 2);
+    } else {
+        XPU_ROWQ(16, 1, NB);
+    }
+#undef XPU_ROWQ
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------ K split over waves
 // Products too small to fill the chip with LDS-staged tiles: a block of NW
 // waves owns a (16 MB) x (16 NB) tile and its waves take every NW-th 64-byte
@@ -2654,6 +2829,30 @@ hipError_t gemm_dequant_packed(hipStream_t st, const int8_t* At, const int8_t* B
                        EpiDequant{static_cast<uint16_t*>(out), ldo, xs, ws, bias, bias16});
 }
 
+// Whether the product quantizes its rows itself (launch_rowq)
+bool rowq_applies(int M, int K) {
+    return M <= 16 && K % kGroup == 0 && int64_t(M) * (K / kGroup) <= kRowqGroups;
+}
+
+hipError_t gemm_dequant_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out,
+                             int64_t ldo, const float* ws, const float* bias,
+                             const uint16_t* bias16, int M, int N, int K) {
+    return launch_rowq(st, x, Wp, nullptr, M, N, K,
+                          EpiDequant{static_cast<uint16_t*>(out), ldo, nullptr, ws, bias, bias16});
+}
+
+hipError_t gemm_act_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out, int64_t ldo,
+                         const float* ws, int M, int N, int K, int act) {
+    uint16_t* o = static_cast<uint16_t*>(out);
+    const uint16_t* tab = activation_tables();
+    switch (act) {
+        case 3: return launch_rowq(st, x, Wp, nullptr, M, N, K, EpiAct<3>{o, ldo, nullptr, ws, N, tab});
+        case 4: return launch_rowq(st, x, Wp, nullptr, M, N, K, EpiAct<4>{o, ldo, nullptr, ws, N, tab});
+        case 5: return launch_rowq(st, x, Wp, nullptr, M, N, K, EpiAct<5>{o, ldo, nullptr, ws, N, tab});
+        default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t gemm_act_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,
                           void* out, int64_t ldo, const float* xs, const float* ws, int M, int N,
                           int K, int act) {
@@ -2730,6 +2929,19 @@ hipError_t gemm_dequant_residual_packed(hipStream_t st, const int8_t* At, const 
                                         int64_t ldr, const void* rscale, int M, int N, int K) {
     return packed_gemm(st, At, Bp, M, N, K,
                        residual_epi(out, ldo, xs, ws, bias, bias16, res, ldr, rscale));
+}
+
+hipError_t gemm_dequant_residual_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out,
+                                      int64_t ldo, const float* ws, const float* bias,
+                                      const uint16_t* bias16, const void* res, int64_t ldr,
+                                      const void* rscale, int M, int N, int K) {
+    return launch_rowq(st, x, Wp, nullptr, M, N, K,
+                          residual_epi(out, ldo, nullptr, ws, bias, bias16, res, ldr, rscale));
+}
+
+hipError_t gemm_i32_rowq(hipStream_t st, const void* x, const int8_t* Wp, int32_t* C, int64_t ldc,
+                         float* xs, int M, int N, int K) {
+    return launch_rowq(st, x, Wp, xs, M, N, K, EpiI32{C, ldc});
 }
 
 hipError_t gemm_i32_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int64_t ldb,

@@ -127,6 +127,20 @@ hipError_t gemm_i32_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int
                           int32_t* C, int64_t ldc, int M, int N, int K);
 hipError_t gemm_i32_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, int32_t* C,
                            int64_t ldc, int M, int N, int K);
+// the same products of x itself, bf16 [M, K], quantized in the same launch (callers
+// check rowq_applies; out must not overlap x); xs: its row scales, written
+bool rowq_applies(int M, int K);
+hipError_t gemm_dequant_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out,
+                             int64_t ldo, const float* ws, const float* bias,
+                             const uint16_t* bias16, int M, int N, int K);
+hipError_t gemm_act_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out, int64_t ldo,
+                         const float* ws, int M, int N, int K, int act);
+hipError_t gemm_dequant_residual_rowq(hipStream_t st, const void* x, const int8_t* Wp, void* out,
+                                      int64_t ldo, const float* ws, const float* bias,
+                                      const uint16_t* bias16, const void* res, int64_t ldr,
+                                      const void* rscale, int M, int N, int K);
+hipError_t gemm_i32_rowq(hipStream_t st, const void* x, const int8_t* Wp, int32_t* C, int64_t ldc,
+                         float* xs, int M, int N, int K);
 // out[m, n] = act(bf16(acc(n) * ws[n] * xs[m]), bf16(acc(N + n) * ws[N + n] * xs[m])) for the
 // paired activations 3 (situ) and 4 (GEGLU), whose B has 2N rows; act 5 (GELU) takes N rows
 hipError_t gemm_act(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,
