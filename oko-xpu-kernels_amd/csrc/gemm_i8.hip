@@ -2270,8 +2270,8 @@ hipError_t launch_wavek(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int 
     return hipGetLastError();
 }
 
-// Tile choice: the 256 x 320 ping-pong tile when it gives at least one tile
-// per CU (8-12% faster than the two-block 256 x 160 kernel at M=4096, K=1280
+// Tile choice for a row-major weight (launch_gemm; packed ones: launch_tiles): the
+// 256 x 320 ping-pong tile when it gives at least one tile per CU (8-12% faster than the two-block 256 x 160 kernel at M=4096, K=1280
 // and 2560, N=5120 and 10240, interleaved A/B timing); else the large tile
 // (256 x 160, 4 waves of 128 x 80, two blocks per CU, two LDS stages) when it
 // gives at least 192 tiles; otherwise the small one (128 x 128, 4 waves of
