@@ -173,13 +173,23 @@ int check_dx(int64_t M, int64_t N, int64_t K) {
 // quantize_row (column-scaled) -> w8^T -> GEMM with the row-scale epilogue ->
 // inverse rotation, all on one stream, through the workspace at `work`.
 // wnn (optional): pack_weight_nn's copy of w8, read by the split-K GEMM.
+// dbias (optional): the column sums of dy too, through cpart (colsum_work_bytes).
 int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t* w8, void* dx,
-             int64_t M, int64_t N, int64_t K, char* work, const int8_t* wnn = nullptr) {
+             int64_t M, int64_t N, int64_t K, char* work, const int8_t* wnn = nullptr,
+             void* dbias = nullptr, float* cpart = nullptr, bool dbias_fp32 = false) {
     const DxWork L = dx_work_layout(M, N, K);
     int8_t* q = reinterpret_cast<int8_t*>(work + L.q);
     float* a = reinterpret_cast<float*>(work + L.a);
     int8_t* wt = reinterpret_cast<int8_t*>(work + L.wt);
     void* pre = work + L.pre;
+    auto quantize = [&](bool tiled) {
+        if (!dbias) return quantize_row(st, dy, w_scale, q, a, M, int(N), tiled);
+        if (quantize_row_sums(M, int(N)))
+            return quantize_row_colsum(st, dy, w_scale, q, a, M, int(N), tiled, dbias, cpart,
+                                       dbias_fp32);
+        const hipError_t e = column_sum_bf16(st, dy, dbias, M, int(N), cpart, dbias_fp32);
+        return e != hipSuccess ? e : quantize_row(st, dy, w_scale, q, a, M, int(N), tiled);
+    };
     // one round of the split-K kernel's 128 x 160 tiles: it reads w8 [N, K] as
     // it is stored (transposing LDS reads) and q in the MFMA block layout,
     // written so by the quantizer.  (More than one round: the tiles below are
@@ -188,7 +198,7 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
     // 43.7 against 48.1 there, at 128, 984 x 5136 x 2560, 40.6 against 43.1.)
     const bool one_round = ((M + 127) / 128) * ((K + 159) / 160) <= device_cus();
     if (one_round && splitk_nn_applies(int(M), int(K), int(N), K) && rowquant_can_tile(int(N))) {
-        XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N), true),
+        XPU_TRY(launched(quantize(true),
                          "linear_dx_int8 (quantize_row)"));
         XPU_TRY(launched(gemm_dequant_nn_xt(st, q, wnn ? wnn : w8, K, pre, K, a, int(M), int(K),
                                             int(N), wnn != nullptr),
@@ -205,7 +215,7 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
     // the product goes to dx, where the rotation takes each 256-column group
     // through registers in place.
     if (rowquant_can_tile(int(N)) && tiled_bytes(K, N) <= int64_t(L.part - L.wt)) {
-        XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N), true),
+        XPU_TRY(launched(quantize(true),
                          "linear_dx_int8 (quantize_row)"));
         XPU_TRY(launched(transpose_i8(st, w8, wt, N, K, true), "linear_dx_int8 (transpose)"));
         XPU_TRY(launched(gemm_dequant_packed(st, q, wt, dx, K, a, nullptr, nullptr, nullptr, int(M),
@@ -220,7 +230,7 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
     // scale, row scale a)
     if (const int nsl = gemm_slices(int(M), int(K), int(N))) {
         int32_t* part = reinterpret_cast<int32_t*>(work + L.part);
-        XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N)),
+        XPU_TRY(launched(quantize(false),
                          "linear_dx_int8 (quantize_row)"));
         if (slices_need_nt(int(M))) {
             XPU_TRY(launched(transpose_i8(st, w8, wt, N, K), "linear_dx_int8 (transpose)"));
@@ -236,7 +246,7 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
                          "linear_dx_int8 (dequant)"));
         return launched(rotate_bf16(st, pre, dx, M, int(K)), "linear_dx_int8 (rotate)");
     }
-    XPU_TRY(launched(quantize_row(st, dy, w_scale, q, a, M, int(N)), "linear_dx_int8 (quantize_row)"));
+    XPU_TRY(launched(quantize(false), "linear_dx_int8 (quantize_row)"));
     bool nn = false;
     XPU_TRY(launched(gemm_dequant_nn(st, q, N, w8, K, pre, K, a, int(M), int(K), int(N), &nn),
                      "linear_dx_int8 (gemm)"));
@@ -937,11 +947,8 @@ int xpuint8_linear_backward_int8_stream(const void* stream, const void* dy, cons
     XPU_TRY(ensure_device());
     hipStream_t st = as_stream(stream);
     char* w = static_cast<char*>(work);
-    if (dbias)
-        XPU_TRY(launched(column_sum_bf16(st, dy, dbias, M, int(N), reinterpret_cast<float*>(w + dxw),
-                                         dbias_fp32 != 0),
-                         "linear_backward_int8 (column sum)"));
-    return dx_chain(st, dy, w_scale, w8, dx, M, N, K, w, w8_packed_nn);
+    return dx_chain(st, dy, w_scale, w8, dx, M, N, K, w, w8_packed_nn, dbias,
+                    reinterpret_cast<float*>(w + dxw), dbias_fp32 != 0);
 }
 
 int xpuint8_linear_dx_int8_noalloc_stream(const void* stream, const void* dy,

@@ -50,6 +50,12 @@ hipError_t convrot_quantize_tiled(hipStream_t st, const void* x, int8_t* q, floa
 int64_t colsum_work_bytes(int64_t M, int64_t N);
 hipError_t column_sum_bf16(hipStream_t st, const void* x, void* out, int64_t M, int N,
                            float* part, bool out_f32 = false);
+// quantize_row with a column scale and column_sum_bf16 of the same x, reading it in
+// one launch (callers check quantize_row_sums)
+bool quantize_row_sums(int64_t M, int N);
+hipError_t quantize_row_colsum(hipStream_t st, const void* x, const float* colscale, int8_t* q,
+                               float* scale, int64_t M, int N, bool tiled, void* out, float* part,
+                               bool out_f32);
 
 // gemm_i8.hip
 hipError_t gemm_i32(hipStream_t st, const int8_t* A, int64_t lda, const int8_t* B, int64_t ldb,
