@@ -146,12 +146,16 @@ PyObject* packed_entry(const Tensor& w) {
         return nullptr;
     return e;
 }
-// entry e's packed copy (which = 3) or second form (4); null for none
-const int8_t* packed_ptr(PyObject* e, int which) {
-    if (!e) return nullptr;
+// entry e's packed copy (which = 3) or second form (4), undefined for none.  The
+// caller holds it until its kernels are enqueued: another thread may pack the
+// weight anew, or free it, as soon as the library call lets go of the GIL.
+Tensor packed_form(PyObject* e, int which) {
+    if (!e) return Tensor();
     PyObject* p = PyList_GET_ITEM(e, which);
-    if (p == Py_None) return nullptr;
-    return static_cast<const int8_t*>(THPVariable_Unpack(p).data_ptr());
+    return p == Py_None ? Tensor() : THPVariable_Unpack(p);
+}
+const int8_t* codes(const Tensor& t) {
+    return t.defined() ? static_cast<const int8_t*>(t.data_ptr()) : nullptr;
 }
 
 // ------------------------------------------------------------ the call
@@ -242,7 +246,8 @@ PyObject* host_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const int64_t need = g_lib.linear_size(m, n, k);
         if (need < 0) fail("linear");
         const Tensor work = workspace(need, *x), out = empty(with_last(*x, n), at::kBFloat16, *x);
-        const int8_t* p = packed_ptr(packed_entry(*w), 3);
+        const Tensor packed = packed_form(packed_entry(*w), 3);
+        const int8_t* p = codes(packed);
         const void* st = current_stream(*x);
         call("linear", [&] {
             return g_lib.linear(st, x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), p,
@@ -266,7 +271,8 @@ PyObject* host_linear_acc(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (need < 0) fail("linear_acc");
         const Tensor work = workspace(need, *x), acc = empty({m, n}, at::kInt, *x),
                      xs = empty({m}, at::kFloat, *x);
-        const int8_t* p = packed_ptr(packed_entry(*w), 3);
+        const Tensor packed = packed_form(packed_entry(*w), 3);
+        const int8_t* p = codes(packed);
         const void* st = current_stream(*x);
         call("linear_acc", [&] {
             return g_lib.linear_acc(st, x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), p,
@@ -300,8 +306,9 @@ PyObject* host_ffn(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const int64_t need = g_lib.ffn_size(m, inner, k, int32_t(act));
         if (need < 0) fail("ffn");
         const Tensor work = workspace(need, *x), out = empty(x->sizes(), at::kBFloat16, *x);
-        const int8_t *up_p = packed_ptr(packed_entry(*up), 3),
-                     *down_p = packed_ptr(packed_entry(*down), 3);
+        const Tensor up_packed = packed_form(packed_entry(*up), 3),
+                     down_packed = packed_form(packed_entry(*down), 3);
+        const int8_t *up_p = codes(up_packed), *down_p = codes(down_packed);
         const void* st = current_stream(*x);
         call("ffn", [&] {
             return g_lib.ffn(st, x->data_ptr(), static_cast<const int8_t*>(up->data_ptr()), up_p,
@@ -331,12 +338,13 @@ PyObject* host_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
                   dense = PyObject_IsTrue(a[5]);
         if (want < 0 || f32 < 0 || dense < 0) throw python_error();
         const char* what = dense ? "linear_dx" : "linear_dx_int8";
-        const int8_t* nn = nullptr;
+        Tensor packed_nn;
         if (!dense) {
             PyObject* e = packed_entry(*w);
-            nn = packed_ptr(e, 4);
-            if (e && !nn) Py_RETURN_NONE;
+            packed_nn = packed_form(e, 4);
+            if (e && !packed_nn.defined()) Py_RETURN_NONE;
         }
+        const int8_t* nn = codes(packed_nn);
         const int64_t need = (dense ? g_lib.bwd_dense_size : g_lib.bwd_int8_size)(m, n, k);
         if (need < 0) fail(what);
         const Tensor work = workspace(need, *dy), dx = empty({m, k}, at::kBFloat16, *dy);

@@ -180,6 +180,34 @@ def test_packed_rules_same(dev, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_packed_copy_lives_through_the_call(dev):
+    """The registry lets go of the packed copy after the call has looked it up, as a
+    second thread's pack_weight may: its memory stays until the kernels are enqueued."""
+    w8, ws = int8.prepare_weight(_bf(512, 256, dev=dev))
+    x = _bf(8, 256, dev=dev, seed=1)
+    want = int8.linear(x, w8, ws)
+    entry, seen = L.PACKED[w8.untyped_storage().data_ptr()], []
+
+    def stream(index):
+        before = torch.cuda.memory_allocated(dev)
+        entry[3] = None
+        seen.append((before, torch.cuda.memory_allocated(dev)))
+        return L._RAW_STREAM(index)
+
+    lib = L.load()
+    addresses = tuple(L.ctypes.cast(getattr(lib, n), L.ctypes.c_void_p).value
+                      for n in L._HOST_ENTRIES)
+    L.HOST.bind(addresses, stream, L.PACKED)
+    try:
+        got = int8.linear(x, w8, ws)
+    finally:
+        L.HOST.bind(addresses, L._RAW_STREAM, L.PACKED)
+    assert len(seen) == 1 and seen[0][0] == seen[0][1]
+    assert torch.equal(got, want)
+    assert torch.equal(int8.linear(x, w8, ws), want)
+
+
+@pytest.mark.gpu
 def test_modes_take_the_python_path(dev):
     """A torch-function or dispatch mode sees the call's torch operations."""
     from torch.overrides import TorchFunctionMode
