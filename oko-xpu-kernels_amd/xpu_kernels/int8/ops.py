@@ -432,8 +432,9 @@ def _linear_backward(dy, w8, w_scale, want_dbias, bias_dtype, mode):
         f32 = 1 if bias_dtype == torch.float32 else 0
         dbias = torch.empty((n,), device=dy.device, dtype=torch.float32 if f32 else torch.bfloat16)
     if mode == "int8":
+        nn = _packed_nn_for(w8c)   # held: another thread may pack the weight anew
         rc = lib.xpuint8_linear_backward_int8_stream(
-            _stream(dy.device), _ptr(d2), _ptr(ws), _ptr(w8c), _opt(_packed_nn_for(w8c)),
+            _stream(dy.device), _ptr(d2), _ptr(ws), _ptr(w8c), _opt(nn),
             _ptr(dx), _opt(dbias), f32, m, n, k, _ptr(work), nbytes)
     else:
         rc = lib.xpuint8_linear_backward_dense_stream(
@@ -775,9 +776,10 @@ def _linear_acc_bf16(lib, x2, w8c, m, n, k):
     work = torch.empty(int(need), device=x2.device, dtype=torch.uint8)
     acc = torch.empty((m, n), device=x2.device, dtype=torch.int32)
     xs = torch.empty((m,), device=x2.device, dtype=torch.float32)
+    packed = _packed_for(w8c)   # held through the call
     rc = lib.xpuint8_linear_acc_packed_stream(_stream(x2.device), _ptr(x2), _ptr(w8c),
-                                              _opt(_packed_for(w8c)), _ptr(acc), _ptr(xs), m, n,
-                                              k, _ptr(work), int(need))
+                                              _opt(packed), _ptr(acc), _ptr(xs), m, n, k,
+                                              _ptr(work), int(need))
     if rc != 0:
         _err(lib, "linear_acc")
     return acc, xs
@@ -792,8 +794,9 @@ def _linear_residual_bf16(lib, x2, w8c, ws, b, b16, res, rs, m, n, k):
         _err(lib, "linear")
     work = torch.empty(int(need), device=x2.device, dtype=torch.uint8)
     out = torch.empty((m, n), device=x2.device, dtype=torch.bfloat16)
+    packed = _packed_for(w8c)   # held through the call
     rc = lib.xpuint8_linear_residual_packed_stream(
-        _stream(x2.device), _ptr(x2), _ptr(w8c), _opt(_packed_for(w8c)), _ptr(ws), _opt(b), b16,
+        _stream(x2.device), _ptr(x2), _ptr(w8c), _opt(packed), _ptr(ws), _opt(b), b16,
         _ptr(res), _ptr(rs), _ptr(out), m, n, k, _ptr(work), int(need))
     if rc != 0:
         _err(lib, "linear")
