@@ -335,8 +335,10 @@ int xpuint8_linear_backward_int8_stream(const void *stream, const void *dy, cons
  * w_scale) (xpuint8_dequant_weight_stream then xpuint8_linear_dx_stream, bit
  * for bit), the dequantized weight in `work`
  * (xpuint8_linear_backward_dense_workspace_size(M, N, K) bytes: 2*N*K for it,
- * the column sums' partials, and a small batch's split contraction).  K % 256
- * == 0, N % 16 == 0.  Replaces the bias-gradient sum, dequant_weight and
+ * the column sums' partials, and a split contraction's fp32 partial sums; the
+ * last part may be as small as xpuint8_linear_dx_workspace_size(M, N, K), and
+ * the contraction is then split less).  The size may be asked for without a
+ * device, and holds on every device.  K % 256 == 0, N % 16 == 0.  Replaces the bias-gradient sum, dequant_weight and
  * linear_dx of python/xpu_kernels/int8/ops.py:270-289; no counterpart as one
  * call. */
 int64_t xpuint8_linear_backward_dense_workspace_size(int64_t M, int64_t N, int64_t K);

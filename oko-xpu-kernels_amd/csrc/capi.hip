@@ -1021,8 +1021,13 @@ int xpuint8_linear_dx_stream(const void* stream, const void* dy, const void* w, 
 // The workspace of xpuint8_linear_backward_dense_stream: the dequantized
 // weight bf16 [N, K], the column sums' partials, and (for a contraction split
 // across blocks) the bf16 GEMM's fp32 partials, each on a 256-byte boundary.
+// `need`, what a call has to bring, follows from M, N and K alone; the slices
+// that the GEMM would like depend on the device's CU count, which a caller that
+// asks for the size before the first call, or with another device current, does
+// not name.  `total`, what the size entry gives, is never less than `need`, and
+// the GEMM splits as far as the bytes it is given allow.
 struct DenseBwdWork {
-    size_t wd, colsum, part, total;
+    size_t wd, colsum, part, need, total;
 };
 static DenseBwdWork dense_bwd_layout(int64_t M, int64_t N, int64_t K) {
     auto up = [](int64_t b) { return (size_t(b) + 255) & ~size_t(255); };
@@ -1030,7 +1035,8 @@ static DenseBwdWork dense_bwd_layout(int64_t M, int64_t N, int64_t K) {
     w.wd = 0;
     w.colsum = up(2 * N * K);
     w.part = w.colsum + up(colsum_work_bytes(M, N));
-    w.total = w.part + size_t(bf16_dx_work_bytes(int(M), int(N), int(K)));
+    w.need = w.part + size_t(bf16_nn_slices(int(M), int(N), int(K))) * size_t(M) * size_t(K) * 4;
+    w.total = std::max(w.need, w.part + size_t(bf16_dx_work_bytes(int(M), int(N), int(K))));
     return w;
 }
 
@@ -1049,7 +1055,7 @@ int xpuint8_linear_backward_dense_stream(const void* stream, const void* dy, con
     XPU_ALIGNED_OPT(dbias);
     if (dbias_fp32 != 0 && dbias_fp32 != 1) return fail(2, "dbias_fp32 must be 0 or 1");
     const DenseBwdWork L = dense_bwd_layout(M, N, K);
-    if (work_bytes < int64_t(L.total))
+    if (work_bytes < int64_t(L.need))
         return fail(2, "work must hold xpuint8_linear_backward_dense_workspace_size(M, N, K) bytes");
     XPU_TRY(ensure_device());
     hipStream_t st = as_stream(stream);
@@ -1063,7 +1069,7 @@ int xpuint8_linear_backward_dense_stream(const void* stream, const void* dy, con
                      "linear_backward_dense (dequant_weight)"));
     return launched(gemm_bf16_nn(st, dy, N, wd, K, dx, K, int(M), int(N), int(K),
                                  reinterpret_cast<float*>(w + L.part),
-                                 int64_t(L.total - L.part)),
+                                 work_bytes - int64_t(L.part)),
                     "linear_backward_dense (gemm)");
 }
 

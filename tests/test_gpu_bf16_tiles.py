@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from xpu_kernels import int8
+from xpu_kernels.int8 import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,28 @@ def test_linear_dx_wide_rows(dev):
     dx = int8.linear_dx(dy, w)
     for cut in (slice(0, 4096), slice(k // 2, k // 2 + 4096), slice(k - 4096, k)):
         check(dx[:, cut], dy, w[:, cut])
+
+
+@pytest.mark.parametrize("m,n,k", [(205, 2672, 768), (322, 5648, 2048), (1024, 5120, 1280)])
+def test_dense_backward_in_less_workspace(dev, m, n, k):
+    """xpuint8_linear_backward_dense_stream in the least workspace it takes (a size
+    that names no device), nothing written past it: dx as linear_dx_stream gives it
+    with that much for its partial sums, bit for bit."""
+    lib = L._lib()
+    dy = operand(m, n, 1e-3, m, dev)
+    w8, ws = int8.prepare_weight(operand(n, k, 0.02, n + k, dev))
+    wd = int8.dequant_weight(w8, ws)
+    part = lib.xpuint8_linear_dx_workspace_size(m, n, k)
+    least = (2 * n * k + 255) // 256 * 256 + (-(-m // 32) * n * 4 + 255) // 256 * 256 + part
+    work = torch.full((least + 4096,), 0x55, device=dev, dtype=torch.uint8)
+    dx = torch.empty(m, k, device=dev, dtype=torch.bfloat16)
+    rc = lib.xpuint8_linear_backward_dense_stream(L._stream(dev), L._ptr(dy), L._ptr(w8), L._ptr(ws),
+                                                  L._ptr(dx), None, 0, m, n, k, L._ptr(work), least)
+    assert rc == 0, lib.xpuint8_last_error()
+    assert bool((work[least:] == 0x55).all())
+    want = torch.empty_like(dx)
+    w2 = torch.empty(max(part, 16), device=dev, dtype=torch.uint8)
+    assert lib.xpuint8_linear_dx_stream(L._stream(dev), L._ptr(dy), L._ptr(wd), L._ptr(want), m, n,
+                                        k, L._ptr(w2) if part else None, part) == 0
+    assert torch.equal(dx, want)
+    check(dx, dy, wd)

@@ -207,6 +207,30 @@ def test_linear_dx_workspace_size(lib):
     assert lib.xpuint8_linear_dx_workspace_size(100, 215040, 20000) == 0
 
 
+# contractions the GEMM would like to split (by the device's CU count) where
+# xpuint8_linear_dx_workspace_size has no slices, fewer, and as many or more
+DENSE_SHAPES = [(205, 2672, 768), (322, 5648, 2048), (1024, 5120, 1280), (200, 2048, 1280),
+                (4096, 5120, 1280), (3, 16, 256)]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="calls with pointers no device may read")
+@pytest.mark.parametrize("m,n,k", DENSE_SHAPES)
+def test_dense_backward_size_needs_no_device(lib, m, n, k):
+    """What xpuint8_linear_backward_dense_stream requires follows from M, N and K
+    alone: bf16 [N, K] weight, the column sums' partials and
+    xpuint8_linear_dx_workspace_size; the size entry, whose split also follows the
+    device, is never below it.  Without a device: enough bytes fail for the
+    device (code 1), one fewer for the workspace (code 2)."""
+    fixed = up256(2 * n * k) + up256(-(-m // 32) * n * 4)
+    least = fixed + lib.xpuint8_linear_dx_workspace_size(m, n, k)
+    assert lib.xpuint8_linear_backward_dense_workspace_size(m, n, k) == max(
+        least, fixed + lib.xpuint8_linear_dx_split_workspace_size(m, n, k))
+    for nbytes, code, substr in ((least, 1, "device"), (least - 1, 2, "workspace_size")):
+        rc, msg = _rc(lib, "xpuint8_linear_backward_dense_stream", Z, P, P, P, P, Z, 0, m, n, k, P,
+                      nbytes)
+        assert rc == code and substr in msg, (nbytes, rc, msg)
+
+
 def test_linear_workspace_size(lib):
     """The linear's workspace: the quantized activation (row-major or in the
     block layout, whichever is larger) rounded up to 256 bytes, then its fp32
