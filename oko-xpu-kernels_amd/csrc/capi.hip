@@ -430,8 +430,10 @@ int act_ok(int32_t act) {
 int device_cus() {
     int dev = 0;
     (void)hipGetDevice(&dev);
-    const int n = (dev >= 0 && dev < kMaxDevices) ? g_cus[dev] : 0;
-    return n > 0 ? n : 256;
+    // g_cus is written once, before g_ready is released: the size entries come here
+    // without ensure_device, beside another thread's first call
+    if (dev < 0 || dev >= kMaxDevices || !g_ready[dev].load(std::memory_order_acquire)) return 256;
+    return g_cus[dev];
 }
 
 const uint16_t* activation_tables() {
