@@ -21,6 +21,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
+#include <cstdio>
+#include <cstring>
 #include <exception>
 #include <vector>
 
@@ -478,6 +480,35 @@ PyMethodDef kMethods[] = {XPU_HOST("bind", host_bind),
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host",
                        "The int8 API's hot calls in native code (see host_ops.cpp).", -1, kMethods};
 
+// Tensors are read by the layout that torch's headers gave at build time, and
+// another build of torch can export the same symbols over another layout: the
+// module loads only into the Python and the torch (version and commit) that the
+// Makefile found, XPU_BUILT_FOR = "3.10/2.10.0+rocm7.0/<commit>", and raises
+// ImportError elsewhere.
+bool built_for_this() {
+    int major = 0, minor = 0;
+    std::sscanf(Py_GetVersion(), "%d.%d", &major, &minor);
+    PyObject* v = PyImport_ImportModule("torch.version");
+    PyObject* version = v ? PyObject_GetAttrString(v, "__version__") : nullptr;
+    PyObject* commit = version ? PyObject_GetAttrString(v, "git_version") : nullptr;
+    PyObject* now = commit ? PyUnicode_FromFormat("%d.%d/%S/%S", major, minor, version, commit)
+                           : nullptr;
+    const bool ok = now && PyUnicode_CompareWithASCIIString(now, XPU_BUILT_FOR) == 0;
+    if (!ok) {
+        PyErr_Clear();
+        PyErr_Format(PyExc_ImportError, "_host.so was built for " XPU_BUILT_FOR ", not %S",
+                     now ? now : Py_None);
+    }
+    Py_XDECREF(now);
+    Py_XDECREF(commit);
+    Py_XDECREF(version);
+    Py_XDECREF(v);
+    return ok;
+}
+
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__host(void) {
+    if (!built_for_this()) return nullptr;
+    return PyModule_Create(&kModule);
+}

@@ -158,7 +158,8 @@ _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 def _bind_host(lib):
     """The native host path bound to the loaded library, or None: not built, built
-    for another torch, or torch without the raw stream accessor."""
+    for another Python or torch (it compares itself with the running ones when
+    it is imported), or torch without the raw stream accessor."""
     if _RAW_STREAM is None:
         return None
     try:

@@ -5,6 +5,7 @@ batch dims, empty batches, refused shapes, active torch modes -- and the packed
 copy's rules."""
 
 import importlib
+import os
 
 import pytest
 import torch
@@ -25,6 +26,24 @@ def test_module_is_built_and_answers_none_unbound():
         host.linear(x, w8)
     with pytest.raises(TypeError):
         host.bind((), None, {})
+
+
+@pytest.mark.parametrize("name", ["__version__", "git_version"])
+def test_module_refuses_another_torch(name):
+    """Built for one torch (version and commit); under another, whose tensors may be
+    laid out differently, it is not loaded and the Python path stays."""
+    import subprocess
+    import sys
+    code = (f"import torch.version as v; v.{name} = v.{name} + '0'\n"
+            "from xpu_kernels.int8 import _lib as L\n"
+            "assert L._bind_host(L.open_library(L.library_path())) is None\n"
+            "try:\n    from xpu_kernels.int8 import _host\n"
+            "except ImportError as e:\n    assert 'built for' in str(e), e\n"
+            "else:\n    raise AssertionError('loaded')\n")
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(p for p in sys.path if p))
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stderr
 
 
 def _outcome(fn):
