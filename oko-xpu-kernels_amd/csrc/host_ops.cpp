@@ -26,39 +26,33 @@
 #include <exception>
 #include <vector>
 
+#include "xpuint8.h"
+
 namespace {
 
 using at::Tensor;
 
 // ---------------------------------------------------------- the library
-// Addresses of the loaded libxpuint8.so's entry points (include/xpuint8.h), in the
-// order bind() receives them.
+// Addresses of the loaded libxpuint8.so's entry points, in the order bind()
+// receives them (_lib.py's _HOST_ENTRIES), called by the header's own types.
 struct Library {
-    const char* (*last_error)();
-    int64_t (*linear_size)(int64_t, int64_t, int64_t);
-    int (*linear)(const void*, const void*, const int8_t*, const int8_t*, const float*, const void*,
-                  int32_t, void*, int64_t, int64_t, int64_t, void*, int64_t);
-    int64_t (*ffn_size)(int64_t, int64_t, int64_t, int32_t);
-    int (*ffn)(const void*, const void*, const int8_t*, const int8_t*, const float*, const int8_t*,
-               const int8_t*, const float*, const void*, int32_t, void*, int64_t, int64_t, int64_t,
-               int32_t, void*, int64_t);
-    int64_t (*bwd_int8_size)(int64_t, int64_t, int64_t);
-    int (*bwd_int8)(const void*, const void*, const float*, const int8_t*, const int8_t*, void*,
-                    void*, int32_t, int64_t, int64_t, int64_t, void*, int64_t);
-    int64_t (*bwd_dense_size)(int64_t, int64_t, int64_t);
-    int (*bwd_dense)(const void*, const void*, const int8_t*, const float*, void*, void*, int32_t,
-                     int64_t, int64_t, int64_t, void*, int64_t);
-    int64_t (*dx_size)(int64_t, int64_t, int64_t);
-    int (*dx)(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, void*,
-              int64_t);
-    int64_t (*dw_size)(int64_t, int64_t, int64_t);
-    int (*dw)(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, void*,
-              int64_t);
-    int64_t (*colsum_size)(int64_t, int64_t);
-    int (*colsum)(const void*, const void*, void*, int64_t, int64_t, void*, int64_t);
-    int (*quantize)(const void*, const void*, int8_t*, float*, int64_t, int64_t);
-    int (*linear_acc)(const void*, const void*, const int8_t*, const int8_t*, int32_t*, float*,
-                      int64_t, int64_t, int64_t, void*, int64_t);
+    decltype(&xpuint8_last_error) last_error;
+    decltype(&xpuint8_linear_workspace_size) linear_size;
+    decltype(&xpuint8_linear_packed_stream) linear;
+    decltype(&xpuint8_ffn_workspace_size) ffn_size;
+    decltype(&xpuint8_ffn_packed_stream) ffn;
+    decltype(&xpuint8_linear_backward_int8_workspace_size) bwd_int8_size;
+    decltype(&xpuint8_linear_backward_int8_stream) bwd_int8;
+    decltype(&xpuint8_linear_backward_dense_workspace_size) bwd_dense_size;
+    decltype(&xpuint8_linear_backward_dense_stream) bwd_dense;
+    decltype(&xpuint8_linear_dx_split_workspace_size) dx_size;
+    decltype(&xpuint8_linear_dx_stream) dx;
+    decltype(&xpuint8_linear_dw_workspace_size) dw_size;
+    decltype(&xpuint8_linear_dw_work_stream) dw;
+    decltype(&xpuint8_column_sum_workspace_size) colsum_size;
+    decltype(&xpuint8_column_sum_stream) colsum;
+    decltype(&xpuint8_convrot_quantize_stream) quantize;
+    decltype(&xpuint8_linear_acc_packed_stream) linear_acc;
 };
 constexpr int kEntries = 17;
 static_assert(sizeof(Library) == kEntries * sizeof(void*), "one address per entry");

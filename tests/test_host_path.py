@@ -46,6 +46,18 @@ def test_module_refuses_another_torch(name):
     assert r.returncode == 0, r.stderr
 
 
+def test_entries_are_called_by_the_headers_types():
+    """The addresses bind() receives, one for one: the native table holds the same
+    entry points in the same order, each with the type xpuint8.h declares."""
+    import re
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src = open(os.path.join(root, "oko-xpu-kernels_amd", "csrc", "host_ops.cpp")).read()
+    table = src[src.index("struct Library {"):]
+    table = table[:table.index("};")]
+    assert re.findall(r"decltype\(&(xpuint8_\w+)\) \w+;", table) == list(L._HOST_ENTRIES)
+    assert "(*" not in table and '#include "xpuint8.h"' in src
+
+
 def _outcome(fn):
     try:
         r = fn()
