@@ -6,6 +6,7 @@ convention, src/xpuint8.cpp:733-776, 999-1002)."""
 import ctypes
 import os
 import re
+import sys
 
 import pytest
 import torch
@@ -51,6 +52,19 @@ def test_c_consumer_is_built_and_links():
     assert os.path.exists(binp), "not built (run __graft_entry__.build())"
     r = subprocess.run([binp], capture_output=True, text=True, timeout=60)
     assert r.returncode == 2 and "usage" in r.stderr, r.stderr
+
+
+@pytest.mark.parametrize("python,host", [("false", False), (sys.executable, True)])
+def test_library_builds_without_torch(python, host):
+    """`make` as a C consumer of the library runs it, where Python has no torch (or
+    there is no Python): the library and the C programs, without the Python
+    API's host path."""
+    import subprocess
+    r = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "oko-xpu-kernels_amd", "csrc"),
+                        f"PYTHON={python}"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    assert "libxpuint8.so" in r.stdout and "linear_consumer" in r.stdout
+    assert ("_host.so" in r.stdout) == host
 
 
 P = ctypes.c_void_p(0x1000)   # never dereferenced: validation runs first
