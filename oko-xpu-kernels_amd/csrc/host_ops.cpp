@@ -181,12 +181,22 @@ Tensor workspace(int64_t bytes, const Tensor& like) { return empty({bytes}, at::
     throw python_error();
 }
 
-// f() without the GIL (as a ctypes call runs); its error, if any, raised
+// The GIL released for a scope, an exception's way out of it included
+struct NoGil {
+    PyThreadState* s = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(s); }
+};
+
+// f() without the GIL: the allocations (as torch.empty makes them: one that
+// misses the allocator's cache can wait for the device) and the library call
+// (as ctypes makes it); its error, if any, raised
 template <class F>
 void call(const char* what, const F& f) {
-    PyThreadState* s = PyEval_SaveThread();
-    const int rc = f();
-    PyEval_RestoreThread(s);
+    int rc;
+    {
+        NoGil g;
+        rc = f();
+    }
     if (rc != 0) fail(what);
 }
 
@@ -241,11 +251,13 @@ PyObject* host_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (!ws || !b.ok) Py_RETURN_NONE;
         const int64_t need = g_lib.linear_size(m, n, k);
         if (need < 0) fail("linear");
-        const Tensor work = workspace(need, *x), out = empty(with_last(*x, n), at::kBFloat16, *x);
         const Tensor packed = packed_form(packed_entry(*w), 3);
         const int8_t* p = codes(packed);
         const void* st = current_stream(*x);
+        Tensor work, out;
         call("linear", [&] {
+            work = workspace(need, *x);
+            out = empty(with_last(*x, n), at::kBFloat16, *x);
             return g_lib.linear(st, x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), p,
                                 static_cast<const float*>(ws->data_ptr()), b.p, b.bf16,
                                 out.data_ptr(), m, n, k, work.data_ptr(), need);
@@ -265,12 +277,14 @@ PyObject* host_linear_acc(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (x->size(-1) != k || k % 256 != 0 || n % 16 != 0) Py_RETURN_NONE;
         const int64_t need = g_lib.linear_size(m, n, k);
         if (need < 0) fail("linear_acc");
-        const Tensor work = workspace(need, *x), acc = empty({m, n}, at::kInt, *x),
-                     xs = empty({m}, at::kFloat, *x);
         const Tensor packed = packed_form(packed_entry(*w), 3);
         const int8_t* p = codes(packed);
         const void* st = current_stream(*x);
+        Tensor work, acc, xs;
         call("linear_acc", [&] {
+            work = workspace(need, *x);
+            acc = empty({m, n}, at::kInt, *x);
+            xs = empty({m}, at::kFloat, *x);
             return g_lib.linear_acc(st, x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), p,
                                     static_cast<int32_t*>(acc.data_ptr()),
                                     static_cast<float*>(xs.data_ptr()), m, n, k, work.data_ptr(),
@@ -301,12 +315,14 @@ PyObject* host_ffn(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (!us || !ds || !b.ok) Py_RETURN_NONE;
         const int64_t need = g_lib.ffn_size(m, inner, k, int32_t(act));
         if (need < 0) fail("ffn");
-        const Tensor work = workspace(need, *x), out = empty(x->sizes(), at::kBFloat16, *x);
         const Tensor up_packed = packed_form(packed_entry(*up), 3),
                      down_packed = packed_form(packed_entry(*down), 3);
         const int8_t *up_p = codes(up_packed), *down_p = codes(down_packed);
         const void* st = current_stream(*x);
+        Tensor work, out;
         call("ffn", [&] {
+            work = workspace(need, *x);
+            out = empty(x->sizes(), at::kBFloat16, *x);
             return g_lib.ffn(st, x->data_ptr(), static_cast<const int8_t*>(up->data_ptr()), up_p,
                              static_cast<const float*>(us->data_ptr()),
                              static_cast<const int8_t*>(down->data_ptr()), down_p,
@@ -343,14 +359,15 @@ PyObject* host_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const int8_t* nn = codes(packed_nn);
         const int64_t need = (dense ? g_lib.bwd_dense_size : g_lib.bwd_int8_size)(m, n, k);
         if (need < 0) fail(what);
-        const Tensor work = workspace(need, *dy), dx = empty({m, k}, at::kBFloat16, *dy);
-        Tensor db;
-        if (want) db = empty({n}, f32 ? at::kFloat : at::kBFloat16, *dy);
-        void* dbp = want ? db.data_ptr() : nullptr;
         const int8_t* wp = static_cast<const int8_t*>(w->data_ptr());
         const float* wsp = static_cast<const float*>(ws->data_ptr());
         const void* st = current_stream(*dy);
+        Tensor work, dx, db;
         call(what, [&] {
+            work = workspace(need, *dy);
+            dx = empty({m, k}, at::kBFloat16, *dy);
+            if (want) db = empty({n}, f32 ? at::kFloat : at::kBFloat16, *dy);
+            void* dbp = want ? db.data_ptr() : nullptr;
             return dense ? g_lib.bwd_dense(st, dy->data_ptr(), wp, wsp, dx.data_ptr(), dbp,
                                            want && f32, m, n, k, work.data_ptr(), need)
                          : g_lib.bwd_int8(st, dy->data_ptr(), wsp, wp, nn, dx.data_ptr(), dbp,
@@ -370,10 +387,11 @@ PyObject* host_linear_dx(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (dy->size(-1) != n || n % 16 != 0 || k % 16 != 0) Py_RETURN_NONE;
         const int64_t need = g_lib.dx_size(m, n, k);
         if (need < 0) fail("linear_dx");
-        const Tensor work = need > 0 ? workspace(need, *dy) : Tensor(),
-                     dx = empty(with_last(*dy, k), at::kBFloat16, *dy);
         const void* st = current_stream(*dy);
+        Tensor work, dx;
         call("linear_dx", [&] {
+            if (need > 0) work = workspace(need, *dy);
+            dx = empty(with_last(*dy, k), at::kBFloat16, *dy);
             return g_lib.dx(st, dy->data_ptr(), w->data_ptr(), dx.data_ptr(), m, n, k,
                             need > 0 ? work.data_ptr() : nullptr, need);
         });
@@ -392,10 +410,11 @@ PyObject* host_linear_dw(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (n % 16 != 0 || k % 16 != 0) Py_RETURN_NONE;
         const int64_t need = g_lib.dw_size(m, n, k);
         if (need < 0) fail("linear_dw");
-        const Tensor work = need > 0 ? workspace(need, *dy) : Tensor(),
-                     dw = empty({n, k}, at::kBFloat16, *dy);
         const void* st = current_stream(*dy);
+        Tensor work, dw;
         call("linear_dw", [&] {
+            if (need > 0) work = workspace(need, *dy);
+            dw = empty({n, k}, at::kBFloat16, *dy);
             return g_lib.dw(st, dy->data_ptr(), x->data_ptr(), dw.data_ptr(), m, n, k,
                             need > 0 ? work.data_ptr() : nullptr, need);
         });
@@ -410,10 +429,11 @@ PyObject* host_column_sum(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (!dy || dy->dim() != 2 || dy->size(1) % 16 != 0) Py_RETURN_NONE;
         const int64_t m = dy->size(0), n = dy->size(1), need = g_lib.colsum_size(m, n);
         if (need < 0) fail("column_sum");
-        const Tensor work = workspace(std::max<int64_t>(need, 16), *dy),
-                     out = empty({n}, at::kBFloat16, *dy);
         const void* st = current_stream(*dy);
+        Tensor work, out;
         call("column_sum", [&] {
+            work = workspace(std::max<int64_t>(need, 16), *dy);
+            out = empty({n}, at::kBFloat16, *dy);
             return g_lib.colsum(st, dy->data_ptr(), out.data_ptr(), m, n, work.data_ptr(), need);
         });
         return THPVariable_Wrap(out);
@@ -426,10 +446,11 @@ PyObject* host_quantize(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const Tensor* x = plain(a[0], at::kBFloat16);
         if (!x || x->dim() < 1) Py_RETURN_NONE;
         const int64_t k = x->size(-1), m = x->numel() / k;
-        const Tensor q = empty(x->sizes(), at::kChar, *x),
-                     s = empty(x->sizes().slice(0, x->dim() - 1), at::kFloat, *x);
         const void* st = current_stream(*x);
+        Tensor q, s;
         call("quantize", [&] {
+            q = empty(x->sizes(), at::kChar, *x);
+            s = empty(x->sizes().slice(0, x->dim() - 1), at::kFloat, *x);
             return g_lib.quantize(st, x->data_ptr(), static_cast<int8_t*>(q.data_ptr()),
                                   static_cast<float*>(s.data_ptr()), m, k);
         });
