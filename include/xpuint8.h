@@ -349,7 +349,10 @@ int xpuint8_linear_backward_dense_stream(const void *stream, const void *dy, con
 
 /* xpuint8_linear_dx_int8_stream, bit for bit, reading w8_packed_nn (w8 packed
  * by xpuint8_pack_weight_nn_stream; null reads w8) where the split-K GEMM
- * takes the product. */
+ * takes the product: where xpuint8_linear_dx_int8_reads_packed(M, N, K) is 1 (0:
+ * the packed copy is not read, -1: a shape the entry point rejects), which
+ * depends on the current device's CU count (256 before its first use). */
+int32_t xpuint8_linear_dx_int8_reads_packed(int64_t M, int64_t N, int64_t K);
 int xpuint8_linear_dx_int8_packed_stream(const void *stream, const void *dy, const float *w_scale,
                                          const int8_t *w8, const int8_t *w8_packed_nn, void *dx,
                                          int64_t M, int64_t N, int64_t K, void *work,

@@ -170,6 +170,17 @@ int check_dx(int64_t M, int64_t N, int64_t K) {
     return check_gemm(M, K, N);              // q [M,N] @ w8 [N,K], contraction over N
 }
 
+// Whether dx_chain takes one round of the split-K kernel's 128 x 160 tiles, which
+// reads w8 [N, K] as it is stored (transposing LDS reads), or pack_weight_nn's
+// copy of it.  (More than one round: the packed tiles are faster, whole chain
+// 73.3 -> 57.3 us at M=2263, N=5216, K=2560, 288 tiles, 59.5 -> 51.6 at 3522 x 3584 x
+// 2048, 364 tiles; at 252 tiles, 1527 x 4672 x 3328, 43.7 against 48.1 there, at
+// 128, 984 x 5136 x 2560, 40.6 against 43.1.)
+bool dx_one_round(int64_t M, int64_t N, int64_t K) {
+    return ((M + 127) / 128) * ((K + 159) / 160) <= device_cus() &&
+           splitk_nn_applies(int(M), int(K), int(N), K) && rowquant_can_tile(int(N));
+}
+
 // quantize_row (column-scaled) -> w8^T -> GEMM with the row-scale epilogue ->
 // inverse rotation, all on one stream, through the workspace at `work`.
 // wnn (optional): pack_weight_nn's copy of w8, read by the split-K GEMM.
@@ -190,14 +201,8 @@ int dx_chain(hipStream_t st, const void* dy, const float* w_scale, const int8_t*
         const hipError_t e = column_sum_bf16(st, dy, dbias, M, int(N), cpart, dbias_fp32);
         return e != hipSuccess ? e : quantize_row(st, dy, w_scale, q, a, M, int(N), tiled);
     };
-    // one round of the split-K kernel's 128 x 160 tiles: it reads w8 [N, K] as
-    // it is stored (transposing LDS reads) and q in the MFMA block layout,
-    // written so by the quantizer.  (More than one round: the tiles below are
-    // faster, whole chain 73.3 -> 57.3 us at M=2263, N=5216, K=2560, 288 tiles, 59.5
-    // -> 51.6 at 3522 x 3584 x 2048, 364 tiles; at 252 tiles, 1527 x 4672 x 3328,
-    // 43.7 against 48.1 there, at 128, 984 x 5136 x 2560, 40.6 against 43.1.)
-    const bool one_round = ((M + 127) / 128) * ((K + 159) / 160) <= device_cus();
-    if (one_round && splitk_nn_applies(int(M), int(K), int(N), K) && rowquant_can_tile(int(N))) {
+    // q in the MFMA block layout, written so by the quantizer
+    if (dx_one_round(M, N, K)) {
         XPU_TRY(launched(quantize(true),
                          "linear_dx_int8 (quantize_row)"));
         XPU_TRY(launched(gemm_dequant_nn_xt(st, q, wnn ? wnn : w8, K, pre, K, a, int(M), int(K),
@@ -912,6 +917,11 @@ int xpuint8_pack_weight_nn_stream(const void* stream, const int8_t* w8, int8_t* 
     XPU_NONNULL(w8); XPU_NONNULL(packed);
     XPU_TRY(ensure_device());
     return launched(pack_weight_nn(as_stream(stream), w8, packed, N, int(K)), "pack_weight_nn");
+}
+
+int32_t xpuint8_linear_dx_int8_reads_packed(int64_t M, int64_t N, int64_t K) {
+    if (check_dx(M, N, K) != 0) return -1;
+    return dx_one_round(M, N, K) ? 1 : 0;
 }
 
 int xpuint8_linear_dx_int8_packed_stream(const void* stream, const void* dy, const float* w_scale,

@@ -53,8 +53,9 @@ struct Library {
     decltype(&xpuint8_column_sum_stream) colsum;
     decltype(&xpuint8_convrot_quantize_stream) quantize;
     decltype(&xpuint8_linear_acc_packed_stream) linear_acc;
+    decltype(&xpuint8_linear_dx_int8_reads_packed) dx_reads_packed;
 };
-constexpr int kEntries = 17;
+constexpr int kEntries = 18;
 static_assert(sizeof(Library) == kEntries * sizeof(void*), "one address per entry");
 
 Library g_lib;
@@ -334,8 +335,8 @@ PyObject* host_ffn(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // backward(dy, w8, w_scale, want_dbias, dbias_fp32, dense): ops._linear_backward's
-// (dx, dbias or None).  The int8 mode of a weight whose second packed form is
-// still to be made goes through Python, which makes it.
+// (dx, dbias or None).  The int8 mode of a weight whose second packed form this
+// product reads and is still to be made goes through Python, which makes it.
 PyObject* host_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     return guarded(n_args, 6, [&]() -> PyObject* {
         const Tensor* dy = plain(a[0], at::kBFloat16);
@@ -354,7 +355,7 @@ PyObject* host_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (!dense) {
             PyObject* e = packed_entry(*w);
             packed_nn = packed_form(e, 4);
-            if (e && !packed_nn.defined()) Py_RETURN_NONE;
+            if (e && !packed_nn.defined() && g_lib.dx_reads_packed(m, n, k) == 1) Py_RETURN_NONE;
         }
         const int8_t* nn = codes(packed_nn);
         const int64_t need = (dense ? g_lib.bwd_dense_size : g_lib.bwd_int8_size)(m, n, k);

@@ -42,7 +42,8 @@ _HOST_ENTRIES = (
     "xpuint8_linear_dx_split_workspace_size", "xpuint8_linear_dx_stream",
     "xpuint8_linear_dw_workspace_size", "xpuint8_linear_dw_work_stream",
     "xpuint8_column_sum_workspace_size", "xpuint8_column_sum_stream",
-    "xpuint8_convrot_quantize_stream", "xpuint8_linear_acc_packed_stream")
+    "xpuint8_convrot_quantize_stream", "xpuint8_linear_acc_packed_stream",
+    "xpuint8_linear_dx_int8_reads_packed")
 
 
 def _candidate_paths():
@@ -114,6 +115,7 @@ def _signatures():
         "xpuint8_column_sum_stream": ([vp] * 3 + [i64] * 2 + [vp, i64], c_int),
         "xpuint8_column_sum_workspace_size": ([i64] * 2, i64),
         "xpuint8_linear_dx_int8_workspace_size": ([i64] * 3, i64),
+        "xpuint8_linear_dx_int8_reads_packed": ([i64] * 3, i32),
         "xpuint8_linear_dx_int8_noalloc_stream": ([vp] * 5 + [i64] * 3, c_int),
         "xpuint8_prepare_weight_stream": ([vp] * 4 + [i64] * 2, c_int),
         "xpuint8_prepare_weight_packed_stream": ([vp] * 5 + [i64] * 2, c_int),

@@ -55,8 +55,8 @@ def _opt(t):
 # the storage is.  Writes the version counter does not see (through
 # ``.data``, DLPack or raw pointers) need a new :func:`pack_weight`.
 # _PACKED: storage data_ptr -> [weakref to the storage, version, shape, packed,
-# packed_nn] (packed_nn: the form linear_dx_int8's product reads, made at its
-# first use); csrc/host_ops.cpp reads it by the same rules
+# packed_nn] (packed_nn: the form linear_dx_int8's split-K product reads, made at the
+# first that does); csrc/host_ops.cpp reads it by the same rules
 
 
 def _pack_key(w8):
@@ -142,16 +142,18 @@ def _packed_for(w8):
     return None if e is None else e[3]
 
 
-def _packed_nn_for(w8):
+def _packed_nn_for(w8, m):
     """The second packed form of a weight with a valid packed copy (the order
     in which linear_dx_int8's split-K product reads w8 [N, K] as its right
-    operand), made at the first call outside a graph capture; else None."""
+    operand), made at the first call outside a graph capture whose product (dy
+    of ``m`` rows) reads it; else None."""
     e = _packed_entry(w8)
     if e is None:
         return None
-    if e[4] is None and not is_capturing():
-        lib = _lib()
-        n, k = e[2]
+    lib = _lib()
+    n, k = e[2]
+    if (e[4] is None and not is_capturing()
+            and lib.xpuint8_linear_dx_int8_reads_packed(m, n, k) == 1):
         need = lib.xpuint8_packed_weight_nn_bytes(n, k)
         if need < 0:
             return None
@@ -432,7 +434,7 @@ def _linear_backward(dy, w8, w_scale, want_dbias, bias_dtype, mode):
         f32 = 1 if bias_dtype == torch.float32 else 0
         dbias = torch.empty((n,), device=dy.device, dtype=torch.float32 if f32 else torch.bfloat16)
     if mode == "int8":
-        nn = _packed_nn_for(w8c)   # held: another thread may pack the weight anew
+        nn = _packed_nn_for(w8c, m)   # held: another thread may pack the weight anew
         rc = lib.xpuint8_linear_backward_int8_stream(
             _stream(dy.device), _ptr(d2), _ptr(ws), _ptr(w8c), _opt(nn),
             _ptr(dx), _opt(dbias), f32, m, n, k, _ptr(work), nbytes)
@@ -542,7 +544,7 @@ def linear_dx_int8(dy, w8, w_scale):
         _err(lib, "linear_dx_int8")
     work = torch.empty((nbytes,), device=dy.device, dtype=torch.int8)
     dx = torch.empty((m, k), device=dy.device, dtype=torch.bfloat16)
-    nn = _packed_nn_for(w8c)
+    nn = _packed_nn_for(w8c, m)
     if nn is not None:
         rc = lib.xpuint8_linear_dx_int8_packed_stream(_stream(dy.device), _ptr(d2), _ptr(ws),
                                                       _ptr(w8c), _ptr(nn), _ptr(dx), m, n, k,

@@ -14,6 +14,7 @@ import oracle as O
 from gpu_util import bits, mismatch, npy, weight
 from xpu_kernels import int8
 from xpu_kernels.int8 import _lib as L
+from xpu_kernels.int8 import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +44,23 @@ def test_dx_int8_by_shape_exact(dev, m, n, k):
         want = O.linear_dx_int8(bits(dy), npy(w8), npy(ws))
         assert np.array_equal(got, want), mismatch(got, want)
         assert bool((guard[m * k:] == 7.0).all())
+
+
+# one round of the split-K kernel (which reads the second packed form); more rounds,
+# few tiles, a short contraction (which do not)
+@pytest.mark.parametrize("m,n,k,reads", [(2060, 2064, 1280, True), (4096, 1040, 1536, False),
+                                         (300, 2608, 768, False), (2060, 528, 1280, False)])
+def test_second_packed_form_only_where_read(dev, m, n, k, reads):
+    """int8 backwards and linear_dx_int8 make the weight's second packed form, which
+    stays with it, only for a product that reads it."""
+    w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
+    dy = (torch.randn(m, n, generator=torch.Generator().manual_seed(m)) * 1e-3).to(torch.bfloat16)
+    want = int8.linear_dx_int8(dy.to(dev), w8.clone(), ws)      # (no packed copy)
+    x = torch.zeros(m, k, device=dev, dtype=torch.bfloat16, requires_grad=True)
+    for _ in range(2):
+        x.grad = None
+        int8.int8_linear(x, w8, ws, mode="int8").backward(dy.to(dev))
+        assert torch.equal(x.grad, want)
+        assert (ops._packed_entry(w8)[4] is not None) == reads
+    assert torch.equal(int8.linear_dx_int8(dy.to(dev), w8, ws), want)
+    assert (ops._packed_entry(w8)[4] is not None) == reads

@@ -174,6 +174,16 @@ def test_dx_workspace_size(lib):
     assert lib.xpuint8_linear_dx_int8_workspace_size(4, 32, 300) == -1
 
 
+def test_dx_reads_packed(lib):
+    """The NN packed copy is read by one round of the split-K kernel's 128 x 160 tiles
+    of dx [M, K] (128 to 256 of them, a contraction of at least 1024): 256 CUs
+    before a device is set up."""
+    for (m, n, k), want in {(4096, 5120, 1280): 1, (4096, 1280, 5120): 0, (2060, 2064, 1280): 1,
+                            (1024, 5120, 1280): 0, (4096, 1008, 1280): 0, (33, 528, 256): 0,
+                            (4096, 5120, 1536): 0, (4, 24, 512): -1, (4, 32, 300): -1}.items():
+        assert lib.xpuint8_linear_dx_int8_reads_packed(m, n, k) == want, (m, n, k)
+
+
 def k_slices(m, n, k):
     """The K slices of a product split across blocks.  First the skinny
     kernel's, for 33 <= m <= 128 (at m <= 64 only with n < 2048): the fewest
