@@ -639,6 +639,13 @@ int xpuint8_linear_gemm_stream(const void* stream, const int8_t* xq, const float
                     "linear_gemm");
 }
 
+// The shapes of linear_gemm_tiled: the persistent kernel's, whatever their slices (on
+// a device of few CUs a product can have both), and the split-K kernel's without
+static bool reads_block_layout(int64_t M, int64_t N, int64_t K) {
+    return pp_applies(int(M), int(N), int(K), false) ||
+           (splitk_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0);
+}
+
 int xpuint8_linear_gemm_tiled_stream(const void* stream, const int8_t* xq, const float* x_scale,
                                      const int8_t* w8, const float* w_scale, const void* bias,
                                      int32_t bias_bf16, void* out, int64_t M, int64_t N,
@@ -654,7 +661,7 @@ int xpuint8_linear_gemm_tiled_stream(const void* stream, const int8_t* xq, const
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
     hipStream_t st = as_stream(stream);
-    if (xt_applies(int(M), int(N), int(K)) && gemm_slices(int(M), int(N), int(K)) == 0)
+    if (reads_block_layout(M, N, K))
         return launched(gemm_dequant_xt(st, xq, w8, K, out, N, x_scale, w_scale, b32, b16,
                                         int(M), int(N), int(K)),
                         "linear_gemm_tiled");
@@ -784,8 +791,7 @@ int xpuint8_linear_gemm_packed_stream(const void* stream, const int8_t* xq, cons
     const float* b32 = bias_bf16 ? nullptr : static_cast<const float*>(bias);
     const uint16_t* b16 = bias_bf16 ? static_cast<const uint16_t*>(bias) : nullptr;
     hipStream_t st = as_stream(stream);
-    if (gemm_slices(int(M), int(N), int(K)) == 0 &&
-        (M <= 64 || xt_applies(int(M), int(N), int(K))))
+    if (reads_block_layout(M, N, K) || (M <= 64 && gemm_slices(int(M), int(N), int(K)) == 0))
         return launched(gemm_dequant_packed(st, xq, w8_packed, out, N, x_scale, w_scale, b32, b16,
                                             int(M), int(N), int(K)),
                         "linear_gemm_packed");
