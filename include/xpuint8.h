@@ -484,6 +484,17 @@ int xpuint8_linear_dx_stream(const void *stream, const void *dy, const void *w, 
 int64_t xpuint8_linear_dx_split_workspace_size(int64_t M, int64_t N, int64_t K);
 int64_t xpuint8_linear_dx_workspace_size(int64_t M, int64_t N, int64_t K);
 
+/* Which kernel and tile a product takes on the current device (one of 256 CUs
+ * before its first use; no device needed): the choice its launch makes, so that
+ * tests and profiles can name it.  product: 0 linear (dequant or residual), 1
+ * linear_acc, 3-5 the up-projection [M, N] with that activation, each of a
+ * quantized x and a packed weight; 6 linear_dx, 7 linear_dw, with the workspace
+ * their size entries name (M, N, K as there).  choice (host memory, four values):
+ * the kernel (0 skinny, 1 K split over a block's waves, 2 split K, 3
+ * persistent), its tile (rows; columns, or weight rows), and the slices of the
+ * contraction.  No reference counterpart. */
+int xpuint8_gemm_choice(int32_t product, int64_t M, int64_t N, int64_t K, int32_t *choice);
+
 /* RMSNorm + rotary embedding of q or k read straight from the int32
  * accumulator of a quantized qkv projection (one [B,S,H,D] slice of it):
  *   x = bf16(float(acc) * (w_scale[h*D+d] * x_scale[b,s])),

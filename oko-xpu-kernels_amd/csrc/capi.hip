@@ -1091,6 +1091,18 @@ int xpuint8_linear_backward_dense_stream(const void* stream, const void* dy, con
                     "linear_backward_dense (gemm)");
 }
 
+int xpuint8_gemm_choice(int32_t product, int64_t M, int64_t N, int64_t K, int32_t* choice) {
+    XPU_TRY(product == 6 || product == 7 ? check_linear_dx(M, N, K) : check_gemm(M, N, K));
+    if (product < 0 || product == 2 || product > 7)
+        return fail(6, "gemm_choice: product must be 0, 1 or 3..7");
+    if (!choice) return fail(6, "choice must not be null");
+    const GemmChoice c = product == 6   ? bf16_choice(int(M), int(K), int(N), false)
+                         : product == 7 ? bf16_choice(int(N), int(K), int(M), true)
+                                        : packed_choice(int(M), int(N), int(K), product);
+    choice[0] = c.kernel, choice[1] = c.rows, choice[2] = c.cols, choice[3] = c.slices;
+    return 0;
+}
+
 // ------------------------------------------------------------- rms + rope
 int xpuint8_rms_rope_dequant_stream(const void* stream, const int32_t* acc, int64_t acc_stride_b,
                                     int64_t acc_stride_s, int64_t acc_stride_h,

@@ -400,6 +400,15 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_splitk_kernel(
     else finish(std::integral_constant<int, 1>{});
 }
 
+// fragments b = 0 .. COUNT-1 of a plainly read operand, 1 KB apart
+template <int COUNT, int I = 0, int NF>
+__device__ __forceinline__ void plain_read_frags(v8s (&f)[NF], uint32_t addr) {
+    if constexpr (I < COUNT) {
+        f[I] = plain_read_at<I * 1024>(addr);
+        plain_read_frags<COUNT, I + 1>(f, addr);
+    }
+}
+
 // ------------------------------------------------------------ large outputs
 // Products with at least a round of large tiles: the persistent ping-pong
 // scheme of the int8 GEMM in bf16, one block of 8 waves per CU over BB x BC
@@ -434,15 +443,6 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_splitk_kernel(
 // (float*)out + blockIdx.y * sl_stride instead of the bf16 output.
 // Off: the lanes' byte offsets from a block's first row, at most 15 rows
 // (uint32_t; uint64_t for leading dimensions past 2^27).
-// fragments b = 0 .. COUNT-1 of a plainly read operand, 1 KB apart
-template <int COUNT, int I = 0, int NF>
-__device__ __forceinline__ void plain_read_frags(v8s (&f)[NF], uint32_t addr) {
-    if constexpr (I < COUNT) {
-        f[I] = plain_read_at<I * 1024>(addr);
-        plain_read_frags<COUNT, I + 1>(f, addr);
-    }
-}
-
 template <int BB, int BC, int WGM, bool YT, bool SL, class Off = uint32_t>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_pp_kernel(
     const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ Y, int64_t ldy,
@@ -870,6 +870,13 @@ int64_t bf16_dw_work_bytes(int R, int N, int K) {
     if (bf16_splitk_applies(N, 160, R, K, K, N, true)) return 0;
     const int n = bf16_plan(N, K, R, true, int64_t(1) << 62).slices;
     return n > 1 ? int64_t(n) * N * K * 4 : 0;
+}
+
+GemmChoice bf16_choice(int nbr, int nc, int R, bool yt) {
+    if (bf16_splitk_applies(nbr, yt ? 160 : 128, R, nc, nc, yt ? nbr : R, yt))
+        return GemmChoice{kSplitKKernel, yt ? 160 : 128, 160, 1};
+    const Bf16Plan p = bf16_plan(nbr, nc, R, yt, int64_t(1) << 62);
+    return GemmChoice{kPersistentKernel, kBf16Tiles[p.tile].bb, kBf16Tiles[p.tile].bc, p.slices};
 }
 
 // out[b, c] = sum over r of a[r, c] * y (y[b, r], or y[r, b] with YT) on the

@@ -982,8 +982,8 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     const int g = wm / (WGM / 2);                               // group: the row half
-    // issues PER loads per step, else PER - 1 (REM = 4: group 0 and group 1)
-    const bool full_share = REM == 0 || (REM == 4 ? g == 0 : wave < REM);
+    static_assert(REM == 0 || REM == 4, "group 0 issues PER, group 1 PER or PER - 1");
+    const bool full_share = REM == 0 || g == 0;                 // PER loads per step, else PER - 1
 
     // tile origin of sequence number i: each XCD (i % 8, as blockIdx % 8)
     // takes a contiguous eighth of the tiles (rounded up: the last XCDs may
@@ -2389,31 +2389,42 @@ struct IsActEpi : std::false_type {};
 template <class Epi>
 struct IsActEpi<Epi, std::void_t<decltype(Epi::kWinTab)>> : std::true_type {};
 
-// X and W both in the block layout, unpaired epilogues
+// The kernel and its tile (an index into the kernel's list) for a product
+struct TileChoice {
+    int kernel, tile;           // GemmKernel
+};
+// X and W both in the block layout, unpaired epilogues (splitk: one that has the
+// split-K form)
+inline TileChoice choose_tiles(int M, int N, int K, bool splitk) {
+    const int64_t cus = device_cus();
+    double t = 0;
+    TileChoice c{kPersistentKernel, pp_tile(kPpModel, kPpTiles, false, M, N, K, cus, &t)};
+    if (splitk) {
+        const double ts = 1.03 * splitk_time(M, N, K, cus);
+        if (ts < t) c = TileChoice{kSplitKKernel, 0}, t = ts;
+    }
+    const int w = wavek_tile(kWavekModel, kWavekTiles, 1.06, M, N, K, N, cus, &t);
+    return w < 0 ? c : TileChoice{kWavekKernel, w};
+}
 template <class Epi>
 hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N, int K,
                         const Epi& epi) {
     constexpr bool kSplitK = Epi::kStaged && !IsActEpi<Epi>::value;
-    const int64_t cus = device_cus();
-    double t = 0;
-    const int tile = pp_tile(kPpModel, kPpTiles, false, M, N, K, cus, &t);
-    bool splitk = false;
-    if constexpr (kSplitK) {
-        const double ts = 1.03 * splitk_time(M, N, K, cus);
-        if (ts < t) splitk = true, t = ts;
-    }
-    switch (wavek_tile(kWavekModel, kWavekTiles, 1.06, M, N, K, N, cus, &t)) {
-        case 0: return launch_wavek<1, 1, 8, 4>(st, Xt, Wp, M, N, K, epi);
-        case 1: return launch_wavek<1, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
-        case 2: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
-        case 3: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
-        case 4: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
-        default: break;
+    const TileChoice c = choose_tiles(M, N, K, kSplitK);
+    if (c.kernel == kWavekKernel) {
+        switch (c.tile) {
+            case 0: return launch_wavek<1, 1, 8, 4>(st, Xt, Wp, M, N, K, epi);
+            case 1: return launch_wavek<1, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+            case 2: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+            case 3: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
+            default: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
+        }
     }
     if constexpr (kSplitK) {
-        if (splitk) return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
+        if (c.kernel == kSplitKKernel)
+            return launch_splitk<false, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
     }
-    switch (tile) {
+    switch (c.tile) {
         case 0: return launch_pp<true, true, 256, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 1: return launch_pp<true, true, 192, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 2: return launch_pp<true, true, 192, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
@@ -2438,23 +2449,36 @@ hipError_t launch_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int 
 constexpr PpTile kPairTiles[] = {{256, 320}, {256, 256}, {192, 256}, {128, 256}, {128, 192}};
 constexpr WavekTile kPairWavekTiles[] = {
     {1, 2, 8, 4, 3}, {2, 2, 4, 4, 5}, {2, 4, 4, 4, 3}, {4, 4, 4, 2, 2}};
-template <class Epi>
-hipError_t launch_pair_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N,
-                             int K, bool situ, const Epi& epi) {
-    if (M <= 16) return launch_skinny<4, Epi, true, true>(st, Xt, 0, Wp, 0, M, N, K, epi);
+inline TileChoice choose_pair_tiles(int M, int N, int K, bool situ) {
+    if (M <= 16) return TileChoice{kSkinnyKernel, 0};
     const PpModel pm = {4.05, 0.0771, 0.1875, 0.76, situ ? 1.76 : 0.85, 0.77};
     const WavekModel wm = {1.88, 0.0058, 0.42, (situ ? 0.32 : 0.236) / 16, 0.084e-6};
     const int64_t cus = device_cus();
     double t = 0;
     const int tile = pp_tile(pm, kPairTiles, true, M, N, K, cus, &t);
-    switch (wavek_tile(wm, kPairWavekTiles, 1.03, M, 2 * int64_t(N), K, N, cus, &t)) {
-        case 0: return launch_wavek<1, 2, 8, 4>(st, Xt, Wp, M, N, K, epi);
-        case 1: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
-        case 2: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
-        case 3: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
-        default: break;
+    const int w = wavek_tile(wm, kPairWavekTiles, 1.03, M, 2 * int64_t(N), K, N, cus, &t);
+    return w < 0 ? TileChoice{kPersistentKernel, tile} : TileChoice{kWavekKernel, w};
+}
+template <class Epi>
+hipError_t launch_pair_tiles(hipStream_t st, const int8_t* Xt, const int8_t* Wp, int M, int N,
+                             int K, bool situ, const Epi& epi) {
+    const TileChoice c = choose_pair_tiles(M, N, K, situ);
+    if (c.kernel == kSkinnyKernel) {
+        // one row block, two output column blocks and four waves a block
+        hipLaunchKernelGGL((gemm_i8_skinny_kernel<1, 4, 4, Epi, true, true>),
+                           dim3(unsigned((N + 31) / 32)), dim3(256), 0, st, Xt, 0, Wp, 0, M, N, K,
+                           epi);
+        return hipGetLastError();
     }
-    switch (tile) {
+    if (c.kernel == kWavekKernel) {
+        switch (c.tile) {
+            case 0: return launch_wavek<1, 2, 8, 4>(st, Xt, Wp, M, N, K, epi);
+            case 1: return launch_wavek<2, 2, 4, 4>(st, Xt, Wp, M, N, K, epi);
+            case 2: return launch_wavek<2, 4, 4, 4>(st, Xt, Wp, M, N, K, epi);
+            default: return launch_wavek<4, 4, 4, 2>(st, Xt, Wp, M, N, K, epi);
+        }
+    }
+    switch (c.tile) {
         case 0: return launch_pp<true, true, 256, 320>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 1: return launch_pp<true, true, 256, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
         case 2: return launch_pp<true, true, 192, 256>(st, Xt, 0, Wp, 0, M, N, K, epi);
@@ -2812,14 +2836,36 @@ hipError_t gemm_dequant_xt(hipStream_t st, const int8_t* At, const int8_t* B, in
 
 bool xt_applies(int M, int N, int K) { return splitk_applies(M, N, K) || pp_applies(M, N, K, false); }
 
+// 33-64 rows of a narrow, long product have too few 16-column blocks for the
+// skinny kernel (those whose row-major form is split in K across blocks)
+static bool packed_skinny(int M, int N, int K) { return M <= 64 && skinny_slices(M, N, K) == 0; }
+
 template <class Epi>
 static hipError_t packed_gemm(hipStream_t st, const int8_t* At, const int8_t* Bp, int M, int N,
                               int K, const Epi& epi) {
-    // 33-64 rows of a narrow, long product have too few 16-column blocks for the
-    // skinny kernel (those whose row-major form is split in K across blocks)
-    if (M <= 64 && skinny_slices(M, N, K) == 0)
+    if (packed_skinny(M, N, K))
         return launch_skinny<1, Epi, true, true>(st, At, 0, Bp, 0, M, N, K, epi);
     return launch_tiles(st, At, Bp, M, N, K, epi);
+}
+
+GemmChoice packed_choice(int M, int N, int K, int epilogue) {
+    const bool paired = act_paired(epilogue);
+    TileChoice c{kSkinnyKernel, 0};
+    if (paired) c = choose_pair_tiles(M, N, K, epilogue == 3);
+    else if (!(epilogue == 5 ? M <= 64 : packed_skinny(M, N, K)))
+        c = choose_tiles(M, N, K, epilogue == 0);
+    switch (c.kernel) {
+        case kWavekKernel: {
+            const WavekTile& t = paired ? kPairWavekTiles[c.tile] : kWavekTiles[c.tile];
+            return GemmChoice{c.kernel, 16 * t.mb, 16 * t.nb, 1};
+        }
+        case kPersistentKernel: {
+            const PpTile& t = paired ? kPairTiles[c.tile] : kPpTiles[c.tile];
+            return GemmChoice{c.kernel, t.bm, t.bn, 1};
+        }
+        case kSplitKKernel: return GemmChoice{c.kernel, 128, 160, 1};
+        default: return GemmChoice{c.kernel, (M + 15) / 16 * 16, paired ? 64 : 16, 1};
+    }
 }
 
 hipError_t gemm_dequant_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, void* out,

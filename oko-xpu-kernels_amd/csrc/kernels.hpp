@@ -133,6 +133,17 @@ hipError_t gemm_i32_pp_xt(hipStream_t st, const int8_t* At, const int8_t* B, int
                           int32_t* C, int64_t ldc, int M, int N, int K);
 hipError_t gemm_i32_packed(hipStream_t st, const int8_t* At, const int8_t* Bp, int32_t* C,
                            int64_t ldc, int M, int N, int K);
+// Which kernel and tile a product takes on the current device: the choice that its
+// launch makes, for tests and profiles (xpuint8_gemm_choice)
+enum GemmKernel : int { kSkinnyKernel = 0, kWavekKernel = 1, kSplitKKernel = 2, kPersistentKernel = 3 };
+struct GemmChoice {
+    int kernel, rows, cols, slices;
+};
+// of x and a packed weight: epilogue 0 dequant or residual, 1 int32, 3-5 an activation
+GemmChoice packed_choice(int M, int N, int K, int epilogue);
+// out[b, c] of the bf16 products (gemm_bf16_nn, yt: gemm_bf16_tn), contraction R, with
+// the workspace that it would like
+GemmChoice bf16_choice(int nbr, int nc, int R, bool yt);
 // the same products of x itself, bf16 [M, K], quantized in the same launch (callers
 // check rowq_applies; out must not overlap x); xs: its row scales, written
 bool rowq_applies(int M, int K);

@@ -126,6 +126,7 @@ def _signatures():
         "xpuint8_linear_dx_stream": ([vp] * 4 + [i64] * 3 + [vp, i64], c_int),
         "xpuint8_linear_dx_workspace_size": ([i64] * 3, i64),
         "xpuint8_linear_dx_split_workspace_size": ([i64] * 3, i64),
+        "xpuint8_gemm_choice": ([i32] + [i64] * 3 + [vp], c_int),
         "xpuint8_rms_rope_dequant_stream": ([vp, vp] + [i64] * 3 + [vp] + [i64] * 2 + [vp, vp]
                                             + [i64] * 7 + [vp, vp] + [i64] * 4
                                             + [ctypes.c_float, i32], c_int),

@@ -29,24 +29,64 @@ def operand(rows, cols, std, seed, dev):
     return (torch.randn(rows, cols, generator=g, device=dev) * std).to(torch.bfloat16)
 
 
-# (M, N, K): 256x320 (one round, 1040 % 32 = 16), 192x256 (one; several), 128x256 (two
-# slices), 128x192 (one tile row; two, three slices), 128x128 (a single short step;
-# one slice; four, six and eight slices with a ragged last one)
-@pytest.mark.parametrize("m,n,k", [(3800, 1040, 5120), (3000, 3072, 3072), (2500, 528, 2576),
-                                   (3665, 7056, 1024), (1500, 1040, 2000), (40, 16, 272),
-                                   (1206, 848, 768), (322, 5648, 2048), (205, 2672, 768),
-                                   (1166, 3824, 1024), (129, 80, 16), (300, 4112, 528)])
+# (M, N, K) and the kernel, tile and contraction slices that it takes (checked in
+# test_kernel_choice.py): every tile of the persistent kernel in one round and, where
+# a product can have them, in several, whole and in slices, with ragged rows and
+# columns, contractions that end inside a 32-row step (1040, 3824) or a slice and one
+# of a single short step; and the split-K kernel
+DX_SHAPES = {
+    (3800, 1040, 5120): ("persistent", 256, 320, 1),    # 240 tiles
+    (2500, 1040, 10240): ("persistent", 256, 320, 1),    # 320 tiles
+    (3000, 3072, 3072): ("persistent", 192, 256, 1),    # 192 tiles
+    (3969, 224, 5280): ("persistent", 192, 256, 1),    # 441 tiles
+    (2500, 528, 2576): ("persistent", 128, 256, 1),    # 220 tiles
+    (2394, 128, 2512): ("persistent", 128, 256, 1),    # 190 tiles
+    (3665, 7056, 1024): ("persistent", 128, 256, 2),    # 232 tiles
+    (130, 7168, 3328): ("persistent", 128, 256, 8),    # 208 tiles
+    (3798, 128, 1184): ("persistent", 128, 192, 1),    # 210 tiles
+    (2346, 288, 4896): ("persistent", 128, 192, 1),    # 494 tiles
+    (561, 2080, 3216): ("persistent", 128, 192, 2),    # 170 tiles
+    (129, 1936, 5440): ("persistent", 128, 192, 4),    # 232 tiles
+    (1500, 1040, 2000): ("persistent", 128, 128, 1),    # 192 tiles
+    (40, 16, 272): ("persistent", 128, 128, 1),    # 3 tiles
+    (1206, 848, 768): ("persistent", 128, 128, 1),    # 60 tiles
+    (129, 80, 16): ("persistent", 128, 128, 1),    # 2 tiles
+    (322, 5648, 2048): ("persistent", 128, 128, 5),    # 240 tiles
+    (205, 2672, 768): ("persistent", 128, 128, 8),    # 96 tiles
+    (1166, 3824, 1024): ("persistent", 128, 128, 3),    # 240 tiles
+    (300, 4112, 528): ("persistent", 128, 128, 8),    # 120 tiles
+    (390, 2080, 5120): ("splitk", 128, 160, 1),    # 128 tiles
+}
+# the contraction over M: batches of 1, of 17 and odd ones
+DW_SHAPES = {
+    (267, 3856, 3584): ("persistent", 256, 256, 1),    # 224 tiles
+    (1001, 5120, 5120): ("persistent", 256, 256, 1),    # 400 tiles
+    (103, 1648, 4944): ("persistent", 192, 256, 1),    # 180 tiles
+    (373, 8544, 2816): ("persistent", 192, 256, 1),    # 495 tiles
+    (1585, 2480, 3072): ("persistent", 128, 256, 1),    # 240 tiles
+    (105, 3136, 4944): ("persistent", 128, 256, 1),    # 500 tiles
+    (2129, 2768, 768): ("persistent", 128, 256, 3),    # 198 tiles
+    (3077, 160, 4720): ("persistent", 128, 256, 6),    # 228 tiles
+    (615, 4896, 1024): ("persistent", 128, 192, 1),    # 234 tiles
+    (105, 3712, 4432): ("persistent", 128, 192, 1),    # 696 tiles
+    (3009, 976, 2816): ("persistent", 128, 192, 2),    # 240 tiles
+    (1407, 160, 5408): ("persistent", 128, 192, 4),    # 232 tiles
+    (17, 48, 144): ("persistent", 128, 128, 1),    # 2 tiles
+    (1, 160, 272): ("persistent", 128, 128, 1),    # 6 tiles
+    (33, 16, 16): ("persistent", 128, 128, 1),    # 1 tiles
+    (2893, 544, 768): ("persistent", 128, 128, 7),    # 210 tiles
+    (1971, 672, 512): ("persistent", 128, 128, 7),    # 168 tiles
+    (2112, 1680, 2000): ("splitk", 160, 160, 1),    # 143 tiles
+}
+
+
+@pytest.mark.parametrize("m,n,k", list(DX_SHAPES))
 def test_linear_dx_tiles(dev, m, n, k):
     dy, w = operand(m, n, 1e-3, m, dev), operand(n, k, 0.02, n + k, dev)
     check(int8.linear_dx(dy, w), dy, w)
 
 
-# (M, N, K), the contraction over M: 256x256, 192x256, 128x256, 128x192 (a batch of
-# 1, of 17 and odd ones), 128x128 whole and in slices
-@pytest.mark.parametrize("m,n,k", [(267, 3856, 3584), (1001, 5120, 5120), (373, 8544, 2816),
-                                   (1585, 2480, 3072), (615, 4896, 1024), (17, 48, 144),
-                                   (1, 160, 272), (2893, 544, 768), (2129, 2768, 768),
-                                   (3009, 976, 2816), (1971, 672, 512), (33, 16, 16)])
+@pytest.mark.parametrize("m,n,k", list(DW_SHAPES))
 def test_linear_dw_tiles(dev, m, n, k):
     dy, x = operand(m, n, 1e-3, m, dev), operand(m, k, 1.0, n + k, dev)
     check(int8.linear_dw(dy, x), dy.t(), x)

@@ -24,21 +24,41 @@ def reference(x, w8, ws, bias, res=None, rscale=None):
     return acc, y if res is None else torch.addcmul(res, y, rscale)
 
 
-# (M, N, K): the persistent kernel's 256x320 (one round), 192x320 (one and two
-# rounds), 192x256 (one and two), 192x192 (one, a long K; two), 128x192 (one; four);
-# split K (a long K)
-PP_SHAPES = [(4090, 5104, 2048), (1050, 10912, 256), (3000, 10240, 1280), (3974, 3072, 3072),
-             (1355, 6160, 256), (2060, 9232, 1280), (920, 6224, 256), (1541, 3856, 5120),
-             (2323, 6144, 256), (1251, 4752, 3072), (2147, 11024, 256), (4090, 1264, 6144)]
-# the K-split-over-waves kernel's 16x16 (one row block and one column block past
-# the batch; fewer K steps than waves; a long K at 33 rows), 16x32, 32x32, 32x64
-# and 64x64 tiles, each with ragged rows and columns
-WAVEK_SHAPES = [(65, 16, 256), (129, 208, 256), (35, 320, 5120), (64, 1280, 5120),
-                (525, 976, 2048), (438, 496, 1024), (135, 992, 3840), (1000, 1296, 1280),
-                (700, 2064, 6144), (400, 1936, 2048), (1218, 624, 6400), (449, 1696, 256)]
+# (M, N, K) and the kernel and tile that the dequant product takes (checked in
+# test_kernel_choice.py): the persistent kernel's five tiles in one round and in
+# several, split K (a long K), and the tiles of the kernel that splits K over a
+# block's waves (one row block and one column block past the batch; fewer K steps
+# than waves; a long K at 33 rows), each with ragged rows and columns.  linear_acc takes
+# the same, but for split K, which has no int32 form
+SHAPES = {
+    (4090, 5104, 2048): ("persistent", 256, 320),
+    (1050, 10912, 256): ("persistent", 192, 320),
+    (3000, 10240, 1280): ("persistent", 192, 320),
+    (3974, 3072, 3072): ("persistent", 192, 256),
+    (1355, 6160, 256): ("persistent", 192, 256),
+    (2060, 9232, 1280): ("persistent", 192, 256),
+    (920, 6224, 256): ("persistent", 192, 192),
+    (1541, 3856, 5120): ("persistent", 192, 192),
+    (2323, 6144, 256): ("persistent", 192, 192),
+    (1251, 4752, 3072): ("persistent", 128, 192),
+    (2147, 11024, 256): ("persistent", 128, 192),
+    (4090, 1264, 6144): ("splitk", 128, 160),
+    (65, 16, 256): ("wavek", 16, 16),
+    (129, 208, 256): ("wavek", 16, 16),
+    (35, 320, 5120): ("wavek", 16, 16),
+    (64, 1280, 5120): ("wavek", 16, 32),
+    (525, 976, 2048): ("wavek", 16, 32),
+    (438, 496, 1024): ("wavek", 32, 32),
+    (135, 992, 3840): ("wavek", 32, 32),
+    (1000, 1296, 1280): ("wavek", 32, 64),
+    (700, 2064, 6144): ("wavek", 32, 64),
+    (400, 1936, 2048): ("wavek", 64, 64),
+    (1218, 624, 6400): ("wavek", 64, 64),
+    (449, 1696, 256): ("wavek", 64, 64),
+}
 
 
-@pytest.mark.parametrize("m,n,k", PP_SHAPES + WAVEK_SHAPES)
+@pytest.mark.parametrize("m,n,k", list(SHAPES))
 def test_packed_tiles_exact(dev, m, n, k):
     w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
     x = activation(m, k, seed=m + k).to(dev)
@@ -53,15 +73,23 @@ def test_packed_tiles_exact(dev, m, n, k):
     assert torch.equal(int8.linear(x, w8, ws, bias, residual=res, residual_scale=rscale), yr)
 
 
-# The FFN's up-projection, (M, inner, K): the paired 256x320 tile (a ragged batch),
-# 256x256, 192x256, 128x256 and 128x192, the wave-split 64x64, 32x64, 32x32 and 16x32,
-# and the skinny kernel's 16 rows
-FFN_SHAPES = [(4090, 5120, 512), (2315, 2560, 256), (892, 5376, 512), (514, 5120, 256),
-              (357, 4608, 256), (304, 1280, 512), (45, 2816, 256), (33, 1536, 256), (19, 512, 256),
-              (16, 1024, 512)]
+# The FFN's up-projection, (M, inner, K): what its product takes for the paired
+# activations (a ragged batch in each) and for GELU
+FFN_SHAPES = {
+    (4090, 5120, 512): (("persistent", 256, 320), ("persistent", 256, 320)),
+    (2315, 2560, 256): (("persistent", 256, 256), ("persistent", 192, 192)),
+    (892, 5376, 512): (("persistent", 192, 256), ("persistent", 128, 192)),
+    (514, 5120, 256): (("persistent", 128, 256), ("persistent", 128, 192)),
+    (357, 4608, 256): (("persistent", 128, 192), ("wavek", 64, 64)),
+    (304, 1280, 512): (("wavek", 64, 64), ("wavek", 32, 64)),
+    (45, 2816, 256): (("wavek", 32, 64), ("skinny", 48, 16)),
+    (33, 1536, 256): (("wavek", 32, 32), ("skinny", 48, 16)),
+    (19, 512, 256): (("wavek", 16, 32), ("skinny", 32, 16)),
+    (16, 1024, 512): (("skinny", 16, 64), ("skinny", 16, 16)),
+}
 
 
-@pytest.mark.parametrize("m,inner,k", FFN_SHAPES)
+@pytest.mark.parametrize("m,inner,k", list(FFN_SHAPES))
 @pytest.mark.parametrize("act", ["situ", "geglu_erf", "gelu_erf"])
 def test_ffn_packed_tiles_exact(dev, act, m, inner, k):
     """Against the library's unfused chain (int32 product, the row kernel that
