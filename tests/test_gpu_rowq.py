@@ -77,6 +77,55 @@ def test_rowq_ffn_exact(dev, m, f, k, act):
     assert torch.equal(int8.ffn(x, up8, ups, down8, downs, b, act=act), want)
 
 
+def same(a, b):
+    """Equal but for the payload of NaNs."""
+    nan = a.isnan()
+    return torch.equal(nan, b.isnan()) and torch.equal(a[~nan], b[~nan])
+
+
+def non_finite_rows(m, k, dev):
+    x = activation(m, k, seed=m + k).to(dev)
+    x[0, 7] = float("inf")
+    if m > 1:
+        x[1, 3] = float("nan")
+    if m > 2:
+        x[2, 0], x[2, k - 1] = float("inf"), -float("inf")
+    return x
+
+
+# 4, 8 and 16 waves, two groups a lane's segment, two weight blocks a block
+@pytest.mark.parametrize("m,n,k", [(1, 1280, 1280), (3, 1296, 2560), (16, 208, 1024), (2, 8224, 4096),
+                                   (11, 8240, 768)])
+def test_rowq_non_finite(dev, m, n, k):
+    """Rows with infinities and NaN: what the separate quantizer and product give, in
+    those rows and in the others, which share their waves."""
+    w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
+    x = non_finite_rows(m, k, dev)
+    acc, y, xs = product(x, w8, ws)
+    got, gxs = int8.linear_acc(x, w8, ws)
+    assert torch.equal(got, acc) and same(gxs, xs)
+    assert same(int8.linear(x, w8, ws), y.to(torch.bfloat16))
+    assert same(int8.linear(x, w8.clone(), ws), y.to(torch.bfloat16))
+
+
+# the up-projection that quantizes its rows, K split over waves, and the persistent
+# kernel with its tables in LDS windows (256x256, 192x256 and GELU's 192x192)
+@pytest.mark.parametrize("act", ["situ", "geglu_erf", "gelu_erf"])
+@pytest.mark.parametrize("m,f,k", [(6, 768, 1280), (304, 1280, 512), (892, 5376, 512),
+                                   (2315, 2560, 256)])
+def test_ffn_non_finite(dev, m, f, k, act):
+    """The same through an FFN: a row scale that is no number in the epilogues'
+    activations, against the unfused chain."""
+    up8, ups = int8.prepare_weight(weight((1 if act == "gelu_erf" else 2) * f, k, seed=f).to(dev))
+    down8, downs = int8.prepare_weight(weight(k, f, seed=k).to(dev))
+    ups[3], ups[f - 1] = float("inf"), float("nan")
+    x = non_finite_rows(m, k, dev)
+    acc, xs = int8.linear_acc(x, up8, ups)
+    q, s = int8.dequant_act_quantize(acc, xs, ups, act)
+    want = int8.dequant(int8.int_mm(q, down8.t()), s, downs)
+    assert same(int8.ffn(x, up8, ups, down8, downs, act=act), want)
+
+
 def test_rowq_output_over_x(dev):
     lib = L._lib()
     m, k = 4, 1024
