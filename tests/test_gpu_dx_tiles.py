@@ -23,7 +23,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(2060, 2064, 1280), (2180, 1104, 2560),                # split K; 16 * 16 + 16 tiles more
           (33, 528, 256), (65, 1040, 512), (130, 48, 256), (300, 2608, 768), (1273, 528, 512),
           (24, 16, 256), (23, 16, 256), (1, 16, 512), (7, 1296, 256), (16, 64, 256),
-          (3, 32784, 256), (70, 33024, 256)]
+          # N > 32768: whole; in contraction slices through the transposed weight (M <=
+          # 256) and on the weight as stored
+          (3, 32784, 256), (70, 33024, 256), (300, 33024, 256)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
@@ -44,6 +46,21 @@ def test_dx_int8_by_shape_exact(dev, m, n, k):
         want = O.linear_dx_int8(bits(dy), npy(w8), npy(ws))
         assert np.array_equal(got, want), mismatch(got, want)
         assert bool((guard[m * k:] == 7.0).all())
+
+
+def test_dx_int8_long_rows_unsplit(dev):
+    """N > 32768 with enough tiles for the split-K kernel, row-major dy codes and the
+    weight as stored: the row quantizer's codes, the exact product in float64 and
+    the inverse rotation, each checked elsewhere."""
+    m, n, k = 2060, 33024, 1280
+    g = torch.Generator(device=dev).manual_seed(5)
+    w8 = torch.randint(-127, 128, (n, k), generator=g, device=dev, dtype=torch.int8)
+    ws = torch.rand(n, generator=g, device=dev) * 1e-2 + 1e-4
+    dy = (torch.randn(m, n, generator=g, device=dev) * 1e-3).to(torch.bfloat16)
+    q, a = int8.quantize_row(dy, ws)
+    acc = (q.double() @ w8.double()).to(torch.int32)
+    want = int8.rotate((acc.float() * a[:, None]).to(torch.bfloat16))
+    assert torch.equal(int8.linear_dx_int8(dy, w8, ws), want)
 
 
 # one round of the split-K kernel (which reads the second packed form); more rounds,

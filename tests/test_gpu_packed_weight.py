@@ -1,10 +1,8 @@
 """The packed weight (``pack_weight``; ``xpuint8_pack_weight_stream``): its
 bytes against a torch restatement of the MFMA block layout, and every GEMM
-that reads it -- the persistent kernel (config 3's shape and a ragged batch),
-the split-K kernel (the N = 1280 shapes, a ragged one), both projections of
-the FFN -- bit for bit the row-major weight's result and the oracle's; shapes
-whose GEMMs read the weight row-major (K slices, the skinny kernel) through
-the packed entry point; and the rules that decide when the copy is used (an
+that reads it (at large and ragged shapes of the persistent and split-K kernels, at
+small batches, in both projections of the FFN) bit for bit the row-major
+weight's result and the oracle's; and the rules that decide when the copy is used (an
 in-place write, an alias, an offset view, a module's weight moved or written,
 a storage that is freed)."""
 
@@ -73,11 +71,12 @@ def _both(dev, n, k, seed):
     return w8p, w8r, ws
 
 
-# (M, N, K): the persistent kernel (config 3; a batch that is not a multiple
-# of 256), the split-K kernel (the SDXL N = 1280 shapes; ragged rows and a
-# last column tile of 16), K slices (M = 200, 512; M = 48 at N < 2048) and the
-# skinny kernel reading the packed weight (M = 1, 7, 16, 48 at N >= 2048, 64;
-# the row counts one m-block to four, N = 1296 a last weight block alone)
+# (M, N, K), row-major weights on the persistent kernel (config 3; a batch that is
+# not a multiple of 256), the split-K kernel (the SDXL N = 1280 shapes; ragged
+# rows and a last column tile of 16), K slices (M = 200, 512; M = 48 at N < 2048)
+# and the skinny kernel (M = 1, 7, 16, 48 at N >= 2048, 64; the row counts one
+# m-block to four, N = 1296 a last weight block alone), each against the kernel
+# that the packed weight takes there
 LINEAR_SHAPES = [(4096, 10240, 1280), (3000, 10240, 1280), (4096, 1280, 5120),
                  (4096, 1280, 2048), (4096, 1280, 1280), (2100, 1296, 2048), (200, 1280, 4096),
                  (512, 4096, 4096), (16, 4096, 4096), (1, 4096, 4096), (7, 1296, 2048),
@@ -320,9 +319,9 @@ def test_int8_linear_backward_packed(dev):
 
 
 # linear with the residual update and linear_acc, each one library call that
-# quantizes into the layout its GEMM reads: the persistent kernel (config 3;
-# a ragged batch), the split-K kernel, and a batch whose GEMM reads the
-# activation row-major (K slices)
+# quantizes into the layout its GEMM reads; from a row-major weight the persistent
+# kernel (config 3; a ragged batch), the split-K kernel, and a batch whose GEMM
+# reads the activation row-major (K slices)
 ONE_CALL_SHAPES = [(4096, 10240, 1280), (3000, 10240, 1280), (4096, 1280, 5120), (200, 1280, 4096)]
 
 

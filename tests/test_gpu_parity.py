@@ -16,6 +16,7 @@ import oracle as O
 from gpu_util import activation, bits, from_bits, mismatch, npy, weight
 from xpu_kernels import int8
 from xpu_kernels.int8 import _lib as L
+from xpu_kernels.int8 import ops
 
 pytestmark = pytest.mark.gpu
 
@@ -534,11 +535,19 @@ def test_linear_one_call_exact(dev, m, n, k):
         assert np.array_equal(bits(out), want), (kind, mismatch(bits(out), want))
 
 
-# one shape per kernel the plain linear dispatches to (M <= 64: the skinny
-# kernel; few tiles: the 128 x 128 kernel; more: the two-block 256 x 160
-# kernel; a 256 x 320 tile per CU: the persistent kernel; narrow output with
+def packed_and_row_major(w8):
+    """A prepared weight with its packed copy and the same codes without one: the
+    two sets of kernels that a call can take."""
+    row_major = w8.clone()
+    assert ops._packed_for(w8) is not None and ops._packed_for(row_major) is None
+    return w8, row_major
+
+
+# one shape per kernel the plain linear dispatches to from a row-major weight (M <=
+# 64: the skinny kernel; few tiles: the 128 x 128 kernel; more: the two-block 256
+# x 160 kernel; a 256 x 320 tile per CU: the persistent kernel; narrow output with
 # a long K: split K over the block-layout activation), with ragged rows and
-# columns
+# columns; and the same shapes from the packed one
 @pytest.mark.parametrize("m,n,k", [(16, 528, 768), (64, 2048, 1024), (65, 1040, 512),
                                    (2000, 4000, 512), (4100, 5120, 256), (1500, 1920, 2048),
                                    (2050, 1296, 3072)])
@@ -548,18 +557,19 @@ def test_linear_dispatch_sweep(dev, m, n, k):
     w = weight(n, k, seed=n + 1)
     bias = weight(1, n, seed=n + k, std=0.01)[0]
     w8, ws = int8.prepare_weight(w.to(dev))
-    y = int8.linear(x.to(dev), w8, ws, bias.to(dev))
     want = O.linear(bits(x), npy(w8), npy(ws), O.bf16_to_f32(bits(bias)))
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for form in packed_and_row_major(w8):
+        y = int8.linear(x.to(dev), form, ws, bias.to(dev))
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
-# Too few 128 x 160 output tiles for the chip: the product split in K across
-# blocks (4, 4 and 4 slices through the split-K kernel; 32 and 2 through the
+# Too few 128 x 160 output tiles for the chip: from a row-major weight the product
+# split in K across blocks (4, 4 and 4 slices through the split-K kernel; 32 and 2 through the
 # 128 x 128 kernel for M <= 256; 2, 4, 4 and 2 through the skinny kernel for
 # 33 <= M <= 128, with 8, 4, 7 and 3 row blocks), the int32 partial sums
 # added by the dequant pass; ragged row and column tiles (1296 columns: a
 # half-empty last pair of weight blocks); with a bf16 bias, an fp32 bias and
-# none
+# none; and the same shapes from the packed weight
 @pytest.mark.parametrize("m,n,k", [(1024, 1280, 5120), (2048, 640, 5120), (1000, 1296, 4096),
                                    (200, 160, 16384), (128, 4096, 4096), (65, 4080, 1024),
                                    (64, 1280, 5120), (100, 1296, 5120), (33, 1040, 2048)])
@@ -570,14 +580,16 @@ def test_linear_k_slices_exact(dev, m, n, k):
     w8, ws = int8.prepare_weight(w.to(dev))
     acc, xs = O.linear_acc(bits(x), npy(w8))              # the oracle's linear, shared
     for b in (bias.to(dev), bias.float().to(dev), None):
-        y = int8.linear(x.to(dev), w8, ws, b)
         bref = None if b is None else O.bf16_to_f32(bits(bias))
         want = O.dequant(acc, xs, npy(ws), bref)
-        assert np.array_equal(bits(y), want), (None if b is None else b.dtype,
-                                               mismatch(bits(y), want))
+        for form in packed_and_row_major(w8):
+            y = int8.linear(x.to(dev), form, ws, b)
+            assert np.array_equal(bits(y), want), (None if b is None else b.dtype,
+                                                   mismatch(bits(y), want))
 
 
-# Each side of every threshold of the linear's GEMM choice: M = 32 / 33
+# Each side of every threshold of the linear's GEMM choice from a row-major weight
+# (and the same shapes from the packed one): M = 32 / 33
 # (skinny kernel / K slices on it), N = 2048 / 2032 at M = 64 (the skinny
 # kernel whole / in K slices), M = 64 / 65 at N = 2048 (skinny kernel / K
 # slices on it), M = 128 / 129 (slices on the skinny / 128 x 128 kernel), no
@@ -598,9 +610,10 @@ def test_linear_dispatch_boundaries(dev, m, n, k):
     w = weight(n, k, seed=n + 5)
     bias = weight(1, n, seed=n + k + 2, std=0.01)[0]
     w8, ws = int8.prepare_weight(w.to(dev))
-    y = int8.linear(x.to(dev), w8, ws, bias.to(dev))
     want = O.linear(bits(x), npy(w8), npy(ws), O.bf16_to_f32(bits(bias)))
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for form in packed_and_row_major(w8):
+        y = int8.linear(x.to(dev), form, ws, bias.to(dev))
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
 def test_linear_shapes_and_dtypes(dev):
@@ -629,19 +642,21 @@ def test_ffn_geglu_exact(dev):
 @pytest.mark.parametrize("m", [1, 64, 128, 200, 1024])
 def test_ffn_small_batch_k_slices_exact(dev, m):
     """An FFN whose down-projection (K = 5120, N = 1280) has too few output
-    tiles to fill the chip: the product is split in K across blocks (4 slices
-    on the skinny kernel at M = 64 and 128, 8 on the 128 x 128 kernel at
-    M = 200, 4 on the split-K kernel at M = 1024; the skinny kernel whole at
-    M = 1).  Up to M = 128 the up-projection takes the skinny kernel with the
-    hidden and gate rows in one block."""
+    tiles to fill the chip: from row-major weights the product is split in K
+    across blocks (4 slices on the skinny kernel at M = 64 and 128, 8 on the
+    128 x 128 kernel at M = 200, 4 on the split-K kernel at M = 1024; the
+    skinny kernel whole at M = 1), and up to M = 256 the up-projection takes
+    the skinny kernel with the hidden and gate rows in one block.  The same
+    from the packed weights."""
     k, inner = 1280, 5120
     x = activation(m, k, seed=11 + m)
     up8, ups = int8.prepare_weight(weight(2 * inner, k, seed=12).to(dev))
     dn8, dns = int8.prepare_weight(weight(k, inner, seed=13).to(dev))
     db = weight(1, k, seed=14, std=0.01)[0].float()
-    y = int8.ffn(x.to(dev), up8, ups, dn8, dns, db.to(dev), act="geglu_erf")
     want = O.ffn(bits(x), npy(up8), npy(ups), npy(dn8), npy(dns), npy(db), act=4)
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for up, dn in zip(packed_and_row_major(up8), packed_and_row_major(dn8)):
+        y = int8.ffn(x.to(dev), up, ups, dn, dns, db.to(dev), act="geglu_erf")
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
 def test_ffn_stream_dirty_workspace_exact(dev):
@@ -687,18 +702,19 @@ def test_ffn_up_epilogue_exact(dev, act, m, inner, k):
     check_ffn_up(dev, act, m, inner, k)
 
 
-@pytest.mark.parametrize("act", [4, 5])
+@pytest.mark.parametrize("act", [3, 4, 5])
 def test_ffn_up_persistent_tiles_exact(dev, act):
     """The same through the persistent 256x320 kernel: 578 paired tiles
-    (GEGLU) or 289 plain ones (GELU), ragged in both dimensions, K % 64 != 0."""
+    (situ, GEGLU) or 289 plain ones (GELU), ragged in both dimensions, K % 64 != 0."""
     check_ffn_up(dev, act, 4100, 5200, 1040)
 
 
-@pytest.mark.parametrize("act", [4, 5])
+@pytest.mark.parametrize("act", [3, 4, 5])
 def test_ffn_up_wide_range_exact(dev, act):
-    """The persistent kernel reads the GELU (erf) table through a window in LDS
-    that holds the inputs with |g| in [2^-12, 16), and the table in global
-    memory for the others: column scales spread over twelve decades put the
+    """The persistent kernel reads the GELU (erf) table, or situ's gate factor,
+    through a window in LDS that holds the inputs with |g| in [2^-12, 16), situ's
+    tanh through one for [2^-10, 16), and the table in global memory for the
+    others: column scales spread over twelve decades put the
     activation's inputs on both sides of the window, both signs, in every
     wave."""
     check_ffn_up(dev, act, 4100, 5200, 1040, wide=True)
@@ -748,12 +764,12 @@ def test_ffn_full_size_c4(dev):
     assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
-# (2080, 3000, 1200) and (2048, 4000, 1280) take the split-K kernel with
+# (2080, 2992, 1200) and (2048, 4000, 1280) take the split-K kernel with
 # ragged output rows and columns, the first with an odd number of 32-row
-# contraction steps
+# contraction steps; 3000 is no multiple of 16 (torch's product)
 @pytest.mark.parametrize("m,n,k", [(4096, 5120, 1280), (1000, 272, 208), (1, 16, 16),
                                    (77, 1280, 4096), (300, 2000, 2000), (33, 2400, 1600),
-                                   (2080, 3000, 1200), (2048, 4000, 1280)])
+                                   (2080, 3000, 1200), (2080, 2992, 1200), (2048, 4000, 1280)])
 def test_linear_dw(dev, m, n, k):
     """dL/dW = dy^T x through the bf16 MFMA kernel, against float64: each
     element within one bf16 rounding of the exact value plus the fp32
@@ -825,8 +841,9 @@ def test_linear_dx_int8_full_size_c5(dev):
 def test_linear_dx_int8_split_k_shapes(dev, m, n, k):
     """Shapes where dx's GEMM reads the weight as stored (the split-K kernel's
     transposing LDS reads): a contraction that is not a multiple of 64
-    (2080, zero-filled tail), output columns that leave a partial 160-wide
-    tile (768), and a short one (2048)."""
+    (2080, zero-filled tail) and output columns that leave a partial 160-wide
+    tile (768); and one of 64 tiles, too few for it (the transposed weight in
+    the block layout)."""
     dy = activation(m, n, seed=n, scale=1e-3, n_out=0)
     w8, ws = int8.prepare_weight(weight(n, k, seed=k).to(dev))
     dx = int8.linear_dx_int8(dy.to(dev), w8, ws)
@@ -837,12 +854,10 @@ def test_linear_dx_int8_split_k_shapes(dev, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(200, 5120, 1280), (1024, 5120, 1280), (300, 2560, 1024),
                                    (64, 5120, 1280), (100, 5120, 1280)])
 def test_linear_dx_int8_k_slices_exact(dev, m, n, k):
-    """Small batches, too few output tiles for the chip: the contraction is
-    split across blocks (8 slices on the 128 x 128 kernel through the
-    transposed weight at M = 200; 4 and 2 slices on the split-K kernel
-    reading the weight as stored, the last with a ragged 160-column tile; 4
-    slices on the skinny kernel through the transposed weight at M = 64 and
-    100)."""
+    """Small batches whose row-major product would be split in K across blocks:
+    the transposed weight in the block layout, on the tiles of the kernel that
+    splits K over a block's waves (the row-major slices, for a contraction past
+    32768: test_gpu_dx_tiles.py)."""
     dy = activation(m, n, seed=m + n, scale=1e-3, n_out=0)
     w8, ws = int8.prepare_weight(weight(n, k, seed=k + 1).to(dev))
     dx = int8.linear_dx_int8(dy.to(dev), w8, ws)

@@ -6,7 +6,7 @@ linear, on the GPU:
   ``residual + residual_scale * out`` runs in the GEMM's store; it must equal
   the reference chain -- the dequant result rounded to bf16, then
   torch.addcmul on bf16 tensors -- bit for bit, through every GEMM kernel
-  (persistent, two-block, small, split-K, skinny).  Other forms run the
+  (persistent, two-block, small, split-K, skinny; and the packed weight's).  Other forms run the
   reference's torch chain and keep its dtype promotion.
 * Weight formats: per-channel scales stored as [N, 1] (the checkpoint shape,
   reference tests/test_int8_api.py:148-150), per-tensor scales, and an
@@ -43,12 +43,13 @@ def test_linear_residual_fused_exact(dev, m, n, k):
     g = torch.Generator().manual_seed(m + n)
     res = torch.randn(m, n, generator=g).to(torch.bfloat16)
     rscale = (torch.rand(n, generator=g) * 2 - 0.5).to(torch.bfloat16)
-    got = int8.linear(x.to(dev), w8, ws, bias.to(dev), residual=res.to(dev),
-                      residual_scale=rscale.to(dev))
-    assert got.dtype == torch.bfloat16 and tuple(got.shape) == (m, n)
     d = O.linear(bits(x), npy(w8), npy(ws), O.bf16_to_f32(bits(bias)))
     want = _residual_reference(d, bits(res), bits(rscale))
-    assert np.array_equal(bits(got), want), mismatch(bits(got), want)
+    for form in (w8, w8.clone()):       # (the clone carries no packed copy)
+        got = int8.linear(x.to(dev), form, ws, bias.to(dev), residual=res.to(dev),
+                          residual_scale=rscale.to(dev))
+        assert got.dtype == torch.bfloat16 and tuple(got.shape) == (m, n)
+        assert np.array_equal(bits(got), want), mismatch(bits(got), want)
     # the closed form of the same update: one fp32 add of an exact product
     f = lambda b: O.bf16_to_f32(b)
     closed = O.f32_to_bf16(f(bits(res)) + f(d) * f(bits(rscale))[None, :])

@@ -1,12 +1,14 @@
 """Seeded random shapes over the whole dispatch space of the linear, the FFN and
 linear_dx_int8, each bit-exact against the oracle.
 
-The GEMM a call takes depends on M, N and K: the skinny kernel (M <= 64;
-M <= 256 for the FFN's paired up-projection, in 128-row chunks above 128),
+The GEMM a call takes depends on the weight's form and on M, N and K.  From a
+row-major weight: the skinny kernel (M <= 64; M <= 256 for the FFN's paired up-projection, in 128-row chunks above 128),
 K slices on the skinny, the 128 x 128 or the split-K kernel for outputs too
 small to fill the chip (then a dequant pass that adds the slices), the
 split-K and the persistent kernels on the activation in MFMA-block order,
-and the two-block kernel.  The fixed-shape tests sit on each side of every
+and the two-block kernel.  From a packed one: the kernel that quantizes a few
+rows itself, the skinny kernel, K split over a block's waves, split K and the
+tiles of the persistent kernel.  Each shape runs from both.  The fixed-shape tests sit on each side of every
 threshold; these draw shapes between them (ragged M, N any multiple of 16, K
 any multiple of 256), so that no combination of tile remainders and slice
 counts goes untested.  Shapes are drawn once from fixed seeds and appear in
@@ -77,9 +79,10 @@ def test_linear_random_shapes_exact(dev, m, n, k):
     x = activation(m, k, seed=m + 7 * n + k, n_out=3, mult=25.0)
     w8, ws = int8.prepare_weight(weight(n, k, seed=n + k).to(dev))
     bias = weight(1, n, seed=n + 3 * k, std=0.01)[0]
-    y = int8.linear(x.to(dev), w8, ws, bias.to(dev))
     want = O.linear(bits(x), npy(w8), npy(ws), O.bf16_to_f32(bits(bias)))
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for form in (w8, w8.clone()):       # (the clone carries no packed copy)
+        y = int8.linear(x.to(dev), form, ws, bias.to(dev))
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
 @pytest.mark.parametrize("m,k,inner,act", FFN,
@@ -91,10 +94,11 @@ def test_ffn_random_shapes_exact(dev, m, k, inner, act):
     up8, ups = int8.prepare_weight(weight(rows, k, seed=inner + 1).to(dev))
     dn8, dns = int8.prepare_weight(weight(k, inner, seed=inner + 2).to(dev))
     db = weight(1, k, seed=k + 5, std=0.01)[0]
-    y = int8.ffn(x.to(dev), up8, ups, dn8, dns, db.to(dev), act=name)
     want = O.ffn(bits(x), npy(up8), npy(ups), npy(dn8), npy(dns), O.bf16_to_f32(bits(db)),
                  act=act)
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for up, dn in ((up8, dn8), (up8.clone(), dn8.clone())):
+        y = int8.ffn(x.to(dev), up, ups, dn, dns, db.to(dev), act=name)
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
 
 
 @pytest.mark.parametrize("m,n,k", DX, ids=[f"{m}x{n}x{k}" for m, n, k in DX])
@@ -187,9 +191,9 @@ def test_prepare_and_dequant_weight_random_shapes_exact(dev, n, k):
 
 
 # ------------------------------------------------------- bf16 dense GEMMs
-# linear_dx (dy @ w) and linear_dw (dy^T @ x) in bf16: the split-K kernel,
-# K slices for small batches, the 128 x 128 TN / NN kernels for the shapes
-# the split-K kernel does not take (dims % 16 only).  Bar: each element
+# linear_dx (dy @ w) and linear_dw (dy^T @ x) in bf16: the split-K kernel, and
+# the persistent kernel's tiles, whole or in slices of the contraction, for the
+# shapes it does not take (dims % 16 only).  Bar: each element
 # within one bf16 rounding of the float64 product plus the fp32 accumulation
 # error, 2^-8 |ref| + 2^-14 sum |a||b|.
 

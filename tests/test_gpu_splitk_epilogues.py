@@ -3,7 +3,8 @@ tile's rows; the row and column operands loaded before the main loop) with
 every epilogue it serves, at ragged shapes where the last tiles are partly
 outside the output: the dequant with a bf16 bias, an fp32 bias and none; the
 fused residual update; and the GELU up-projection of an FFN whose inner width
-is narrow.  Each is bit for bit the oracle's."""
+is narrow (from a row-major weight: the packed one's tiles leave it out).  Each
+is bit for bit the oracle's, from the packed weight too."""
 
 import numpy as np
 import pytest
@@ -59,23 +60,25 @@ def test_splitk_residual_exact(dev, m, n, k):
     g = torch.Generator().manual_seed(m * n)
     res = torch.randn(m, n, generator=g).to(torch.bfloat16)
     rscale = (torch.rand(n, generator=g) * 2 - 0.5).to(torch.bfloat16)
-    got = int8.linear(x.to(dev), w8, ws, bias.to(dev), residual=res.to(dev),
-                      residual_scale=rscale.to(dev))
     d = O.linear(bits(x), npy(w8), npy(ws), O.bf16_to_f32(bits(bias)))
     f = O.bf16_to_f32
     want = O.f32_to_bf16(f(bits(res)) + f(d) * f(bits(rscale))[None, :])
-    assert np.array_equal(bits(got), want), mismatch(bits(got), want)
+    for form in (w8, w8.clone()):       # (the clone carries no packed copy)
+        got = int8.linear(x.to(dev), form, ws, bias.to(dev), residual=res.to(dev),
+                          residual_scale=rscale.to(dev))
+        assert np.array_equal(bits(got), want), mismatch(bits(got), want)
 
 
 @pytest.mark.parametrize("m,k,inner", [(4096, 2048, 1280), (2100, 1024, 1280)])
 def test_splitk_gelu_up_projection_exact(dev, m, k, inner):
-    """FFN with GELU (erf): the up-projection [m, inner] from K = k takes the
-    split-K kernel with the activation epilogue."""
+    """FFN with GELU (erf): from row-major weights the up-projection [m, inner] from
+    K = k takes the split-K kernel with the activation epilogue."""
     x = activation(m, k, seed=m + inner)
     up8, ups = int8.prepare_weight(weight(inner, k, seed=inner + 1).to(dev))
     dn8, dns = int8.prepare_weight(weight(k, inner, seed=inner + 2).to(dev))
     db = weight(1, k, seed=k + 5, std=0.01)[0]
-    y = int8.ffn(x.to(dev), up8, ups, dn8, dns, db.to(dev), act="gelu_erf")
     want = O.ffn(bits(x), npy(up8), npy(ups), npy(dn8), npy(dns), O.bf16_to_f32(bits(db)),
                  act=5)
-    assert np.array_equal(bits(y), want), mismatch(bits(y), want)
+    for up, dn in ((up8, dn8), (up8.clone(), dn8.clone())):
+        y = int8.ffn(x.to(dev), up, ups, dn, dns, db.to(dev), act="gelu_erf")
+        assert np.array_equal(bits(y), want), mismatch(bits(y), want)
