@@ -277,8 +277,8 @@ int xpuint8_linear_residual_packed_stream(const void *stream, const void *x, con
 /* linear_acc in one call: (q, x_scale) = xpuint8_convrot_quantize_stream(x),
  * acc[M,N] = q @ w8^T (int32, exact), bit for bit, the codes in `work`
  * (xpuint8_linear_workspace_size(M, N, K) bytes suffice) laid out for the
- * GEMM (the MFMA block layout where the persistent kernel takes the shape),
- * and w8_packed (optional) read there in place of w8.  x_scale fp32 [M] is
+ * GEMM (the MFMA block layout with w8_packed (optional), which is then read in
+ * place of w8, and where the persistent kernel takes the shape).  x_scale fp32 [M] is
  * an output.  Replaces quantize + torch._int_mm at
  * python/xpu_kernels/int8/ops.py:571-588; no counterpart as one call. */
 int xpuint8_linear_acc_packed_stream(const void *stream, const void *x, const int8_t *w8,
@@ -375,8 +375,9 @@ int xpuint8_dx_gemm_stream(const void *stream, const int8_t *q, const float *a,
  * of at least xpuint8_linear_dx_int8_workspace_size(M, N, K) bytes (the
  * quantized gradient, its scales, the transposed weight and the product before
  * the inverse rotation; for small batches, whose [M,K] output has too few
- * tiles to fill the GPU, also the int32 partial products of the contraction
- * split across blocks), 16-byte aligned; it is fully written before it is
+ * tiles to fill the GPU, also room for the int32 partial products of the
+ * contraction split across blocks, which rows of dy past 32768 columns use),
+ * 16-byte aligned; it is fully written before it is
  * read, so it needs no clearing.  Replaces linear_dx_int8
  * (python/xpu_kernels/int8/ops.py:353-377): its torch multiply, the Triton
  * quantize_row, torch._int_mm, dequant and rotate. */

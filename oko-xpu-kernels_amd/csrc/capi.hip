@@ -141,13 +141,16 @@ int check_gemm(int64_t M, int64_t N, int64_t K) {
     } while (0)
 
 // The workspace of linear_dx_int8: the row-quantized column-scaled gradient
-// q [M,N] int8 (row-major, or in the MFMA block layout when the split-K
-// kernel reads it) and its row scales a [M] fp32, the transposed weight w8^T
-// [K,N] int8 (the GEMM's K-contiguous operand, for shapes the split-K kernel
-// does not take), and the product before the inverse rotation, bf16 [M,K];
-// for a product split in K across blocks (gemm_slices of the [M,K] output
-// over the contraction N), then the slices' int32 [M,K] partial products.
-// Each piece starts on a 256-byte boundary.
+// q [M,N] int8 (in the MFMA block layout, or row-major where the quantizer cannot
+// write it so) and its row scales a [M] fp32; the transposed weight w8^T [K,N]
+// int8 (for shapes that do not read w8 as stored), in the block layout, whose
+// padding may run on into the next piece, or row-major; the product before the
+// inverse rotation, bf16 [M,K] (the block-layout transpose's product goes to dx
+// instead); and, where gemm_slices of the [M,K] output over the contraction N
+// gives a split, the slices' int32 [M,K] partial products (read by the row-major
+// product alone, N > 32768 or a few rows with N % 64 != 0, but part of the
+// documented size for every such shape).  Each piece starts on a 256-byte
+// boundary.
 struct DxWork {
     size_t q, a, wt, pre, part, total;
 };
